@@ -452,14 +452,50 @@ extern "C" int rjk_vj_upper_with_ri_v_sync(rjk_ctx* ctx, const double* dm, size_
 // ---------------------------------------------------------------------------
 namespace {
 
+// FP64/FP32 tile rows.  128-row tiles share each fetched operand among more MFMAs; 64-row ones
+// are taken where nbf fits one of them.
+size_t k_tile(size_t nbf) { return nbf <= 64 ? 64 : 128; }
+
+// 16-column groups of a half-transform tile for f groups in all: the tile that leaves the fewest
+// padding columns, a tile costing about one group beyond its columns (its share of staging B);
+// never more columns than 64-column tiles would pad to.
+int k_tile_groups(size_t f) {
+    int best = 4;
+    size_t cost = (f + 3) / 4 * 5;
+    for (int fn = 1; fn <= 6; ++fn) {
+        const size_t tiles = (f + fn - 1) / fn, c = tiles * (fn + 1);
+        if (tiles * fn <= round_up(f, 4) && (c < cost || (c == cost && fn > best))) {
+            cost = c;
+            best = fn;
+        }
+    }
+    return best;
+}
+
 void k_plan_cols(KPlan& kp, size_t nbf, const size_t* ncol, int ns, int prec) {
     const size_t gran = is_bf16(prec) ? kBfColGran : kTileK;
-    kp.nbf_pad = round_up(nbf, kTileMN);
+    kp.tile = is_bf16(prec) ? kTileMN : k_tile(nbf);
+    kp.nbf_pad = round_up(nbf, kp.tile);
     kp.col_cnt[0] = round_up(ncol[0], gran);
     kp.col_off[0] = 0;
     kp.col_cnt[1] = ns == 2 ? round_up(ncol[1], gran) : 0;
     kp.col_off[1] = kp.col_cnt[0];
-    kp.nk = round_up(kp.col_cnt[0] + kp.col_cnt[1], kColPad);
+    const size_t tot = kp.col_cnt[0] + kp.col_cnt[1];
+    if (is_bf16(prec)) {
+        kp.nk = round_up(tot, kColPad);
+    } else {
+        kp.fn = k_tile_groups(tot / kTileK);
+        kp.nk = round_up(tot, (size_t)kp.fn * kTileK);
+    }
+}
+
+// split-K partials that some chunk fills: a chunk of Pc columns fills ceil(Pc / ceil(Pc / nsplit))
+size_t k_slots(size_t naux, size_t chunk, size_t nsplit) {
+    auto filled = [&](size_t Pc) {
+        const size_t pps = (Pc + nsplit - 1) / nsplit;
+        return Pc ? (Pc + pps - 1) / pps : 0;
+    };
+    return std::max<size_t>(1, std::max(filled(std::min(chunk, naux)), filled(naux % chunk)));
 }
 
 // chunking and split-K; carves [cocc | sign | kpart | M'] out of the workspace.
@@ -467,38 +503,50 @@ void k_plan_cols(KPlan& kp, size_t nbf, const size_t* ncol, int ns, int prec) {
 // partial tiles are FP64.
 int k_plan_ws(rjk_ctx* ctx, KPlan& kp, int ns, int prec, void** cocc, void** sign, double** kpart, void** m) {
     const size_t es = k_elem_size(prec);
-    const size_t nt = kp.nbf_pad / kTileMN;
-    const size_t ntiles = nt * (nt + 1) / 2;
     const size_t target = 1024;  // SYRK work-groups
     const size_t slot = kp.nbf_pad * kp.nbf_pad;
-    const size_t slot_bytes = (size_t)ns * slot * sizeof(double);
     const size_t perP = kp.nk * kp.nbf_pad * es;
-    const size_t small = round_up(kp.nbf_pad * kp.nk * es, 256) + round_up(kp.nk * es, 256);
-    // split-K slots: a multiple of 8 (one XCD per split), about `target`
-    // work-groups, at most a quarter of the workspace
-    size_t nsplit = round_up(std::max<size_t>(1, target / (ntiles * ns)), 8);
-    const size_t cap = std::max<size_t>(8, ((ctx->ws_limit / 4) / slot_bytes) / 8 * 8);
-    nsplit = std::min(nsplit, cap);
-    size_t fixed = small + nsplit * slot_bytes;
-    size_t avail = ctx->ws_limit > fixed ? ctx->ws_limit - fixed : 0;
-    size_t chunk = perP ? std::min(ctx->naux, std::max<size_t>(1, avail / perP)) : ctx->naux;
-    if (prec != RJK_PREC_FP64 && kp.nk > 0) {
+    size_t nsplit, chunk;
+    if (prec == RJK_PREC_FP64) {
+        // about `target` work-groups, at least 8 k-blocks a split, at most a quarter of the workspace
+        const size_t nt = kp.nbf_pad / kp.tile, ntiles = nt * (nt + 1) / 2;
+        const size_t slot_bytes = (size_t)ns * slot * sizeof(double);
+        const size_t small = round_up(kp.nbf_pad * kp.nk * es, 256) + round_up(kp.nk * es, 256);
+        const size_t blocks = std::max<size_t>(1, ctx->naux * std::max<size_t>(1, kp.nk / kTileK / ns));
+        nsplit = std::min(round_up(std::max<size_t>(1, target / (ntiles * ns)), 8), round_up((blocks + 7) / 8, 8));
+        nsplit = std::min(nsplit, std::max<size_t>(8, ((ctx->ws_limit / 4) / slot_bytes) / 8 * 8));
+        const size_t fixed = small + nsplit * slot_bytes;
+        const size_t avail = ctx->ws_limit > fixed ? ctx->ws_limit - fixed : 0;
+        chunk = perP ? std::min(ctx->naux, std::max<size_t>(1, avail / perP)) : ctx->naux;
+    } else {
         // FP32 accumulators: each split sums at most kFp32Chain products (pps auxiliary
         // columns × nk) before its partial joins the FP64 sum, so rounding does not grow
-        // with naux.  Up to half the workspace goes to the partials.
-        const size_t pps = std::max<size_t>(1, kFp32Chain / kp.nk);
-        const size_t smax = std::max<size_t>(8, ((ctx->ws_limit / 2) / slot_bytes) / 8 * 8);
-        fixed = small + smax * slot_bytes;
-        avail = ctx->ws_limit > fixed ? ctx->ws_limit - fixed : 0;
-        chunk = std::min({ctx->naux, std::max<size_t>(1, avail / perP), smax * pps});
-        nsplit = std::min(smax, std::max(nsplit, round_up((chunk + pps - 1) / pps, 8)));
+        // with naux.  Up to half the workspace goes to the partials.  The splits follow from the sizes
+        // padded to 128 rows and 64 columns, not from the tiles chosen, so that no choice of
+        // tile changes where an FP32 sum ends.
+        const size_t pad = round_up(ctx->nbf, kTileMN), nk = round_up(kp.nk ? kp.col_cnt[0] + kp.col_cnt[1] : 0, kColPad);
+        const size_t nt = pad / kTileMN, ntiles = nt * (nt + 1) / 2;
+        const size_t slot_bytes = (size_t)ns * pad * pad * sizeof(double), perP_ = nk * pad * es;
+        const size_t small = round_up(pad * nk * es, 256) + round_up(nk * es, 256);
+        nsplit = round_up(std::max<size_t>(1, target / (ntiles * ns)), 8);
+        nsplit = std::min(nsplit, std::max<size_t>(8, ((ctx->ws_limit / 4) / slot_bytes) / 8 * 8));
+        chunk = ctx->naux;
+        if (nk > 0) {
+            const size_t pps = std::max<size_t>(1, kFp32Chain / nk);
+            const size_t smax = std::max<size_t>(8, ((ctx->ws_limit / 2) / slot_bytes) / 8 * 8);
+            const size_t fixed = small + smax * slot_bytes;
+            const size_t avail = ctx->ws_limit > fixed ? ctx->ws_limit - fixed : 0;
+            chunk = std::min({ctx->naux, std::max<size_t>(1, avail / perP_), smax * pps});
+            nsplit = std::min(smax, std::max(nsplit, round_up((chunk + pps - 1) / pps, 8)));
+        }
     }
     kp.nsplit = nsplit;
     kp.chunk = chunk;
+    kp.nslot = k_slots(ctx->naux, chunk, nsplit);
     Carve cv;
     size_t ic = cv.add(kp.nbf_pad * kp.nk * es);
     size_t is = cv.add(kp.nk * es);
-    size_t ik = cv.add(kp.nsplit * ns * slot * sizeof(double));
+    size_t ik = cv.add(kp.nslot * ns * slot * sizeof(double));
     size_t im = cv.add(chunk * perP);
     void* ws = nullptr;
     int rc = ws_get(ctx, cv.total, &ws);
@@ -519,18 +567,19 @@ int k_run(rjk_ctx* ctx, const KPlan& kp, int ns, int prec, const void* b, const 
         return RJK_OK;
     }
     const bool bf = is_bf16(prec);
+    const double work_nk = (double)round_up(kp.col_cnt[0] + kp.col_cnt[1], kColPad);   // profiler's column count
     for (size_t P0 = 0; P0 < ctx->naux; P0 += kp.chunk) {
         size_t Pc = std::min(kp.chunk, ctx->naux - P0);
         const double nb = (double)ctx->nbf;
         {
-            PhaseScope ps(ctx, 2, prec, 2.0 * nb * nb * (double)kp.nk * (double)Pc);
+            PhaseScope ps(ctx, 2, prec, 2.0 * nb * nb * work_nk * (double)Pc);
             if (bf) RJK_HIP(ctx, launch_bf_khalf(st, prec, b, ctx->naux, ctx->nbf, P0, Pc, kp, cocc, m));
             else RJK_HIP(ctx, launch_khalf(st, prec, b, ctx->ldb, ctx->nbf, P0, Pc, kp, cocc, m));
         }
         {
-            PhaseScope ps(ctx, 3, prec, nb * (nb + 1.0) * (double)kp.nk * (double)Pc);
+            PhaseScope ps(ctx, 3, prec, nb * (nb + 1.0) * work_nk * (double)Pc);
             if (bf) RJK_HIP(ctx, launch_bf_ksyrk(st, prec, m, Pc, kp, ns, sign, P0 > 0 ? 1 : 0, kpart));
-            else RJK_HIP(ctx, launch_ksyrk(st, prec, m, Pc, kp, ns, sign, P0 > 0 ? 1 : 0, kpart));
+            else RJK_HIP(ctx, launch_ksyrk(st, prec, m, ctx->nbf, Pc, kp, ns, sign, P0 > 0 ? 1 : 0, kpart));
         }
     }
     PhaseScope ps(ctx, 4);
@@ -616,8 +665,10 @@ int vk_dm_general(rjk_ctx* ctx, const double* dm_dev, int ns, double scale, doub
     const size_t nbf = ctx->nbf, n2 = nbf * nbf;
     hipStream_t st = ctx->stream;
     KPlan kp;
-    kp.nbf_pad = round_up(nbf, kTileMN);
-    kp.nk = round_up(nbf, kColPad);
+    kp.tile = k_tile(nbf);
+    kp.nbf_pad = round_up(nbf, kp.tile);
+    kp.fn = k_tile_groups((nbf + kTileK - 1) / kTileK);
+    kp.nk = round_up(nbf, (size_t)kp.fn * kTileK);
     kp.col_cnt[0] = kp.nk;
     const size_t ccol = kp.nbf_pad * kp.nk * sizeof(double);
     const size_t gbytes = n2 * sizeof(double);

@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) void k_b_prep(const BProb* __restrict__ pr, in
 template <typename T, int FM, int FN>
 __global__ __launch_bounds__(kBlock) void k_b_khalf(const BProb* __restrict__ pr, const int* __restrict__ sub,
                                                     const size_t* __restrict__ off, int nsub) {
-    constexpr int TM = 2 * FM * 16, TN = 2 * FN * 16;
+    constexpr int TM = 64 * FM, TN = 16 * FN;
     const size_t total = off[nsub];
     for (size_t it = blockIdx.x; it < total; it += gridDim.x) {
         const int j = find_prob(off, nsub, it);
@@ -240,13 +240,13 @@ __global__ __launch_bounds__(kBlock) void k_b_khalf(const BProb* __restrict__ pr
         if (Pl >= P.naux) continue;   // padding items (uniform per work-group)
         const int rem = (int)(kq % per), mt = rem / ntc, ct = rem % ntc;
         khalf_tile<T, FM, FN>(glb((const T*)P.b) + (size_t)Pl * P.ldb, P.nbf, mt * TM, ct * TN, glb((const T*)P.cocc),
-                              P.nk, P.nbf_pad, glb((T*)P.m) + (size_t)Pl * P.nk * P.nbf_pad);
+                              P.nk, P.nbf_pad, glb((T*)P.m) + (size_t)Pl * P.nk * P.nbf_pad, rotation((int)kq));
     }
 }
 
-template <typename T, int F>
+template <typename T, int FB>
 __global__ __launch_bounds__(kBlock) void k_b_ksyrk(const BProb* __restrict__ pr, int np, Tables tb) {
-    constexpr int Tt = 2 * F * 16;
+    constexpr int Tt = 64 * FB;
     const size_t total = tb.syrk[np];
     for (size_t it = blockIdx.x; it < total; it += gridDim.x) {
         const int q = find_prob(tb.syrk, np, it);
@@ -260,8 +260,9 @@ __global__ __launch_bounds__(kBlock) void k_b_ksyrk(const BProb* __restrict__ pr
         size_t tm, tn;
         upper_tile(t, &tm, &tn);
         const int Pb = split * P.pps, Pe = min(P.naux, Pb + P.pps);
-        ksyrk_tile<T, F>(glb((const T*)P.m), P.nbf_pad, P.nk, (int)tm * Tt, (int)tn * Tt, 0, P.ncb, Pb, Pe,
-                         glb((const T*)P.sign), 0, glb(P.kpart) + (size_t)split * P.nbf_pad * P.nbf_pad);
+        ksyrk_tile<T, FB>(glb((const T*)P.m), P.nbf_pad, P.nk, P.nbf, (int)tm * Tt, (int)tn * Tt, 0, P.ncb, Pb, Pe,
+                          glb((const T*)P.sign), 0, glb(P.kpart) + (size_t)split * P.nbf_pad * P.nbf_pad,
+                          rotation((int)kq));
     }
 }
 
@@ -791,14 +792,14 @@ int enqueue_fp(rjk_batch* b, hipEvent_t* ev) {
     hipLaunchKernelGGL(k_b_prep<T>, dim3(grid_elem(b->t_prep.back())), dim3(256), 0, st, b->d_prob, np, tb);
     mark(4);
     if (b->t_sub_items[0])
-        hipLaunchKernelGGL((k_b_khalf<T, 2, 2>), dim3(grid_items(b, b->t_sub_items[0], b->waves)), dim3(kBlock), 0,
+        hipLaunchKernelGGL((k_b_khalf<T, 1, 4>), dim3(grid_items(b, b->t_sub_items[0], b->waves)), dim3(kBlock), 0,
                            st, b->d_prob, b->d_sub, b->d_suboff, b->t_sub_n[0]);
     mark(5);
     if (b->t_sub_items[3])
-        hipLaunchKernelGGL((k_b_khalf<T, 4, 2>), dim3(grid_items(b, b->t_sub_items[3], b->waves)), dim3(kBlock), 0,
+        hipLaunchKernelGGL((k_b_khalf<T, 2, 4>), dim3(grid_items(b, b->t_sub_items[3], b->waves)), dim3(kBlock), 0,
                            st, b->d_prob, b->d_sub + 3 * np, b->d_suboff + 3 * (np + 1), b->t_sub_n[3]);
     mark(6);
-    hipLaunchKernelGGL((k_b_ksyrk<T, 4>), dim3(grid_items(b, b->t_syrk.back(), b->waves)), dim3(kBlock), 0, st,
+    hipLaunchKernelGGL((k_b_ksyrk<T, 2>), dim3(grid_items(b, b->t_syrk.back(), b->waves)), dim3(kBlock), 0, st,
                        b->d_prob, np, tb);
     mark(7);
     mark(8);

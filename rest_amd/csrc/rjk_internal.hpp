@@ -128,11 +128,14 @@ void j_plan(size_t ldb, size_t naux, int prec, size_t* nchunk, size_t* nsplit);
 
 // K
 struct KPlan {
-    size_t nbf_pad = 0;      // multiple of kTileMN
-    size_t nk = 0;           // padded occupied columns, all spins (multiple of kColPad)
+    size_t tile = kTileMN;   // FP64/FP32: rows of the half-transform and SYRK tiles (64 or 128)
+    int fn = 4;              // FP64/FP32: 16-column groups of a half-transform tile (1..6)
+    size_t nbf_pad = 0;      // multiple of `tile`; BF16: of kTileMN
+    size_t nk = 0;           // padded occupied columns, all spins (multiple of 16·fn; BF16: of kColPad)
     size_t col_off[2] = {0, 0}, col_cnt[2] = {0, 0};   // per-spin column ranges (multiples of 16)
     size_t chunk = 0;        // P per chunk
-    size_t nsplit = 0;       // split-K slots of the SYRK
+    size_t nsplit = 0;       // split-K divisor of the SYRK: a chunk of Pc columns takes ceil(Pc / nsplit) a split
+    size_t nslot = 0;        // split-K partials kept: the splits that hold columns in some chunk (<= nsplit)
 };
 size_t k_elem_size(int prec);   // bytes per element of C', M' and signs (all planes) for a K precision
 hipError_t launch_prep_cocc(hipStream_t st, int prec, const double* eigv, size_t nbf, size_t nstate,
@@ -143,7 +146,7 @@ hipError_t launch_prep_cocc_idx(hipStream_t st, int prec, const double* vecs, si
                                 void* sign);
 hipError_t launch_khalf(hipStream_t st, int prec, const void* b, size_t ldb, size_t nbf, size_t P0, size_t Pc,
                         const KPlan& kp, const void* cocc, void* m);
-hipError_t launch_ksyrk(hipStream_t st, int prec, const void* m, size_t Pc, const KPlan& kp, int nspin,
+hipError_t launch_ksyrk(hipStream_t st, int prec, const void* m, size_t nbf, size_t Pc, const KPlan& kp, int nspin,
                         const void* sign, int beta, double* kpart);
 hipError_t launch_kreduce(hipStream_t st, const double* kpart, const KPlan& kp, int nspin, size_t nbf,
                           double scale, double* vk);

@@ -16,7 +16,7 @@
 // Stage 2 (K-SYRK): Kpart[split][s][ν][μ] (+)= Σ_{P,c} M'[P][c][μ] sign_c M'[P][c][ν]
 //   over upper tile pairs (μ-tile <= ν-tile), split-K over P so that the
 //   small nbf×nbf output still fills 256 CUs; deterministic (no atomics).
-// Stage 3 (K-reduce): vk_s[p(i,j)] = scale · Σ_split Kpart[split][s][j][i].
+// Stage 3 (K-reduce): vk_s[p(i,j)] = scale · Σ_slot Kpart[slot][s][j][i].
 //
 // MFMA: v_mfma_f64_16x16x4f64.  Lane l supplies A[l%16][l/16] and
 // B[l/16][l%16]; register r of lane l receives D[l/16 + 4r][l%16] (probed on
@@ -31,56 +31,79 @@ using namespace kt;
 
 // ---------------------------------------------------------------------------
 // Stage 1 kernel: 1-D grid, XCD-aware — every work-group of auxiliary column P
-// runs on XCD P % 8, so the 12 μ-tiles × column tiles of one packed column
+// runs on XCD P % 8, so the μ-tiles × column tiles of one packed column
 // share it in that XCD's L2.
 // ---------------------------------------------------------------------------
 template <typename T, int FM, int FN>
 __global__ __launch_bounds__(kBlock) void k_khalf(const T* __restrict__ b, size_t ldb, int nbf, size_t P0, int Pc,
                                                   int ntm, int ntc, const T* __restrict__ cocc, int nk, int ldm,
                                                   T* __restrict__ m) {
-    constexpr int TM = 2 * FM * 16, TN = 2 * FN * 16;
+    constexpr int TM = 64 * FM, TN = 16 * FN;
     // XCD-aware decode of the linear work-group id
     const int w = blockIdx.x, xcd = w % kXcd, kq = w / kXcd, per = ntm * ntc;
     const int Pl = (kq / per) * kXcd + xcd;
     if (Pl >= Pc) return;                    // padding work-groups (uniform exit)
     const int rem = kq % per, mt = rem / ntc, ct = rem % ntc;
-    khalf_tile<T, FM, FN>(b + (P0 + Pl) * ldb, nbf, mt * TM, ct * TN, cocc, nk, ldm, m + (size_t)Pl * nk * ldm);
+    khalf_tile<T, FM, FN>(b + (P0 + Pl) * ldb, nbf, mt * TM, ct * TN, cocc, nk, ldm, m + (size_t)Pl * nk * ldm,
+                          rotation(kq));
 }
 
 // ---------------------------------------------------------------------------
-// Stage 2 kernel: 1-D grid of nsplit × nspin × ntile(ntile+1)/2 work-groups,
-// nsplit a multiple of 8; split s runs entirely on XCD s % 8, so the M' slab
-// of a split is streamed into one L2 and shared by all tiles there.
+// Stage 2 kernel: 1-D grid of (nslot rounded up to 8) × nspin × ntile(ntile+1)/2
+// work-groups; split s runs entirely on XCD s % 8, so the M' slab of a split is
+// streamed into one L2 and shared by all tiles there.
 // ---------------------------------------------------------------------------
-template <typename T, int F>
-__global__ __launch_bounds__(kBlock) void k_ksyrk(const T* __restrict__ m, int ldm, int nk, int Pc, int ntile2,
-                                                  int nspin, SyrkCols cols, const T* __restrict__ sign,
-                                                  int p_per_split, int beta, double* __restrict__ kpart,
+template <typename T, int FB>
+__global__ __launch_bounds__(kBlock) void k_ksyrk(const T* __restrict__ m, int ldm, int nk, int nbf, int Pc,
+                                                  int ntile2, int nspin, SyrkCols cols, const T* __restrict__ sign,
+                                                  int nslot, int p_per_split, int beta, double* __restrict__ kpart,
                                                   size_t slot) {
-    constexpr int Tt = 2 * F * 16;
+    constexpr int Tt = 64 * FB;
     // XCD-aware decode: w -> (split on XCD w%8, spin, tile)
     const int w = blockIdx.x, xcd = w % kXcd, kq = w / kXcd;
     const size_t t = (size_t)(kq % ntile2);
     const int rest = kq / ntile2, spin = rest % nspin, split = (rest / nspin) * kXcd + xcd;
+    const int Pb = split * p_per_split, Pe = min(Pc, Pb + p_per_split);
+    if (split >= nslot || (beta && Pb >= Pe)) return;   // uniform exit
     size_t tm, tn;
     upper_tile(t, &tm, &tn);
-    const int Pb = split * p_per_split, Pe = min(Pc, Pb + p_per_split);
-    ksyrk_tile<T, F>(m, ldm, nk, (int)tm * Tt, (int)tn * Tt, cols.off[spin], cols.cnt[spin] / TK, Pb, Pe, sign, beta,
-                     kpart + ((size_t)split * nspin + spin) * slot);
+    ksyrk_tile<T, FB>(m, ldm, nk, nbf, (int)tm * Tt, (int)tn * Tt, cols.off[spin], cols.cnt[spin] / TK, Pb, Pe, sign,
+                      beta, kpart + ((size_t)split * nspin + spin) * slot, rotation(kq));
 }
 
-__global__ void k_kreduce(const double* __restrict__ kpart, int nsplit, int nspin, size_t slot, int ldm,
-                          size_t npair, double scale, double* __restrict__ vk) {
-    size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npair) return;
-    size_t j = (size_t)((sqrt(8.0 * (double)p + 1.0) - 1.0) * 0.5);
-    while (tri(j) > p) --j;
-    while (tri(j + 1) <= p) ++j;
-    size_t i = p - tri(j);
-    for (int s = 0; s < nspin; ++s) {
-        double acc = 0;
-        for (int q = 0; q < nsplit; ++q) acc += kpart[((size_t)q * nspin + s) * slot + j * ldm + i];
-        vk[(size_t)s * npair + p] = acc * scale;
+// vk = scale · Σ_slot Kpart.  A work-group sums 32 pairs with 8 threads each (slots g, g + 8, ...),
+// so that the chain of dependent additions is an eighth of the slot count and the loads of a
+// thread overlap: one thread per pair took 280 us for 1024 slots of 24 × 24, this takes 5.
+constexpr int kRedPairs = 32, kRedGroups = 8;
+__global__ __launch_bounds__(kRedPairs* kRedGroups) void k_kreduce(const double* __restrict__ kpart, int nslot,
+                                                                   int nspin, size_t slot, int ldm, size_t npair,
+                                                                   double scale, double* __restrict__ vk) {
+    __shared__ double sh[kRedGroups][kRedPairs];
+    const int x = threadIdx.x % kRedPairs, g = threadIdx.x / kRedPairs;
+    const size_t p = (size_t)blockIdx.x * kRedPairs + x;
+    const int s = blockIdx.y;
+    double acc = 0;
+    if (p < npair) {
+        size_t i, j;
+        upper_tile(p, &i, &j);   // p = tri(j) + i
+        const double* __restrict__ src = kpart + (size_t)s * slot + j * ldm + i;
+        const size_t step = (size_t)nspin * slot;
+        int q = g;
+        for (; q + 3 * kRedGroups < nslot; q += 4 * kRedGroups) {
+            double v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = src[(size_t)(q + u * kRedGroups) * step];
+            acc += (v[0] + v[1]) + (v[2] + v[3]);
+        }
+        for (; q < nslot; q += kRedGroups) acc += src[(size_t)q * step];
+    }
+    sh[g][x] = acc;
+    __syncthreads();
+    if (g == 0 && p < npair) {
+        double t = 0;
+#pragma unroll
+        for (int u = 0; u < kRedGroups; ++u) t += sh[u][x];
+        vk[(size_t)s * npair + p] = t * scale;
     }
 }
 
@@ -121,12 +144,11 @@ __global__ void k_prep_cocc_idx(const double* __restrict__ vecs, int nbf, const 
     if (nu == 0) sign[col_off + q] = (T)((w > 0) ? 1.0 : ((w < 0) ? -1.0 : 0.0));
 }
 
-template <typename T>
-hipError_t khalf_t(hipStream_t st, const T* b, size_t ldb, size_t nbf, size_t P0, size_t Pc, const KPlan& kp,
-                   const T* cocc, T* m) {
-    constexpr int FM = 4, FN = 2;                       // 128 (μ) × 64 (c) tiles
-    constexpr int TM = 2 * FM * 16, TN = 2 * FN * 16;
-    const int ntm = (int)(kp.nbf_pad / TM), ntc = (int)(kp.nk / TN);
+template <typename T, int FM, int FN>
+hipError_t khalf_go(hipStream_t st, const T* b, size_t ldb, size_t nbf, size_t P0, size_t Pc, const KPlan& kp,
+                    const T* cocc, T* m) {
+    constexpr int TM = 64 * FM, TN = 16 * FN;
+    const int ntm = (int)((nbf + TM - 1) / TM), ntc = (int)(kp.nk / TN);
     const size_t nwg = round_up(Pc, kXcd) * (size_t)ntm * ntc;
     hipLaunchKernelGGL((k_khalf<T, FM, FN>), dim3((unsigned)nwg), dim3(kBlock), 0, st, b, ldb, (int)nbf, P0,
                        (int)Pc, ntm, ntc, cocc, (int)kp.nk, (int)kp.nbf_pad, m);
@@ -134,21 +156,50 @@ hipError_t khalf_t(hipStream_t st, const T* b, size_t ldb, size_t nbf, size_t P0
 }
 
 template <typename T>
-hipError_t ksyrk_t(hipStream_t st, const T* m, size_t Pc, const KPlan& kp, int nspin, const T* sign, int beta,
-                   double* kpart) {
-    constexpr int F = 4;                                // 128 × 128 tiles
-    constexpr int Tt = 2 * F * 16;
-    const size_t nt = kp.nbf_pad / Tt, nt2 = nt * (nt + 1) / 2;
+hipError_t khalf_t(hipStream_t st, const T* b, size_t ldb, size_t nbf, size_t P0, size_t Pc, const KPlan& kp,
+                   const T* cocc, T* m) {
+    if (kp.tile == 64) {
+        switch (kp.fn) {
+            case 1: return khalf_go<T, 1, 1>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+            case 2: return khalf_go<T, 1, 2>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+            case 3: return khalf_go<T, 1, 3>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+            case 4: return khalf_go<T, 1, 4>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+            case 5: return khalf_go<T, 1, 5>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+            default: return khalf_go<T, 1, 6>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+        }
+    }
+    switch (kp.fn) {
+        case 1: return khalf_go<T, 2, 1>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+        case 2: return khalf_go<T, 2, 2>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+        case 3: return khalf_go<T, 2, 3>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+        case 4: return khalf_go<T, 2, 4>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+        case 5: return khalf_go<T, 2, 5>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+        default: return khalf_go<T, 2, 6>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+    }
+}
+
+template <typename T, int FB>
+hipError_t ksyrk_go(hipStream_t st, const T* m, size_t nbf, size_t Pc, const KPlan& kp, int nspin, const T* sign,
+                    int beta, double* kpart) {
+    const size_t nt = kp.nbf_pad / (64 * FB), nt2 = nt * (nt + 1) / 2;
     SyrkCols cols;
     cols.off[0] = (int)kp.col_off[0];
     cols.cnt[0] = (int)kp.col_cnt[0];
     cols.off[1] = (int)kp.col_off[1];
     cols.cnt[1] = (int)kp.col_cnt[1];
     const int pps = (int)((Pc + kp.nsplit - 1) / kp.nsplit);
-    const size_t nwg = kp.nsplit * (size_t)nspin * nt2;   // nsplit is a multiple of 8
-    hipLaunchKernelGGL((k_ksyrk<T, F>), dim3((unsigned)nwg), dim3(kBlock), 0, st, m, (int)kp.nbf_pad, (int)kp.nk,
-                       (int)Pc, (int)nt2, nspin, cols, sign, pps, beta, kpart, kp.nbf_pad * kp.nbf_pad);
+    const size_t nwg = round_up(kp.nslot, kXcd) * (size_t)nspin * nt2;
+    hipLaunchKernelGGL((k_ksyrk<T, FB>), dim3((unsigned)nwg), dim3(kBlock), 0, st, m, (int)kp.nbf_pad, (int)kp.nk,
+                       (int)nbf, (int)Pc, (int)nt2, nspin, cols, sign, (int)kp.nslot, pps, beta, kpart,
+                       kp.nbf_pad * kp.nbf_pad);
     return hipGetLastError();
+}
+
+template <typename T>
+hipError_t ksyrk_t(hipStream_t st, const T* m, size_t nbf, size_t Pc, const KPlan& kp, int nspin, const T* sign,
+                   int beta, double* kpart) {
+    if (kp.tile == 64) return ksyrk_go<T, 1>(st, m, nbf, Pc, kp, nspin, sign, beta, kpart);
+    return ksyrk_go<T, 2>(st, m, nbf, Pc, kp, nspin, sign, beta, kpart);
 }
 
 }  // namespace
@@ -196,18 +247,19 @@ hipError_t launch_khalf(hipStream_t st, int prec, const void* b, size_t ldb, siz
     return khalf_t<float>(st, (const float*)b, ldb, nbf, P0, Pc, kp, (const float*)cocc, (float*)m);
 }
 
-hipError_t launch_ksyrk(hipStream_t st, int prec, const void* m, size_t Pc, const KPlan& kp, int nspin,
+hipError_t launch_ksyrk(hipStream_t st, int prec, const void* m, size_t nbf, size_t Pc, const KPlan& kp, int nspin,
                         const void* sign, int beta, double* kpart) {
     if (prec == RJK_PREC_FP64)
-        return ksyrk_t<double>(st, (const double*)m, Pc, kp, nspin, (const double*)sign, beta, kpart);
-    return ksyrk_t<float>(st, (const float*)m, Pc, kp, nspin, (const float*)sign, beta, kpart);
+        return ksyrk_t<double>(st, (const double*)m, nbf, Pc, kp, nspin, (const double*)sign, beta, kpart);
+    return ksyrk_t<float>(st, (const float*)m, nbf, Pc, kp, nspin, (const float*)sign, beta, kpart);
 }
 
 hipError_t launch_kreduce(hipStream_t st, const double* kpart, const KPlan& kp, int nspin, size_t nbf, double scale,
                           double* vk) {
     size_t npair = nbf * (nbf + 1) / 2;
-    hipLaunchKernelGGL(k_kreduce, dim3((unsigned)((npair + 255) / 256)), dim3(256), 0, st, kpart, (int)kp.nsplit,
-                       nspin, kp.nbf_pad * kp.nbf_pad, (int)kp.nbf_pad, npair, scale, vk);
+    hipLaunchKernelGGL(k_kreduce, dim3((unsigned)((npair + kRedPairs - 1) / kRedPairs), (unsigned)nspin),
+                       dim3(kRedPairs * kRedGroups), 0, st, kpart, (int)kp.nslot, nspin, kp.nbf_pad * kp.nbf_pad,
+                       (int)kp.nbf_pad, npair, scale, vk);
     return hipGetLastError();
 }
 

@@ -196,19 +196,21 @@ __global__ __launch_bounds__(C::NT) void k_bf_khalf(const __bf16* __restrict__ b
 }
 
 // ---- stage 2 -------------------------------------------------------------------
-// 1-D grid of nsplit × nspin × ntile2 work-groups (nsplit a multiple of 8; split s
+// 1-D grid of (nslot rounded up to 8) × nspin × ntile2 work-groups (split s
 // on XCD s % 8).  Upper tile pairs (μ tile <= ν tile) of 128 × 128.
 template <class C>
 __global__ __launch_bounds__(C::NT) void k_bf_ksyrk(const __bf16* __restrict__ mpl, int Pc, int nbf_pad,
                                                     int nk, int ntile2, int nspin, int off0, int cnt0,
                                                     int off1, int cnt1,
-                                                    const unsigned short* __restrict__ smask,
+                                                    const unsigned short* __restrict__ smask, int nslot,
                                                     int p_per_split, int beta, double* __restrict__ kpart,
                                                     size_t slot) {
     __shared__ __bf16 lds[C::LDS_ELEMS];
     const int w = blockIdx.x, xcd = w % kXcdB, kq = w / kXcdB;
     const size_t t = (size_t)(kq % ntile2);
     const int rest = kq / ntile2, spin = rest % nspin, split = (rest / nspin) * kXcdB + xcd;
+    const int Pb = split * p_per_split, Pe = min(Pc, Pb + p_per_split);
+    if (split >= nslot || (beta && Pb >= Pe)) return;   // uniform exit
     size_t tn = (size_t)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
     while (tri_b(tn) > t) --tn;
     while (tri_b(tn + 1) <= t) ++tn;
@@ -216,7 +218,6 @@ __global__ __launch_bounds__(C::NT) void k_bf_ksyrk(const __bf16* __restrict__ m
     const int mu0 = (int)tm * C::WGY, nu0 = (int)tn * C::WGX;
     const int cb = spin == 0 ? off0 : off1, cnt = spin == 0 ? cnt0 : cnt1;
     const int ncb = (cnt + C::TK - 1) / C::TK;
-    const int Pb = split * p_per_split, Pe = min(Pc, Pb + p_per_split);
     const int nq = (Pe > Pb ? Pe - Pb : 0) * ncb;
     const size_t mplane = (size_t)Pc * nbf_pad * nk, mP = (size_t)nbf_pad * nk;
     bft::f4 acc[C::FX][C::FY];
@@ -320,10 +321,10 @@ hipError_t bf_ksyrk_t(hipStream_t st, const void* mpl, size_t Pc, const KPlan& k
                       int beta, double* kpart) {
     const size_t nt = kp.nbf_pad / C::WGX, nt2 = nt * (nt + 1) / 2;
     const int pps = (int)((Pc + kp.nsplit - 1) / kp.nsplit);
-    const size_t nwg = kp.nsplit * (size_t)nspin * nt2;
+    const size_t nwg = round_up(kp.nslot, kXcdB) * (size_t)nspin * nt2;
     hipLaunchKernelGGL(k_bf_ksyrk<C>, dim3((unsigned)nwg), dim3(C::NT), 0, st, (const __bf16*)mpl, (int)Pc,
                        (int)kp.nbf_pad, (int)kp.nk, (int)nt2, nspin, (int)kp.col_off[0], (int)kp.col_cnt[0],
-                       (int)kp.col_off[1], (int)kp.col_cnt[1], (const unsigned short*)smask, pps, beta, kpart,
+                       (int)kp.col_off[1], (int)kp.col_cnt[1], (const unsigned short*)smask, (int)kp.nslot, pps, beta, kpart,
                        kp.nbf_pad * kp.nbf_pad);
     return hipGetLastError();
 }

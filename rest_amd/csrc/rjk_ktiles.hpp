@@ -15,7 +15,7 @@ namespace kt {
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-constexpr int kBlock = 256;           // 4 waves, 2×2
+constexpr int kBlock = 256;           // 4 waves
 constexpr int TK = kTileK;            // 16
 // LDS row padding (elements).  FP64: rows of 128 + 2 (or 64 + 2) doubles put the 16 rows that
 // one transposed stash instruction writes (one element each, 16 lanes at a time) on 16 distinct
@@ -33,6 +33,11 @@ __device__ inline size_t tri(size_t j) { return j * (j + 1) / 2; }
 // so these accesses stay global loads and stores.
 #define RJK_GLB __attribute__((address_space(1)))
 template <typename T> __device__ __forceinline__ RJK_GLB T* glb(T* p) { return (RJK_GLB T*)p; }
+
+// Rotation of a work-group's rows over its waves.  Work-groups that share a CU are about 32 apart in
+// the XCD-local order, so neighbours on a CU get different rotations and the waves that skip padding
+// or below-diagonal fragments do not all sit on the same SIMD.
+__device__ __forceinline__ int rotation(int kq) { return (kq + kq / 32) & 3; }
 
 // One 16x16x4 MFMA per element type.  Lane l supplies A[l%16][l/16] and
 // B[l/16][l%16]; register r of lane l holds D[row(l, r)][l%16] (probed on
@@ -64,63 +69,123 @@ __device__ inline void upper_tile(size_t t, size_t* tm, size_t* tn) {
     *tm = t - tri(n);
 }
 
+// What bounds these tiles: on gfx950 the FP64 and FP32 MFMAs run at the rate of the vector unit and
+// keep it busy, so every other vector instruction of any wave on that SIMD costs about 5 cycles of
+// MFMA time (measured: 8 FP64 MFMAs alone 523 cycles a wave, with 64 integer instructions 859; FP32
+// 274 and 595; BF16 MFMAs overlap with them).  The tiles therefore address memory through wave-
+// uniform bases (scalar registers) plus lane offsets that stay the same for the whole tile, and
+// choose the way an operand is read per k-block by scalar branches: 20-40 vector instructions per
+// k-block of 16 (32-64 MFMAs) in place of about 250.
+template <typename T, int N> struct VecOf {
+    typedef T raw __attribute__((ext_vector_type(N)));
+    typedef T type __attribute__((ext_vector_type(N), aligned(sizeof(T))));   // element alignment
+};
+template <typename T> __device__ __forceinline__ RJK_GLB const T* as_glb(const T* p) { return (RJK_GLB const T*)p; }
+template <typename T> __device__ __forceinline__ RJK_GLB const T* as_glb(RJK_GLB const T* p) { return p; }
+// N elements at base (uniform) + off bytes (per lane)
+template <typename T, int N>
+__device__ __forceinline__ typename VecOf<T, N>::raw ldv(RJK_GLB const T* base, unsigned off) {
+    return *(RJK_GLB const typename VecOf<T, N>::type*)((RJK_GLB const char*)base + off);
+}
+
 // ---------------------------------------------------------------------------
 // Stage 1: M'[P][c][μ] = Σ_ν Bsym_P[μ,ν] C'[ν][c], one (μ-tile, c-tile) of one
-//   auxiliary column.  Software pipeline: the next k-block is fetched into
-//   registers while the MFMAs consume the current one from LDS; LDS is
-//   double-buffered, one barrier per k-block.
+//   auxiliary column: 64·FM μ rows on 4 waves, 16·FN columns c.  The caller picks
+//   FN so that few columns are padding; a wave whose 16·FM rows all lie beyond nbf
+//   skips its MFMAs, and `rot` rotates the rows over the waves so that the skipped
+//   ones fall on different SIMDs.  Rows μ >= nbf of M' are left unwritten or hold
+//   finite padding: nothing reads them into an output.  Software pipeline: the next
+//   k-block is fetched into registers while the MFMAs consume the current one from
+//   LDS (double-buffered, one barrier per k-block).  Sums run over ν in ascending
+//   order whatever the tile, so M' does not depend on FM and FN.
+//
+//   Reading the packed column (element (i <= j) at tri(j) + i):
+//     blocks left of the tile's diagonal range (ν < mu0): along ν, two elements a lane at
+//       offsets fixed for the tile, the base moving by 16 elements a block;
+//     blocks beyond it (ν >= mu0 + 64 FM): row ν is contiguous in μ, one row per wave
+//       instruction at a scalar base;
+//     the diagonal blocks and a partial last block: element by element, mirrored and masked.
 // ---------------------------------------------------------------------------
 template <typename T, int FM, int FN, typename BP, typename CP, typename MP>
-__device__ __forceinline__ void khalf_tile(BP __restrict__ bcol, int nbf, int mu0, int c0, CP __restrict__ cocc,
-                                           int nk, int ldm, MP __restrict__ mP) {
+__device__ __forceinline__ void khalf_tile(BP __restrict__ bcol_, int nbf, int mu0, int c0, CP __restrict__ cocc_,
+                                           int nk, int ldm, MP __restrict__ mP, int rot) {
     using MM = Mma<T>;
-    constexpr int TM = 2 * FM * 16, TN = 2 * FN * 16;
-    constexpr int NA = TK * TM / kBlock, NB = TK * TN / kBlock;
-    __shared__ T As[2][TK][TM + Pad<T>::v];
-    __shared__ T Bs[2][TK][TN + Pad<T>::v];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-    T ra[NA], rb[NB];
-    unsigned live = 0;   // bit r: element r of the A fetch lies inside nbf×nbf
+    constexpr int TM = 64 * FM, TN = 16 * FN, NA = 4 * FM;
+    constexpr int VB = 16 / (int)sizeof(T), PRB = TN / VB, NPB = TK * PRB, NB = (NPB + kBlock - 1) / kBlock;
+    using VA = typename VecOf<T, FM>::raw;
+    using V2 = typename VecOf<T, 2>::raw;
+    using VBt = typename VecOf<T, VB>::raw;
+    __shared__ __align__(16) T As[2][TK][TM + Pad<T>::v];
+    __shared__ __align__(16) T Bs[2][TK][TN + Pad<T>::v];
+    const auto bcol = as_glb(bcol_);
+    const auto cocc = as_glb(cocc_);
+    const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ws = (wave + rot) & 3;
+    T ra[NA];
+    VBt rb[NB];
+    unsigned live = 0;   // element-wise blocks: bit r set when element r lies inside nbf × nbf
+    if (mu0 >= nbf) return;   // a tile of padding rows only (nbf_pad beyond the tile grid); uniform
 
-    // A tile As[k][mm] = Bsym(mu0+mm, nu0+k).  Tiles wholly below the diagonal
-    // are read along ν (contiguous there), all others along μ.  Out-of-range
-    // elements read a valid address and are zeroed when stashed, so nothing
-    // waits on the loads before the MFMAs of the current block.
-    auto fetch = [&](int nu0) {
-        live = 0;
-        if (mu0 >= nu0 + TK - 1) {
+    // lane offsets (bytes), fixed for the tile
+    unsigned offd[2 * FM], offb[NB];
 #pragma unroll
-            for (int r = 0; r < NA; ++r) {
-                const int e = tid + r * kBlock, k = e % TK, mm = e / TK;
-                const int mu = mu0 + mm, nu = nu0 + k;
-                const bool ok = mu < nbf && nu < nbf;
-                live |= (unsigned)ok << r;
-                ra[r] = bcol[ok ? tri((size_t)mu) + nu : 0];
+    for (int r = 0; r < 2 * FM; ++r) {
+        const int mu = min(mu0 + (tid >> 3) + 32 * r, nbf - 1);
+        offd[r] = (unsigned)((tri((size_t)mu) - tri((size_t)mu0) + (tid & 7) * 2) * sizeof(T));
+    }
+#pragma unroll
+    for (int r = 0; r < NB; ++r) {
+        const int e = min(tid + r * kBlock, NPB - 1);
+        offb[r] = (unsigned)(((e / PRB) * nk + (e % PRB) * VB) * sizeof(T));
+    }
+    const unsigned offa = lane * FM * sizeof(T);
+
+    enum { BELOW, ABOVE, MIXED };
+    auto fetch = [&](auto kind, int nu0) {
+        if constexpr (kind() == BELOW) {
+            const auto p = bcol + tri((size_t)mu0) + nu0;
+#pragma unroll
+            for (int r = 0; r < 2 * FM; ++r) {
+                const V2 v = ldv<T, 2>(p, offd[r]);
+                ra[2 * r] = v[0];
+                ra[2 * r + 1] = v[1];
+            }
+        } else if constexpr (kind() == ABOVE) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const VA v = ldv<T, FM>(bcol + tri((size_t)(nu0 + wave + 4 * r)) + mu0, offa);
+#pragma unroll
+                for (int q = 0; q < FM; ++q) ra[r * FM + q] = v[q];
             }
         } else {
+            live = 0;
 #pragma unroll
             for (int r = 0; r < NA; ++r) {
-                const int e = tid + r * kBlock, mm = e % TM, k = e / TM;
-                const int mu = mu0 + mm, nu = nu0 + k;
+                const int e = tid + r * kBlock, mu = mu0 + e % TM, nu = nu0 + e / TM;
                 const int lo = mu < nu ? mu : nu, hi = mu < nu ? nu : mu;
-                const bool ok = mu < nbf && nu < nbf;
+                const bool ok = hi < nbf;
                 live |= (unsigned)ok << r;
                 ra[r] = bcol[ok ? tri((size_t)hi) + lo : 0];
             }
         }
+        const auto q = cocc + (size_t)nu0 * nk + c0;   // C' rows are zero-padded beyond nbf
 #pragma unroll
-        for (int r = 0; r < NB; ++r) {
-            const int e = tid + r * kBlock, cc = e % TN, k = e / TN;
-            rb[r] = cocc[(size_t)(nu0 + k) * nk + c0 + cc];   // C' rows are zero-padded to nbf_pad
-        }
+        for (int r = 0; r < NB; ++r) rb[r] = ldv<T, VB>(q, offb[r]);
     };
-    auto stash = [&](int buf, int nu0) {
-        if (mu0 >= nu0 + TK - 1) {
+    auto stash = [&](auto kind, int buf) {
+        if constexpr (kind() == BELOW) {
 #pragma unroll
-            for (int r = 0; r < NA; ++r) {
-                const int e = tid + r * kBlock;
-                As[buf][e % TK][e / TK] = ((live >> r) & 1u) ? ra[r] : T(0);
+            for (int r = 0; r < 2 * FM; ++r) {
+                As[buf][(tid & 7) * 2][(tid >> 3) + 32 * r] = ra[2 * r];
+                As[buf][(tid & 7) * 2 + 1][(tid >> 3) + 32 * r] = ra[2 * r + 1];
+            }
+        } else if constexpr (kind() == ABOVE) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                VA v;
+#pragma unroll
+                for (int q = 0; q < FM; ++q) v[q] = ra[r * FM + q];
+                *(VA*)&As[buf][wave + 4 * r][lane * FM] = v;
             }
         } else {
 #pragma unroll
@@ -132,7 +197,7 @@ __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol, int nbf, int mu
 #pragma unroll
         for (int r = 0; r < NB; ++r) {
             const int e = tid + r * kBlock;
-            Bs[buf][e / TN][e % TN] = rb[r];
+            if ((r + 1) * kBlock <= NPB || e < NPB) *(VBt*)&Bs[buf][e / PRB][(e % PRB) * VB] = rb[r];
         }
     };
 
@@ -141,134 +206,189 @@ __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol, int nbf, int mu
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = MM::zero();
-
-    const int nkb = (nbf + TK - 1) / TK;
-    fetch(0);
-    stash(0, 0);
-    __syncthreads();
-    for (int kb = 0; kb < nkb; ++kb) {
-        const int cur = kb & 1;
-        const bool more = kb + 1 < nkb;
-        if (more) fetch((kb + 1) * TK);
+    const int mrow = ws * 16 * FM;
+    const bool act = mu0 + mrow < nbf;   // wave-uniform
+    auto compute = [&](int cur) {
+        if (!act) return;
 #pragma unroll
         for (int kk = 0; kk < TK; kk += 4) {
             T bmu[FM], ac[FN];
 #pragma unroll
-            for (int i = 0; i < FM; ++i) bmu[i] = As[cur][kk + (lane >> 4)][wm * FM * 16 + i * 16 + (lane & 15)];
+            for (int i = 0; i < FM; ++i) bmu[i] = As[cur][kk + g][mrow + i * 16 + l16];
 #pragma unroll
-            for (int j = 0; j < FN; ++j) ac[j] = Bs[cur][kk + (lane >> 4)][wn * FN * 16 + j * 16 + (lane & 15)];
+            for (int j = 0; j < FN; ++j) ac[j] = Bs[cur][kk + g][j * 16 + l16];
             // D[c][μ] = Σ_ν C'[ν][c] Bsym[ν][μ]
 #pragma unroll
             for (int i = 0; i < FM; ++i)
 #pragma unroll
                 for (int j = 0; j < FN; ++j) acc[i][j] = MM::op(ac[j], bmu[i], acc[i][j]);
         }
-        if (more) stash(cur ^ 1, (kb + 1) * TK);
-        __syncthreads();
-    }
+    };
 
+    // k-blocks [0, e0) below the diagonal range, [e0, e1) across it, [e1, e2) above, [e2, nkb) the partial last
+    const int nkb = (nbf + TK - 1) / TK;
+    const int e0 = mu0 / TK, e1 = min(nkb, (mu0 + TM) / TK), e2 = max(e1, nbf / TK);
+    struct KB { __device__ constexpr int operator()() const { return BELOW; } };
+    struct KA { __device__ constexpr int operator()() const { return ABOVE; } };
+    struct KX { __device__ constexpr int operator()() const { return MIXED; } };
+    int kb = 0;
+    auto run = [&](auto kind, int end) {   // blocks up to `end` are of this kind; block kb is in LDS
+        for (; kb + 1 < end; ++kb) {
+            fetch(kind, (kb + 1) * TK);
+            compute(kb & 1);
+            stash(kind, (kb + 1) & 1);
+            __syncthreads();
+        }
+    };
+    if (e0 > 0) {
+        fetch(KB(), 0);
+        stash(KB(), 0);
+    } else {
+        fetch(KX(), 0);
+        stash(KX(), 0);
+    }
+    __syncthreads();
+    run(KB(), e0);
+    run(KX(), e1);
+    run(KA(), e2);
+    run(KX(), nkb);
+    compute(kb & 1);
+    __syncthreads();   // the persistent callers start their next tile in the same LDS
+
+    if (!act) return;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-            const int mu = mu0 + wm * FM * 16 + i * 16 + (lane & 15);
-            const int cb = c0 + wn * FN * 16 + j * 16;
+            const int mu = mu0 + mrow + i * 16 + l16, cb = c0 + j * 16;
 #pragma unroll
             for (int r = 0; r < 4; ++r) mP[(size_t)(cb + MM::row(lane, r)) * ldm + mu] = acc[i][j][r];
         }
 }
 
-
 // ---------------------------------------------------------------------------
-// Stage 2: Kpart (+)= Σ_{P,c} M'[P][c][μ] sign_c M'[P][c][ν] over the upper tiles.
-//   1-D grid of nsplit × nspin × ntile(ntile+1)/2 work-groups, nsplit a
-//   multiple of 8; split s runs entirely on XCD s % 8, so the M' slab of a
-//   split is streamed into one L2 and shared by all tiles there.  Same
-//   pipeline as stage 1 over the flattened (P, 16-column block) index;
-//   accumulation in the MFMA type, partial tiles kept in FP64.
+// Stage 2: Kpart (+)= Σ_{P,c} M'[P][c][μ] sign_c M'[P][c][ν] over the upper tiles
+//   (mu0 <= nu0) of 64·FB × 64·FB, split-K over P.  Wave w owns 16·FB columns ν and
+//   every row μ of the tile; in a diagonal tile it computes only the μ groups up to its
+//   own (10 of 16 groups), and a wave whose columns all lie beyond nbf computes nothing
+//   (`rot` as in stage 1).  Same pipeline as stage 1 over the flattened (P, 16-column block) index;
+//   the rows of M' are wave-uniform, so every load is one row at a scalar base.  Signs
+//   are looked at once per tile and applied while staging only where one is negative.
+//   Accumulation in the MFMA type, partial tiles kept in FP64.
 // ---------------------------------------------------------------------------
 struct SyrkCols {
     int off[2], cnt[2];
 };
 
-template <typename T, int F, typename MP, typename SP, typename KP>
-__device__ __forceinline__ void ksyrk_tile(MP __restrict__ m, int ldm, int nk, int mu0, int nu0, int cb, int ncb,
-                                           int Pb, int Pe, SP __restrict__ sign, int beta, KP __restrict__ kp) {
+template <typename T, int FB, bool DIAG, typename MP, typename SP, typename KP>
+__device__ __forceinline__ void ksyrk_body(MP m, int ldm, int nk, int nbf, int mu0, int nu0, int cb, int ncb, int Pb,
+                                           int Pe, SP sign, int beta, KP kp, int ws, bool neg, T* __restrict__ lds) {
     using MM = Mma<T>;
-    constexpr int Tt = 2 * F * 16;
-    constexpr int NL = TK * Tt / kBlock;
-    __shared__ T As[2][TK][Tt + Pad<T>::v];
-    __shared__ T Bs[2][TK][Tt + Pad<T>::v];
-    __shared__ T Ss[2][TK];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
+    constexpr int FA = 4 * FB, Tt = 64 * FB, LD = Tt + Pad<T>::v;
+    using VL = typename VecOf<T, FB>::raw;
+    const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto As = [&](int buf, int k) { return lds + (buf * TK + k) * LD; };
+    auto Bs = [&](int buf, int k) { return lds + ((2 + buf) * TK + k) * LD; };
     const int nq = (Pe > Pb ? Pe - Pb : 0) * ncb;
-    T ra[NL], rb[NL], rsg = T(0);
-
-    // raw loads only (the k-block's signs go to LDS and are applied to the
-    // fragments), so the loads stay in flight across the current block's MFMAs
-    auto fetch = [&](int q) {
-        const int P = Pb + q / ncb, c = cb + (q % ncb) * TK;
-        const auto base = m + ((size_t)P * nk + c) * ldm;
+    const unsigned off = lane * FB * sizeof(T);
+    VL ra[4], rb[4];
+    T rs[4];
+    int fP = Pb, fc = 0;   // (P, block) of the next fetch
+    auto fetch = [&]() {
+        const auto base = m + ((size_t)fP * nk + cb + fc * TK + wave) * ldm;
 #pragma unroll
-        for (int r = 0; r < NL; ++r) {
-            const int e = tid + r * kBlock, mm = e % Tt, k = e / Tt;
-            ra[r] = base[(size_t)k * ldm + mu0 + mm];
-            rb[r] = base[(size_t)k * ldm + nu0 + mm];
+        for (int r = 0; r < 4; ++r) {
+            if constexpr (!DIAG) ra[r] = ldv<T, FB>(base + (size_t)(4 * r) * ldm + mu0, off);
+            rb[r] = ldv<T, FB>(base + (size_t)(4 * r) * ldm + nu0, off);
         }
-        if (tid < TK) rsg = sign[c + tid];
+        if (neg) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) rs[r] = sign[cb + fc * TK + wave + 4 * r];
+        }
+        if (++fc == ncb) {
+            fc = 0;
+            ++fP;
+        }
     };
+    // a diagonal tile stages its rows once, and a second time with the signs where one is negative
     auto stash = [&](int buf) {
 #pragma unroll
-        for (int r = 0; r < NL; ++r) {
-            const int e = tid + r * kBlock;
-            As[buf][e / Tt][e % Tt] = ra[r];
-            Bs[buf][e / Tt][e % Tt] = rb[r];
+        for (int r = 0; r < 4; ++r) {
+            if constexpr (DIAG) *(VL*)(As(buf, wave + 4 * r) + lane * FB) = rb[r];
+            else *(VL*)(As(buf, wave + 4 * r) + lane * FB) = ra[r];
+            if (!DIAG || neg) *(VL*)(Bs(buf, wave + 4 * r) + lane * FB) = neg ? rb[r] * rs[r] : rb[r];
         }
-        if (tid < TK) Ss[buf][tid] = rsg;
     };
-
-    typename MM::acc_t acc[F][F];
+    typename MM::acc_t acc[FA][FB];
 #pragma unroll
-    for (int i = 0; i < F; ++i)
+    for (int i = 0; i < FA; ++i)
 #pragma unroll
-        for (int j = 0; j < F; ++j) acc[i][j] = MM::zero();
-
+        for (int j = 0; j < FB; ++j) acc[i][j] = MM::zero();
+    const int ncol = ws * 16 * FB;
+    const bool act = nu0 + ncol < nbf;
+    const int bsel = (!DIAG || neg) ? 2 * TK * LD : 0;   // where the ν operand lies
+    auto compute = [&](int cur) {
+        if (!act) return;
+        const T* __restrict__ a0 = As(cur, g) + l16;
+        const T* __restrict__ b0 = As(cur, g) + bsel + ncol + l16;
+        // D[ν][μ] = Σ_k sign_k M'[k][ν] M'[k][μ]
+        if constexpr (DIAG) {
+            T anu[TK / 4][FB];
+#pragma unroll
+            for (int kk = 0; kk < TK; kk += 4)
+#pragma unroll
+                for (int j = 0; j < FB; ++j) anu[kk / 4][j] = b0[kk * LD + j * 16];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (q > ws) break;   // groups of FB fragments; those right of the wave's own are below the diagonal
+#pragma unroll
+                for (int kk = 0; kk < TK; kk += 4) {
+                    T bmu[FB];
+#pragma unroll
+                    for (int i = 0; i < FB; ++i) bmu[i] = a0[kk * LD + (q * FB + i) * 16];
+#pragma unroll
+                    for (int i = 0; i < FB; ++i)
+#pragma unroll
+                        for (int j = 0; j < FB; ++j)
+                            acc[q * FB + i][j] = MM::op(anu[kk / 4][j], bmu[i], acc[q * FB + i][j]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < TK; kk += 4) {
+                T bmu[FA], anu[FB];
+#pragma unroll
+                for (int j = 0; j < FB; ++j) anu[j] = b0[kk * LD + j * 16];
+#pragma unroll
+                for (int i = 0; i < FA; ++i) bmu[i] = a0[kk * LD + i * 16];
+#pragma unroll
+                for (int i = 0; i < FA; ++i)
+#pragma unroll
+                    for (int j = 0; j < FB; ++j) acc[i][j] = MM::op(anu[j], bmu[i], acc[i][j]);
+            }
+        }
+    };
     if (nq > 0) {
-        fetch(0);
+        fetch();
         stash(0);
     }
     __syncthreads();
-    // branch-free body (one basic block keeps the accumulators in place):
-    // the last iteration re-fetches its own block and stashes it into the
-    // idle buffer, which nothing reads afterwards
-    for (int q = 0; q < nq; ++q) {
-        const int cur = q & 1;
-        fetch(q + 1 < nq ? q + 1 : q);
-#pragma unroll
-        for (int kk = 0; kk < TK; kk += 4) {
-            T bmu[F], anu[F];
-            const T sg = Ss[cur][kk + (lane >> 4)];
-#pragma unroll
-            for (int i = 0; i < F; ++i) bmu[i] = As[cur][kk + (lane >> 4)][wm * F * 16 + i * 16 + (lane & 15)];
-#pragma unroll
-            for (int j = 0; j < F; ++j) anu[j] = sg * Bs[cur][kk + (lane >> 4)][wn * F * 16 + j * 16 + (lane & 15)];
-            // D[ν][μ] = Σ_k sign_k M'[k][ν] M'[k][μ]
-#pragma unroll
-            for (int i = 0; i < F; ++i)
-#pragma unroll
-                for (int j = 0; j < F; ++j) acc[i][j] = MM::op(anu[j], bmu[i], acc[i][j]);
-        }
-        stash(cur ^ 1);
+    for (int q = 0; q + 1 < nq; ++q) {
+        fetch();
+        compute(q & 1);
+        stash((q + 1) & 1);
         __syncthreads();
     }
-
+    if (nq > 0) compute((nq - 1) & 1);
+    __syncthreads();   // the persistent callers start their next tile in the same LDS
+    if (!act) return;
 #pragma unroll
-    for (int i = 0; i < F; ++i)
+    for (int i = 0; i < FA; ++i) {
+        if (DIAG && i / FB > ws) break;
 #pragma unroll
-        for (int j = 0; j < F; ++j) {
-            const int mu = mu0 + wm * F * 16 + i * 16 + (lane & 15);
-            const int nb = nu0 + wn * F * 16 + j * 16;
+        for (int j = 0; j < FB; ++j) {
+            const int mu = mu0 + i * 16 + l16, nb = nu0 + ncol + j * 16;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const auto dst = kp + (size_t)(nb + MM::row(lane, r)) * ldm + mu;
@@ -277,6 +397,25 @@ __device__ __forceinline__ void ksyrk_tile(MP __restrict__ m, int ldm, int nk, i
                 *dst = v;
             }
         }
+    }
+}
+
+template <typename T, int FB, typename MP, typename SP, typename KP>
+__device__ __forceinline__ void ksyrk_tile(MP __restrict__ m, int ldm, int nk, int nbf, int mu0, int nu0, int cb,
+                                           int ncb, int Pb, int Pe, SP __restrict__ sign, int beta,
+                                           KP __restrict__ kp, int rot) {
+    constexpr int LD = 64 * FB + Pad<T>::v;
+    __shared__ __align__(16) T lds[4 * TK * LD];
+    const int ws = (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) + rot) & 3;
+    if (nu0 >= nbf) return;   // padding columns only (uniform)
+    int any = 0;
+    for (int c = threadIdx.x; c < ncb * TK; c += kBlock) any |= sign[cb + c] < T(0);
+    const bool neg = __syncthreads_or(any) != 0;
+    const auto mg = as_glb(m);
+    if (mu0 == nu0)
+        ksyrk_body<T, FB, true>(mg, ldm, nk, nbf, mu0, nu0, cb, ncb, Pb, Pe, sign, beta, kp, ws, neg, lds);
+    else
+        ksyrk_body<T, FB, false>(mg, ldm, nk, nbf, mu0, nu0, cb, ncb, Pb, Pe, sign, beta, kp, ws, neg, lds);
 }
 
 
