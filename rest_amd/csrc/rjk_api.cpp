@@ -452,17 +452,53 @@ extern "C" int rjk_vj_upper_with_ri_v_sync(rjk_ctx* ctx, const double* dm, size_
 // ---------------------------------------------------------------------------
 namespace {
 
-// FP64/FP32 tile rows.  128-row tiles share each fetched operand among more MFMAs; 64-row ones
-// are taken where nbf fits one of them.
-size_t k_tile(size_t nbf) { return nbf <= 64 ? 64 : 128; }
+// FP64/FP32 SYRK tile rows, 64 or 128.  A tile's four waves each own a quarter and skip it where it
+// lies beyond nbf or below the diagonal, so the work goes by blocks of 32 or 64 functions.  FP32
+// takes 64 throughout (nbf 900: 5.6 ms against 6.7; nbf 576: 0.99 against 1.39).  FP64 128-row tiles
+// run 71/66 as fast but leave fewer, longer work-groups: nbf 1536 89 ms against 98, 768 5.78 against 5.86,
+// 1100 (pads more) 18.1 against 17.9, 560 2.1 against 1.6.
+size_t k_tile(size_t nbf, int prec) {
+    if (prec != RJK_PREC_FP64 || nbf <= 640) return 64;
+    auto work = [&](size_t blk) {
+        const double n = (double)((nbf + blk - 1) / blk);
+        return n * (n + 1) / 2 * (double)(blk * blk);
+    };
+    return work(32) * 71.0 < work(64) * 66.0 ? 64 : 128;
+}
+
+// Split-K divisor of the FP64 SYRK for chunks of Pc columns: of the multiples of 8 (one XCD a split),
+// the one with the least of compute time over the share of work-group slots that the last round
+// fills, plus the time to write and sum the partial tiles.
+size_t k_splits(const KPlan& kp, int ns, size_t Pc, size_t cap) {
+    const double nt = (double)(kp.nbf_pad / kp.tile), t2 = nt * (nt + 1) / 2, tile = (double)(kp.tile * kp.tile);
+    const double slots = kp.tile == 64 ? 1024 : 512;   // resident work-groups: 4 or 2 a CU
+    const double cols = (double)(kp.col_cnt[0] + kp.col_cnt[1]);
+    const double flop = 2.0 * t2 * tile * cols * (double)Pc;
+    size_t best = 8;
+    double cost = 1e300;
+    for (size_t n = 8; n <= cap; n += 8) {
+        const double wg = t2 * ns * (double)n, rounds = std::ceil(wg / slots);
+        const double pps = std::ceil((double)Pc / (double)n);          // whole columns a split
+        const double used = std::ceil((double)Pc / pps);
+        const double c = flop / 65e12 * (rounds * slots / wg) * (pps * (double)n / (double)Pc) +
+                         2.0 * 8.0 * used * ns * t2 * tile / 4e12;
+        if (c < cost) {
+            cost = c;
+            best = n;
+        }
+    }
+    return best;
+}
 
 // 16-column groups of a half-transform tile for f groups in all: the tile that leaves the fewest
 // padding columns, a tile costing about one group beyond its columns (its share of staging B);
-// never more columns than 64-column tiles would pad to.
-int k_tile_groups(size_t f) {
+// never more columns than 64-column tiles would pad to.  FP64 stops at 5 groups (beyond, only two
+// work-groups share a CU), FP32 at 8.
+int k_tile_groups(size_t f, int prec) {
     int best = 4;
     size_t cost = (f + 3) / 4 * 5;
-    for (int fn = 1; fn <= 6; ++fn) {
+    for (int fn : {1, 2, 3, 5, 6, 8}) {
+        if (fn > 5 && prec == RJK_PREC_FP64) break;
         const size_t tiles = (f + fn - 1) / fn, c = tiles * (fn + 1);
         if (tiles * fn <= round_up(f, 4) && (c < cost || (c == cost && fn > best))) {
             cost = c;
@@ -474,7 +510,7 @@ int k_tile_groups(size_t f) {
 
 void k_plan_cols(KPlan& kp, size_t nbf, const size_t* ncol, int ns, int prec) {
     const size_t gran = is_bf16(prec) ? kBfColGran : kTileK;
-    kp.tile = is_bf16(prec) ? kTileMN : k_tile(nbf);
+    kp.tile = is_bf16(prec) ? kTileMN : k_tile(nbf, prec);
     kp.nbf_pad = round_up(nbf, kp.tile);
     kp.col_cnt[0] = round_up(ncol[0], gran);
     kp.col_off[0] = 0;
@@ -484,7 +520,7 @@ void k_plan_cols(KPlan& kp, size_t nbf, const size_t* ncol, int ns, int prec) {
     if (is_bf16(prec)) {
         kp.nk = round_up(tot, kColPad);
     } else {
-        kp.fn = k_tile_groups(tot / kTileK);
+        kp.fn = k_tile_groups(tot / kTileK, prec);
         kp.nk = round_up(tot, (size_t)kp.fn * kTileK);
     }
 }
@@ -503,21 +539,22 @@ size_t k_slots(size_t naux, size_t chunk, size_t nsplit) {
 // partial tiles are FP64.
 int k_plan_ws(rjk_ctx* ctx, KPlan& kp, int ns, int prec, void** cocc, void** sign, double** kpart, void** m) {
     const size_t es = k_elem_size(prec);
-    const size_t target = 1024;  // SYRK work-groups
     const size_t slot = kp.nbf_pad * kp.nbf_pad;
     const size_t perP = kp.nk * kp.nbf_pad * es;
     size_t nsplit, chunk;
     if (prec == RJK_PREC_FP64) {
-        // about `target` work-groups, at least 8 k-blocks a split, at most a quarter of the workspace
-        const size_t nt = kp.nbf_pad / kp.tile, ntiles = nt * (nt + 1) / 2;
         const size_t slot_bytes = (size_t)ns * slot * sizeof(double);
         const size_t small = round_up(kp.nbf_pad * kp.nk * es, 256) + round_up(kp.nk * es, 256);
-        const size_t blocks = std::max<size_t>(1, ctx->naux * std::max<size_t>(1, kp.nk / kTileK / ns));
-        nsplit = std::min(round_up(std::max<size_t>(1, target / (ntiles * ns)), 8), round_up((blocks + 7) / 8, 8));
-        nsplit = std::min(nsplit, std::max<size_t>(8, ((ctx->ws_limit / 4) / slot_bytes) / 8 * 8));
-        const size_t fixed = small + nsplit * slot_bytes;
-        const size_t avail = ctx->ws_limit > fixed ? ctx->ws_limit - fixed : 0;
-        chunk = perP ? std::min(ctx->naux, std::max<size_t>(1, avail / perP)) : ctx->naux;
+        const size_t cap = std::min(std::max<size_t>(8, ((ctx->ws_limit / 4) / slot_bytes) / 8 * 8),
+                                    std::min<size_t>(512, round_up(ctx->naux, 8)));
+        auto chunk_for = [&](size_t n) {
+            const size_t fixed = small + n * slot_bytes;
+            const size_t avail = ctx->ws_limit > fixed ? ctx->ws_limit - fixed : 0;
+            return perP ? std::min(ctx->naux, std::max<size_t>(1, avail / perP)) : ctx->naux;
+        };
+        nsplit = k_splits(kp, ns, chunk_for(8), cap);
+        chunk = chunk_for(nsplit);
+        chunk = (ctx->naux + (ctx->naux + chunk - 1) / chunk - 1) / ((ctx->naux + chunk - 1) / chunk);   // even chunks
     } else {
         // FP32 accumulators: each split sums at most kFp32Chain products (pps auxiliary
         // columns × nk) before its partial joins the FP64 sum, so rounding does not grow
@@ -528,7 +565,7 @@ int k_plan_ws(rjk_ctx* ctx, KPlan& kp, int ns, int prec, void** cocc, void** sig
         const size_t nt = pad / kTileMN, ntiles = nt * (nt + 1) / 2;
         const size_t slot_bytes = (size_t)ns * pad * pad * sizeof(double), perP_ = nk * pad * es;
         const size_t small = round_up(pad * nk * es, 256) + round_up(nk * es, 256);
-        nsplit = round_up(std::max<size_t>(1, target / (ntiles * ns)), 8);
+        nsplit = round_up(std::max<size_t>(1, 1024 / (ntiles * ns)), 8);   // about 1024 work-groups
         nsplit = std::min(nsplit, std::max<size_t>(8, ((ctx->ws_limit / 4) / slot_bytes) / 8 * 8));
         chunk = ctx->naux;
         if (nk > 0) {
@@ -665,9 +702,9 @@ int vk_dm_general(rjk_ctx* ctx, const double* dm_dev, int ns, double scale, doub
     const size_t nbf = ctx->nbf, n2 = nbf * nbf;
     hipStream_t st = ctx->stream;
     KPlan kp;
-    kp.tile = k_tile(nbf);
+    kp.tile = k_tile(nbf, RJK_PREC_FP64);
     kp.nbf_pad = round_up(nbf, kp.tile);
-    kp.fn = k_tile_groups((nbf + kTileK - 1) / kTileK);
+    kp.fn = k_tile_groups((nbf + kTileK - 1) / kTileK, RJK_PREC_FP64);
     kp.nk = round_up(nbf, (size_t)kp.fn * kTileK);
     kp.col_cnt[0] = kp.nk;
     const size_t ccol = kp.nbf_pad * kp.nk * sizeof(double);

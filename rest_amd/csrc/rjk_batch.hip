@@ -244,9 +244,9 @@ __global__ __launch_bounds__(kBlock) void k_b_khalf(const BProb* __restrict__ pr
     }
 }
 
-template <typename T, int FB>
+template <typename T, int F>
 __global__ __launch_bounds__(kBlock) void k_b_ksyrk(const BProb* __restrict__ pr, int np, Tables tb) {
-    constexpr int Tt = 64 * FB;
+    constexpr int Tt = 32 * F;
     const size_t total = tb.syrk[np];
     for (size_t it = blockIdx.x; it < total; it += gridDim.x) {
         const int q = find_prob(tb.syrk, np, it);
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(kBlock) void k_b_ksyrk(const BProb* __restrict__ pr
         size_t tm, tn;
         upper_tile(t, &tm, &tn);
         const int Pb = split * P.pps, Pe = min(P.naux, Pb + P.pps);
-        ksyrk_tile<T, FB>(glb((const T*)P.m), P.nbf_pad, P.nk, P.nbf, (int)tm * Tt, (int)tn * Tt, 0, P.ncb, Pb, Pe,
+        ksyrk_tile<T, F>(glb((const T*)P.m), P.nbf_pad, P.nk, P.nbf, (int)tm * Tt, (int)tn * Tt, 0, P.ncb, Pb, Pe,
                           glb((const T*)P.sign), 0, glb(P.kpart) + (size_t)split * P.nbf_pad * P.nbf_pad,
                           rotation((int)kq));
     }
@@ -799,7 +799,7 @@ int enqueue_fp(rjk_batch* b, hipEvent_t* ev) {
         hipLaunchKernelGGL((k_b_khalf<T, 2, 4>), dim3(grid_items(b, b->t_sub_items[3], b->waves)), dim3(kBlock), 0,
                            st, b->d_prob, b->d_sub + 3 * np, b->d_suboff + 3 * (np + 1), b->t_sub_n[3]);
     mark(6);
-    hipLaunchKernelGGL((k_b_ksyrk<T, 2>), dim3(grid_items(b, b->t_syrk.back(), b->waves)), dim3(kBlock), 0, st,
+    hipLaunchKernelGGL((k_b_ksyrk<T, 4>), dim3(grid_items(b, b->t_syrk.back(), b->waves)), dim3(kBlock), 0, st,
                        b->d_prob, np, tb);
     mark(7);
     mark(8);

@@ -128,8 +128,8 @@ void j_plan(size_t ldb, size_t naux, int prec, size_t* nchunk, size_t* nsplit);
 
 // K
 struct KPlan {
-    size_t tile = kTileMN;   // FP64/FP32: rows of the half-transform and SYRK tiles (64 or 128)
-    int fn = 4;              // FP64/FP32: 16-column groups of a half-transform tile (1..6)
+    size_t tile = kTileMN;   // SYRK tile rows (64 or 128; BF16: kTileMN)
+    int fn = 4;              // FP64/FP32: 16-column groups of a half-transform tile
     size_t nbf_pad = 0;      // multiple of `tile`; BF16: of kTileMN
     size_t nk = 0;           // padded occupied columns, all spins (multiple of 16·fn; BF16: of kColPad)
     size_t col_off[2] = {0, 0}, col_cnt[2] = {0, 0};   // per-spin column ranges (multiples of 16)

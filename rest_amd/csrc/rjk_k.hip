@@ -35,7 +35,7 @@ using namespace kt;
 // share it in that XCD's L2.
 // ---------------------------------------------------------------------------
 template <typename T, int FM, int FN>
-__global__ __launch_bounds__(kBlock) void k_khalf(const T* __restrict__ b, size_t ldb, int nbf, size_t P0, int Pc,
+__global__ __launch_bounds__(kBlock, 3) void k_khalf(const T* __restrict__ b, size_t ldb, int nbf, size_t P0, int Pc,
                                                   int ntm, int ntc, const T* __restrict__ cocc, int nk, int ldm,
                                                   T* __restrict__ m) {
     constexpr int TM = 64 * FM, TN = 16 * FN;
@@ -53,12 +53,12 @@ __global__ __launch_bounds__(kBlock) void k_khalf(const T* __restrict__ b, size_
 // work-groups; split s runs entirely on XCD s % 8, so the M' slab of a split is
 // streamed into one L2 and shared by all tiles there.
 // ---------------------------------------------------------------------------
-template <typename T, int FB>
+template <typename T, int F>
 __global__ __launch_bounds__(kBlock) void k_ksyrk(const T* __restrict__ m, int ldm, int nk, int nbf, int Pc,
                                                   int ntile2, int nspin, SyrkCols cols, const T* __restrict__ sign,
                                                   int nslot, int p_per_split, int beta, double* __restrict__ kpart,
                                                   size_t slot) {
-    constexpr int Tt = 64 * FB;
+    constexpr int Tt = 32 * F;
     // XCD-aware decode: w -> (split on XCD w%8, spin, tile)
     const int w = blockIdx.x, xcd = w % kXcd, kq = w / kXcd;
     const size_t t = (size_t)(kq % ntile2);
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kBlock) void k_ksyrk(const T* __restrict__ m, int l
     if (split >= nslot || (beta && Pb >= Pe)) return;   // uniform exit
     size_t tm, tn;
     upper_tile(t, &tm, &tn);
-    ksyrk_tile<T, FB>(m, ldm, nk, nbf, (int)tm * Tt, (int)tn * Tt, cols.off[spin], cols.cnt[spin] / TK, Pb, Pe, sign,
+    ksyrk_tile<T, F>(m, ldm, nk, nbf, (int)tm * Tt, (int)tn * Tt, cols.off[spin], cols.cnt[spin] / TK, Pb, Pe, sign,
                       beta, kpart + ((size_t)split * nspin + spin) * slot, rotation(kq));
 }
 
@@ -155,33 +155,37 @@ hipError_t khalf_go(hipStream_t st, const T* b, size_t ldb, size_t nbf, size_t P
     return hipGetLastError();
 }
 
+// 64-row tiles where nbf fits one, else 128-row ones
+template <typename T, int FN>
+hipError_t khalf_fm(hipStream_t st, const T* b, size_t ldb, size_t nbf, size_t P0, size_t Pc, const KPlan& kp,
+                    const T* cocc, T* m) {
+    if (nbf <= 64) return khalf_go<T, 1, FN>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+    return khalf_go<T, 2, FN>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+}
+
 template <typename T>
 hipError_t khalf_t(hipStream_t st, const T* b, size_t ldb, size_t nbf, size_t P0, size_t Pc, const KPlan& kp,
                    const T* cocc, T* m) {
-    if (kp.tile == 64) {
-        switch (kp.fn) {
-            case 1: return khalf_go<T, 1, 1>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
-            case 2: return khalf_go<T, 1, 2>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
-            case 3: return khalf_go<T, 1, 3>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
-            case 4: return khalf_go<T, 1, 4>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
-            case 5: return khalf_go<T, 1, 5>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
-            default: return khalf_go<T, 1, 6>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
-        }
-    }
     switch (kp.fn) {
-        case 1: return khalf_go<T, 2, 1>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
-        case 2: return khalf_go<T, 2, 2>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
-        case 3: return khalf_go<T, 2, 3>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
-        case 4: return khalf_go<T, 2, 4>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
-        case 5: return khalf_go<T, 2, 5>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
-        default: return khalf_go<T, 2, 6>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+        case 1: return khalf_fm<T, 1>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+        case 2: return khalf_fm<T, 2>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+        case 3: return khalf_fm<T, 3>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+        case 4: return khalf_fm<T, 4>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+        case 5: return khalf_fm<T, 5>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+        case 6:
+            if constexpr (sizeof(T) == 4) return khalf_fm<T, 6>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+            break;
+        case 8:
+            if constexpr (sizeof(T) == 4) return khalf_fm<T, 8>(st, b, ldb, nbf, P0, Pc, kp, cocc, m);
+            break;
     }
+    return hipErrorInvalidValue;
 }
 
-template <typename T, int FB>
+template <typename T, int F>
 hipError_t ksyrk_go(hipStream_t st, const T* m, size_t nbf, size_t Pc, const KPlan& kp, int nspin, const T* sign,
                     int beta, double* kpart) {
-    const size_t nt = kp.nbf_pad / (64 * FB), nt2 = nt * (nt + 1) / 2;
+    const size_t nt = kp.nbf_pad / (32 * F), nt2 = nt * (nt + 1) / 2;
     SyrkCols cols;
     cols.off[0] = (int)kp.col_off[0];
     cols.cnt[0] = (int)kp.col_cnt[0];
@@ -189,7 +193,7 @@ hipError_t ksyrk_go(hipStream_t st, const T* m, size_t nbf, size_t Pc, const KPl
     cols.cnt[1] = (int)kp.col_cnt[1];
     const int pps = (int)((Pc + kp.nsplit - 1) / kp.nsplit);
     const size_t nwg = round_up(kp.nslot, kXcd) * (size_t)nspin * nt2;
-    hipLaunchKernelGGL((k_ksyrk<T, FB>), dim3((unsigned)nwg), dim3(kBlock), 0, st, m, (int)kp.nbf_pad, (int)kp.nk,
+    hipLaunchKernelGGL((k_ksyrk<T, F>), dim3((unsigned)nwg), dim3(kBlock), 0, st, m, (int)kp.nbf_pad, (int)kp.nk,
                        (int)nbf, (int)Pc, (int)nt2, nspin, cols, sign, (int)kp.nslot, pps, beta, kpart,
                        kp.nbf_pad * kp.nbf_pad);
     return hipGetLastError();
@@ -198,7 +202,8 @@ hipError_t ksyrk_go(hipStream_t st, const T* m, size_t nbf, size_t Pc, const KPl
 template <typename T>
 hipError_t ksyrk_t(hipStream_t st, const T* m, size_t nbf, size_t Pc, const KPlan& kp, int nspin, const T* sign,
                    int beta, double* kpart) {
-    if (kp.tile == 64) return ksyrk_go<T, 1>(st, m, nbf, Pc, kp, nspin, sign, beta, kpart);
+    if constexpr (sizeof(T) == 8)
+        if (kp.tile == 128) return ksyrk_go<T, 4>(st, m, nbf, Pc, kp, nspin, sign, beta, kpart);
     return ksyrk_go<T, 2>(st, m, nbf, Pc, kp, nspin, sign, beta, kpart);
 }
 

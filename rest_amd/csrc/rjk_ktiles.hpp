@@ -17,11 +17,11 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int kBlock = 256;           // 4 waves
 constexpr int TK = kTileK;            // 16
-// LDS row padding (elements).  FP64: rows of 128 + 2 (or 64 + 2) doubles put the 16 rows that
-// one transposed stash instruction writes (one element each, 16 lanes at a time) on 16 distinct
-// 4-bank groups, and the 16 consecutive doubles of a fragment read on consecutive banks; a pad of
-// 4 leaves rows k and k + 8 on the same banks.  FP32 keeps 4.
-template <typename T> struct Pad { static constexpr int v = sizeof(T) == 8 ? 2 : 4; };
+// LDS row padding (elements).  A fragment read takes 16 consecutive elements of each of 4 rows.
+// FP64 serves one row a cycle whatever their distance; 2 elements keep the transposed stash of
+// blocks left of the diagonal off one bank.  FP32 serves two rows a cycle, free of conflicts when
+// the row length is an odd multiple of 16.
+template <typename T> constexpr int row_pad(int n) { return sizeof(T) == 8 ? 2 : ((n / 16) % 2 ? 0 : 16); }
 constexpr int kXcd = 8;               // MI355X: 8 XCDs, work-groups dealt round-robin by linear id
 
 __device__ inline size_t tri(size_t j) { return j * (j + 1) / 2; }
@@ -82,11 +82,17 @@ template <typename T, int N> struct VecOf {
 };
 template <typename T> __device__ __forceinline__ RJK_GLB const T* as_glb(const T* p) { return (RJK_GLB const T*)p; }
 template <typename T> __device__ __forceinline__ RJK_GLB const T* as_glb(RJK_GLB const T* p) { return p; }
-// N elements at base (uniform) + off bytes (per lane)
+// N elements at base (uniform) + off bytes (per lane).  The empty asm keeps the widening of `off` next
+// to the load, which is what lets it use the scalar-base form (a widening hoisted out of the loop
+// costs a 64-bit vector addition a load).
 template <typename T, int N>
-__device__ __forceinline__ typename VecOf<T, N>::raw ldv(RJK_GLB const T* base, unsigned off) {
+__device__ __forceinline__ typename VecOf<T, N>::raw ldv(RJK_GLB const T* base, unsigned& off) {
+    asm("" : "+v"(off));
     return *(RJK_GLB const typename VecOf<T, N>::type*)((RJK_GLB const char*)base + off);
 }
+
+// an LDS buffer as a compile-time number, so that it is part of an instruction's offset
+template <int N> struct Buf { static constexpr int n = N; };
 
 // ---------------------------------------------------------------------------
 // Stage 1: M'[P][c][μ] = Σ_ν Bsym_P[μ,ν] C'[ν][c], one (μ-tile, c-tile) of one
@@ -104,7 +110,8 @@ __device__ __forceinline__ typename VecOf<T, N>::raw ldv(RJK_GLB const T* base, 
 //       offsets fixed for the tile, the base moving by 16 elements a block;
 //     blocks beyond it (ν >= mu0 + 64 FM): row ν is contiguous in μ, one row per wave
 //       instruction at a scalar base;
-//     the diagonal blocks and a partial last block: element by element, mirrored and masked.
+//     the diagonal blocks: element by element, mirrored by one select on wave-uniform rows;
+//     a partial last block: element by element, mirrored and masked.
 // ---------------------------------------------------------------------------
 template <typename T, int FM, int FN, typename BP, typename CP, typename MP>
 __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol_, int nbf, int mu0, int c0, CP __restrict__ cocc_,
@@ -115,15 +122,15 @@ __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol_, int nbf, int m
     using VA = typename VecOf<T, FM>::raw;
     using V2 = typename VecOf<T, 2>::raw;
     using VBt = typename VecOf<T, VB>::raw;
-    __shared__ __align__(16) T As[2][TK][TM + Pad<T>::v];
-    __shared__ __align__(16) T Bs[2][TK][TN + Pad<T>::v];
+    __shared__ __align__(16) T As[2][TK][TM + row_pad<T>(TM)];
+    __shared__ __align__(16) T Bs[2][TK][TN + (sizeof(T) == 8 ? 0 : row_pad<T>(TN))];   // FP64: 3 work-groups a CU at FN = 5
     const auto bcol = as_glb(bcol_);
     const auto cocc = as_glb(cocc_);
     const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ws = (wave + rot) & 3;
     T ra[NA];
     VBt rb[NB];
-    unsigned live = 0;   // element-wise blocks: bit r set when element r lies inside nbf × nbf
+    unsigned live = 0;   // partial last block: bit r set when element r lies inside nbf × nbf
     if (mu0 >= nbf) return;   // a tile of padding rows only (nbf_pad beyond the tile grid); uniform
 
     // lane offsets (bytes), fixed for the tile
@@ -138,9 +145,13 @@ __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol_, int nbf, int m
         const int e = min(tid + r * kBlock, NPB - 1);
         offb[r] = (unsigned)(((e / PRB) * nk + (e % PRB) * VB) * sizeof(T));
     }
-    const unsigned offa = lane * FM * sizeof(T);
+    unsigned offa = lane * FM * sizeof(T);
+    // diagonal blocks: row h = max, column l = min of the two tile-relative indices lies h·mu0 + tri(h) + l
+    // beyond element (mu0, mu0); a thread keeps one μ, ν is wave-uniform
+    const int mt = min(tid % TM, nbf - 1 - mu0);
+    const unsigned offm = (unsigned)(mt * sizeof(T)), offr = (unsigned)((mt * mu0 + mt * (mt + 1) / 2) * sizeof(T));
 
-    enum { BELOW, ABOVE, MIXED };
+    enum { BELOW, DIAG, ABOVE, TAIL };
     auto fetch = [&](auto kind, int nu0) {
         if constexpr (kind() == BELOW) {
             const auto p = bcol + tri((size_t)mu0) + nu0;
@@ -157,6 +168,15 @@ __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol_, int nbf, int m
 #pragma unroll
                 for (int q = 0; q < FM; ++q) ra[r * FM + q] = v[q];
             }
+        } else if constexpr (kind() == DIAG) {
+            const auto p = bcol + tri((size_t)mu0) + mu0;
+#pragma unroll
+            for (int r = 0; r < NA; ++r) {
+                const int x = nu0 - mu0 + wave * 64 / TM + r * (kBlock / TM);   // tile-relative ν, uniform
+                unsigned o = x <= mt ? offr + (unsigned)(x * sizeof(T))
+                                     : offm + (unsigned)((x * mu0 + x * (x + 1) / 2) * sizeof(T));
+                ra[r] = ldv<T, 1>(p, o)[0];
+            }
         } else {
             live = 0;
 #pragma unroll
@@ -172,12 +192,15 @@ __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol_, int nbf, int m
 #pragma unroll
         for (int r = 0; r < NB; ++r) rb[r] = ldv<T, VB>(q, offb[r]);
     };
+    T* const sa_below = &As[0][(tid & 7) * 2][tid >> 3];
+    T* const sa_above = &As[0][wave][lane * FM];
+    constexpr int LA = TM + row_pad<T>(TM), LB = TN + (sizeof(T) == 8 ? 0 : row_pad<T>(TN));
     auto stash = [&](auto kind, int buf) {
         if constexpr (kind() == BELOW) {
 #pragma unroll
             for (int r = 0; r < 2 * FM; ++r) {
-                As[buf][(tid & 7) * 2][(tid >> 3) + 32 * r] = ra[2 * r];
-                As[buf][(tid & 7) * 2 + 1][(tid >> 3) + 32 * r] = ra[2 * r + 1];
+                sa_below[buf * TK * LA + 32 * r] = ra[2 * r];
+                sa_below[buf * TK * LA + LA + 32 * r] = ra[2 * r + 1];
             }
         } else if constexpr (kind() == ABOVE) {
 #pragma unroll
@@ -185,19 +208,19 @@ __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol_, int nbf, int m
                 VA v;
 #pragma unroll
                 for (int q = 0; q < FM; ++q) v[q] = ra[r * FM + q];
-                *(VA*)&As[buf][wave + 4 * r][lane * FM] = v;
+                *(VA*)(sa_above + (buf * TK + 4 * r) * LA) = v;
             }
         } else {
 #pragma unroll
             for (int r = 0; r < NA; ++r) {
                 const int e = tid + r * kBlock;
-                As[buf][e / TM][e % TM] = ((live >> r) & 1u) ? ra[r] : T(0);
+                As[buf][e / TM][e % TM] = (kind() == DIAG || ((live >> r) & 1u)) ? ra[r] : T(0);
             }
         }
 #pragma unroll
         for (int r = 0; r < NB; ++r) {
             const int e = tid + r * kBlock;
-            if ((r + 1) * kBlock <= NPB || e < NPB) *(VBt*)&Bs[buf][e / PRB][(e % PRB) * VB] = rb[r];
+            if ((r + 1) * kBlock <= NPB || e < NPB) *(VBt*)(&Bs[0][e / PRB][(e % PRB) * VB] + buf * TK * LB) = rb[r];
         }
     };
 
@@ -208,15 +231,17 @@ __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol_, int nbf, int m
         for (int j = 0; j < FN; ++j) acc[i][j] = MM::zero();
     const int mrow = ws * 16 * FM;
     const bool act = mu0 + mrow < nbf;   // wave-uniform
+    const T* const fa = &As[0][g][mrow + l16];
+    const T* const fb = &Bs[0][g][l16];
     auto compute = [&](int cur) {
         if (!act) return;
 #pragma unroll
         for (int kk = 0; kk < TK; kk += 4) {
             T bmu[FM], ac[FN];
 #pragma unroll
-            for (int i = 0; i < FM; ++i) bmu[i] = As[cur][kk + g][mrow + i * 16 + l16];
+            for (int i = 0; i < FM; ++i) bmu[i] = fa[(cur * TK + kk) * LA + i * 16];
 #pragma unroll
-            for (int j = 0; j < FN; ++j) ac[j] = Bs[cur][kk + g][j * 16 + l16];
+            for (int j = 0; j < FN; ++j) ac[j] = fb[(cur * TK + kk) * LB + j * 16];
             // D[c][μ] = Σ_ν C'[ν][c] Bsym[ν][μ]
 #pragma unroll
             for (int i = 0; i < FM; ++i)
@@ -226,11 +251,12 @@ __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol_, int nbf, int m
     };
 
     // k-blocks [0, e0) below the diagonal range, [e0, e1) across it, [e1, e2) above, [e2, nkb) the partial last
-    const int nkb = (nbf + TK - 1) / TK;
-    const int e0 = mu0 / TK, e1 = min(nkb, (mu0 + TM) / TK), e2 = max(e1, nbf / TK);
+    const int nkb = (nbf + TK - 1) / TK, e2 = nbf / TK;
+    const int e0 = mu0 / TK, e1 = min(e2, (mu0 + TM) / TK);
     struct KB { __device__ constexpr int operator()() const { return BELOW; } };
+    struct KD { __device__ constexpr int operator()() const { return DIAG; } };
     struct KA { __device__ constexpr int operator()() const { return ABOVE; } };
-    struct KX { __device__ constexpr int operator()() const { return MIXED; } };
+    struct KT { __device__ constexpr int operator()() const { return TAIL; } };
     int kb = 0;
     auto run = [&](auto kind, int end) {   // blocks up to `end` are of this kind; block kb is in LDS
         for (; kb + 1 < end; ++kb) {
@@ -243,15 +269,18 @@ __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol_, int nbf, int m
     if (e0 > 0) {
         fetch(KB(), 0);
         stash(KB(), 0);
+    } else if (e1 > 0) {
+        fetch(KD(), 0);
+        stash(KD(), 0);
     } else {
-        fetch(KX(), 0);
-        stash(KX(), 0);
+        fetch(KT(), 0);
+        stash(KT(), 0);
     }
     __syncthreads();
     run(KB(), e0);
-    run(KX(), e1);
+    run(KD(), e1);
     run(KA(), e2);
-    run(KX(), nkb);
+    run(KT(), nkb);
     compute(kb & 1);
     __syncthreads();   // the persistent callers start their next tile in the same LDS
 
@@ -268,127 +297,126 @@ __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol_, int nbf, int m
 
 // ---------------------------------------------------------------------------
 // Stage 2: Kpart (+)= Σ_{P,c} M'[P][c][μ] sign_c M'[P][c][ν] over the upper tiles
-//   (mu0 <= nu0) of 64·FB × 64·FB, split-K over P.  Wave w owns 16·FB columns ν and
-//   every row μ of the tile; in a diagonal tile it computes only the μ groups up to its
-//   own (10 of 16 groups), and a wave whose columns all lie beyond nbf computes nothing
-//   (`rot` as in stage 1).  Same pipeline as stage 1 over the flattened (P, 16-column block) index;
-//   the rows of M' are wave-uniform, so every load is one row at a scalar base.  Signs
-//   are looked at once per tile and applied while staging only where one is negative.
-//   Accumulation in the MFMA type, partial tiles kept in FP64.
+//   (mu0 <= nu0) of 32·F × 32·F, split-K over P, 2 × 2 waves of F × F fragments.  In a
+//   diagonal tile the wave below the diagonal computes nothing and the two on it only
+//   their fragments i <= j; waves beyond nbf compute nothing (`rot` as in stage 1).
+//   Same pipeline as stage 1 over the flattened (P, 16-column block) index: lane offsets
+//   within a k-block's 16 rows are fixed, the base moves by scalar arithmetic.  A diagonal
+//   tile stages its rows once for both operands.  Signs are looked at once per tile and
+//   applied while staging only where one is negative.  Accumulation in the MFMA type,
+//   partial tiles kept in FP64.
+//   Loads run two k-blocks ahead in two register sets, so that a miss to HBM is covered also with
+//   two waves a SIMD; with the LDS buffers as compile-time offsets a k-block costs no vector
+//   instruction beside its MFMAs.  FP64 inner rate (k-blocks from L2, 2 work-groups a CU): F = 4
+//   71 TFLOP/s, F = 2 66 (F = 3 on three work-groups 65; one block ahead and dynamic buffers 67, 62, 65).
 // ---------------------------------------------------------------------------
 struct SyrkCols {
     int off[2], cnt[2];
 };
 
-template <typename T, int FB, bool DIAG, typename MP, typename SP, typename KP>
+template <typename T, int F, bool DIAG, typename MP, typename SP, typename KP>
 __device__ __forceinline__ void ksyrk_body(MP m, int ldm, int nk, int nbf, int mu0, int nu0, int cb, int ncb, int Pb,
                                            int Pe, SP sign, int beta, KP kp, int ws, bool neg, T* __restrict__ lds) {
     using MM = Mma<T>;
-    constexpr int FA = 4 * FB, Tt = 64 * FB, LD = Tt + Pad<T>::v;
-    using VL = typename VecOf<T, FB>::raw;
+    constexpr int Tt = 32 * F, LD = Tt + row_pad<T>(Tt);
+    constexpr int VB = 16 / (int)sizeof(T) < F * 32 * TK / kBlock ? 16 / (int)sizeof(T) : F * 32 * TK / kBlock;
+    constexpr int PR = Tt / VB, NL = TK * PR / kBlock;   // pieces a row, pieces a thread
+    static_assert(NL * kBlock == TK * PR, "load shape");
+    using VL = typename VecOf<T, VB>::raw;
     const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    auto As = [&](int buf, int k) { return lds + (buf * TK + k) * LD; };
-    auto Bs = [&](int buf, int k) { return lds + ((2 + buf) * TK + k) * LD; };
+    // LDS: μ operand of buffers 0 and 1, then the ν operand of both
+    constexpr int kB = 2 * TK * LD;
     const int nq = (Pe > Pb ? Pe - Pb : 0) * ncb;
-    const unsigned off = lane * FB * sizeof(T);
-    VL ra[4], rb[4];
-    T rs[4];
-    int fP = Pb, fc = 0;   // (P, block) of the next fetch
-    auto fetch = [&]() {
-        const auto base = m + ((size_t)fP * nk + cb + fc * TK + wave) * ldm;
+    unsigned off[NL];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if constexpr (!DIAG) ra[r] = ldv<T, FB>(base + (size_t)(4 * r) * ldm + mu0, off);
-            rb[r] = ldv<T, FB>(base + (size_t)(4 * r) * ldm + nu0, off);
-        }
-        if (neg) {
+    for (int r = 0; r < NL; ++r) {
+        const int e = tid + r * kBlock;
+        off[r] = (unsigned)(((e / PR) * ldm + (e % PR) * VB) * sizeof(T));
+    }
+    // two register sets: block q + 2 is under way while block q + 1 waits to be staged
+    VL ra0[NL], rb0[NL], ra1[NL], rb1[NL];
+    int fP = Pb, fc = 0, fq = 0;   // (P, block) of the next fetch; past the last block it repeats that one
+    auto fetch = [&](VL (&ra)[NL], VL (&rb)[NL]) {
+        const auto base = m + ((size_t)fP * nk + cb + fc * TK) * ldm;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) rs[r] = sign[cb + fc * TK + wave + 4 * r];
+        for (int r = 0; r < NL; ++r) {
+            if constexpr (!DIAG) ra[r] = ldv<T, VB>(base + mu0, off[r]);
+            rb[r] = ldv<T, VB>(base + nu0, off[r]);
         }
-        if (++fc == ncb) {
+        if (++fq < nq && ++fc == ncb) {
             fc = 0;
             ++fP;
         }
     };
-    // a diagonal tile stages its rows once, and a second time with the signs where one is negative
-    auto stash = [&](int buf) {
+    T* sw[NL];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if constexpr (DIAG) *(VL*)(As(buf, wave + 4 * r) + lane * FB) = rb[r];
-            else *(VL*)(As(buf, wave + 4 * r) + lane * FB) = ra[r];
-            if (!DIAG || neg) *(VL*)(Bs(buf, wave + 4 * r) + lane * FB) = neg ? rb[r] * rs[r] : rb[r];
+    for (int r = 0; r < NL; ++r) sw[r] = lds + ((tid + r * kBlock) / PR) * LD + ((tid + r * kBlock) % PR) * VB;
+    int sc = 0;   // column block of the next stash
+    auto stash = [&](auto buf, VL (&ra)[NL], VL (&rb)[NL]) {
+        constexpr int o = decltype(buf)::n * TK * LD;
+#pragma unroll
+        for (int r = 0; r < NL; ++r) {
+            if constexpr (DIAG) *(VL*)(sw[r] + o) = rb[r];
+            else *(VL*)(sw[r] + o) = ra[r];
+            if (!DIAG && !neg) *(VL*)(sw[r] + kB + o) = rb[r];
+        }
+        if (neg) {   // signed columns (rare): the signs are read here
+#pragma unroll
+            for (int r = 0; r < NL; ++r)
+                *(VL*)(sw[r] + kB + o) = rb[r] * (T)sign[cb + sc * TK + (tid + r * kBlock) / PR];
+            if (++sc == ncb) sc = 0;
         }
     };
-    typename MM::acc_t acc[FA][FB];
+    typename MM::acc_t acc[F][F];
 #pragma unroll
-    for (int i = 0; i < FA; ++i)
+    for (int i = 0; i < F; ++i)
 #pragma unroll
-        for (int j = 0; j < FB; ++j) acc[i][j] = MM::zero();
-    const int ncol = ws * 16 * FB;
-    const bool act = nu0 + ncol < nbf;
-    const int bsel = (!DIAG || neg) ? 2 * TK * LD : 0;   // where the ν operand lies
-    auto compute = [&](int cur) {
+        for (int j = 0; j < F; ++j) acc[i][j] = MM::zero();
+    const int mrow = (ws & 1) * 16 * F, ncol = (ws >> 1) * 16 * F;
+    const bool act = nu0 + ncol < nbf && mu0 + mrow < nbf && !(DIAG && mrow > ncol);
+    const T* const fa = lds + g * LD + mrow + l16;
+    const T* const fb = lds + g * LD + ncol + l16 + ((!DIAG || neg) ? kB : 0);
+    auto compute = [&](auto cur_) {
+        constexpr int cur = decltype(cur_)::n;
         if (!act) return;
-        const T* __restrict__ a0 = As(cur, g) + l16;
-        const T* __restrict__ b0 = As(cur, g) + bsel + ncol + l16;
         // D[ν][μ] = Σ_k sign_k M'[k][ν] M'[k][μ]
-        if constexpr (DIAG) {
-            T anu[TK / 4][FB];
 #pragma unroll
-            for (int kk = 0; kk < TK; kk += 4)
+        for (int kk = 0; kk < TK; kk += 4) {
+            T bmu[F], anu[F];
 #pragma unroll
-                for (int j = 0; j < FB; ++j) anu[kk / 4][j] = b0[kk * LD + j * 16];
+            for (int j = 0; j < F; ++j) anu[j] = fb[(cur * TK + kk) * LD + j * 16];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if (q > ws) break;   // groups of FB fragments; those right of the wave's own are below the diagonal
+            for (int i = 0; i < F; ++i) bmu[i] = fa[(cur * TK + kk) * LD + i * 16];
 #pragma unroll
-                for (int kk = 0; kk < TK; kk += 4) {
-                    T bmu[FB];
+            for (int i = 0; i < F; ++i)
 #pragma unroll
-                    for (int i = 0; i < FB; ++i) bmu[i] = a0[kk * LD + (q * FB + i) * 16];
-#pragma unroll
-                    for (int i = 0; i < FB; ++i)
-#pragma unroll
-                        for (int j = 0; j < FB; ++j)
-                            acc[q * FB + i][j] = MM::op(anu[kk / 4][j], bmu[i], acc[q * FB + i][j]);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int kk = 0; kk < TK; kk += 4) {
-                T bmu[FA], anu[FB];
-#pragma unroll
-                for (int j = 0; j < FB; ++j) anu[j] = b0[kk * LD + j * 16];
-#pragma unroll
-                for (int i = 0; i < FA; ++i) bmu[i] = a0[kk * LD + i * 16];
-#pragma unroll
-                for (int i = 0; i < FA; ++i)
-#pragma unroll
-                    for (int j = 0; j < FB; ++j) acc[i][j] = MM::op(anu[j], bmu[i], acc[i][j]);
-            }
+                for (int j = 0; j < F; ++j) acc[i][j] = MM::op(anu[j], bmu[i], acc[i][j]);
         }
     };
     if (nq > 0) {
-        fetch();
-        stash(0);
+        fetch(ra0, rb0);
+        fetch(ra1, rb1);
+        stash(Buf<0>(), ra0, rb0);
+        fetch(ra0, rb0);
     }
     __syncthreads();
-    for (int q = 0; q + 1 < nq; ++q) {
-        fetch();
-        compute(q & 1);
-        stash((q + 1) & 1);
+    for (int q = 0; q < nq; q += 2) {   // an odd last block leaves buffer 1 unused
+        compute(Buf<0>());
+        stash(Buf<1>(), ra1, rb1);
+        fetch(ra1, rb1);
+        __syncthreads();
+        if (q + 1 < nq) compute(Buf<1>());
+        stash(Buf<0>(), ra0, rb0);
+        fetch(ra0, rb0);
         __syncthreads();
     }
-    if (nq > 0) compute((nq - 1) & 1);
     __syncthreads();   // the persistent callers start their next tile in the same LDS
     if (!act) return;
 #pragma unroll
-    for (int i = 0; i < FA; ++i) {
-        if (DIAG && i / FB > ws) break;
+    for (int i = 0; i < F; ++i)
 #pragma unroll
-        for (int j = 0; j < FB; ++j) {
-            const int mu = mu0 + i * 16 + l16, nb = nu0 + ncol + j * 16;
+        for (int j = 0; j < F; ++j) {
+            const int mu = mu0 + mrow + i * 16 + l16, nb = nu0 + ncol + j * 16;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const auto dst = kp + (size_t)(nb + MM::row(lane, r)) * ldm + mu;
@@ -397,14 +425,13 @@ __device__ __forceinline__ void ksyrk_body(MP m, int ldm, int nk, int nbf, int m
                 *dst = v;
             }
         }
-    }
 }
 
-template <typename T, int FB, typename MP, typename SP, typename KP>
+template <typename T, int F, typename MP, typename SP, typename KP>
 __device__ __forceinline__ void ksyrk_tile(MP __restrict__ m, int ldm, int nk, int nbf, int mu0, int nu0, int cb,
                                            int ncb, int Pb, int Pe, SP __restrict__ sign, int beta,
                                            KP __restrict__ kp, int rot) {
-    constexpr int LD = 64 * FB + Pad<T>::v;
+    constexpr int LD = 32 * F + row_pad<T>(32 * F);
     __shared__ __align__(16) T lds[4 * TK * LD];
     const int ws = (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) + rot) & 3;
     if (nu0 >= nbf) return;   // padding columns only (uniform)
@@ -413,9 +440,9 @@ __device__ __forceinline__ void ksyrk_tile(MP __restrict__ m, int ldm, int nk, i
     const bool neg = __syncthreads_or(any) != 0;
     const auto mg = as_glb(m);
     if (mu0 == nu0)
-        ksyrk_body<T, FB, true>(mg, ldm, nk, nbf, mu0, nu0, cb, ncb, Pb, Pe, sign, beta, kp, ws, neg, lds);
+        ksyrk_body<T, F, true>(mg, ldm, nk, nbf, mu0, nu0, cb, ncb, Pb, Pe, sign, beta, kp, ws, neg, lds);
     else
-        ksyrk_body<T, FB, false>(mg, ldm, nk, nbf, mu0, nu0, cb, ncb, Pb, Pe, sign, beta, kp, ws, neg, lds);
+        ksyrk_body<T, F, false>(mg, ldm, nk, nbf, mu0, nu0, cb, ncb, Pb, Pe, sign, beta, kp, ws, neg, lds);
 }
 
 
