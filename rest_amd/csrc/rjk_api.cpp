@@ -15,6 +15,8 @@ thread_local std::string g_create_error;
 
 constexpr double kEigRelCut = 1e-13;     // density-only route: |λ| <= cut·max|λ| is dropped
 constexpr double kAsymTol = 1e-10;       // density-only route: D symmetry tolerance
+constexpr double kCholCut = 1e-14;       // its Cholesky factor: remaining diagonal that ends it, of the largest
+constexpr double kCholTol = 1e-13;       // and the largest element it may leave out, of max|D|
 
 struct Carve {
     std::vector<size_t> off;
@@ -750,9 +752,14 @@ int vk_dm_general(rjk_ctx* ctx, const double* dm_dev, int ns, double scale, doub
 
 // Density-only K on device memory, K_s = scaling_factor · upper(Σ_P B_P D_s B_P) into vk_dev
 // (spin_channel × npair).  A device reduction measures max|D − Dᵀ| against max|D| per spin.
-// When every D is symmetric to kAsymTol, (D + Dᵀ)/2 is eigen-decomposed (rocSOLVER dsyevd) and
-// the eigenpairs with |λ| > kEigRelCut·max|λ| go through the occupied route with signed
-// weights λ; otherwise the general route above reads every D in full.
+// When every D is symmetric to kAsymTol, it goes through the occupied route over columns whose signed
+// squares add up to (D + Dᵀ)/2; otherwise the general route above reads every D in full.  The
+// columns, per call:
+//   FP64, nbf <= 4096, D positive semidefinite of low rank (an SCF density has rank nocc):
+//     the pivoted Cholesky factor, unless it leaves out more than kCholTol·max|D| (nbf 192, rank
+//     40: 0.08 ms against 3 ms for the eigenpairs; nbf 1536, rank 320: 3 against 38);
+//   else the eigenpairs with |λ| > kEigRelCut·max|λ| (rocSOLVER dsyevd), weights λ.
+// The lower precisions keep the eigenpairs: their K depends on the columns at its own rounding.
 int vk_dm_device(rjk_ctx* ctx, const void* b, const double* dm_dev, size_t spin_channel, double scaling_factor,
                  int prec, double* vk_dev) {
     const size_t nbf = ctx->nbf, n2 = nbf * nbf;
@@ -762,14 +769,23 @@ int vk_dm_device(rjk_ctx* ctx, const void* b, const double* dm_dev, size_t spin_
     int rc = solver_handle(ctx, &h);
     if (rc) return rc;
     hipStream_t st = ctx->stream;
+    const bool chol = prec == RJK_PREC_FP64 && nbf <= 4096;
+    // columns worth finding: beyond 256 functions a step is one launch (5 us), and a quarter of the
+    // functions bounds what a D of higher rank costs in vain to a few percent of its eigenproblem
+    const size_t kmax = std::min(nbf <= 256 ? std::max<size_t>(1, nbf / 2) : nbf / 4 + 64, kCholMaxRank);
+    const size_t nb32 = (nbf + 31) / 32;
+    const unsigned nblk = asym_stats_blocks(nbf);
+    // per spin: [asymmetry statistics | residual | rank], read back in one copy
+    const size_t nstat = 2 * (size_t)nblk + 2;
     Carve cv;
-    const size_t i_st = cv.add(2 * kAsymBlocks * spin_channel * sizeof(double));
+    const size_t i_st = cv.add(nstat * spin_channel * sizeof(double));
     const size_t i_vec = cv.add(spin_channel * n2 * sizeof(double));
-    const size_t i_lam = cv.add(spin_channel * nbf * sizeof(double));
+    const size_t i_lam = cv.add(2 * spin_channel * nbf * sizeof(double));   // eigenvalues, or diagonals of the factor
     const size_t i_E = cv.add(nbf * sizeof(double));
     const size_t i_sel = cv.add(spin_channel * nbf * sizeof(double));
     const size_t i_idx = cv.add(spin_channel * nbf * sizeof(int));
     const size_t i_info = cv.add(sizeof(int));
+    const size_t i_blk = cv.add((nb32 * nb32 + 2) * sizeof(double));
     void* aux = nullptr;
     rc = buf_get(ctx, &ctx->aux, &ctx->aux_size, cv.total, &aux);
     if (rc) return rc;
@@ -781,30 +797,52 @@ int vk_dm_device(rjk_ctx* ctx, const void* b, const double* dm_dev, size_t spin_
     double* d_sel = (double*)(base + cv.off[i_sel]);
     int* d_idx = (int*)(base + cv.off[i_idx]);
     int* d_info = (int*)(base + cv.off[i_info]);
-    // symmetry of every D
-    const unsigned nblk = asym_stats_blocks(nbf);
-    std::vector<double> stats(2 * nblk * spin_channel);
+    double* d_blk = (double*)(base + cv.off[i_blk]);
+    // symmetry of every D, and its Cholesky factor (kmax columns at most) where it may serve
+    std::vector<double> stats(nstat * spin_channel);
     for (int s = 0; s < ns; ++s) {
-        RJK_HIP(ctx, launch_asym_stats(st, dm_dev + s * n2, nbf, d_stats + 2 * kAsymBlocks * s));
-        RJK_HIP(ctx, hipMemcpyAsync(stats.data() + 2 * nblk * s, d_stats + 2 * kAsymBlocks * s,
-                                    2 * nblk * sizeof(double), hipMemcpyDeviceToHost, st));
+        double* ds = d_stats + nstat * s;
+        RJK_HIP(ctx, launch_asym_stats(st, dm_dev + s * n2, nbf, ds));
+        if (chol)
+            RJK_HIP(ctx, launch_pivot_chol(st, dm_dev + s * n2, nbf, kmax, kCholCut, d_lam + 2 * s * nbf, d_vec + s * n2,
+                                           (int*)(ds + 2 * nblk + 1), d_blk, ds + 2 * nblk));
     }
+    RJK_HIP(ctx, hipMemcpyAsync(stats.data(), d_stats, stats.size() * sizeof(double), hipMemcpyDeviceToHost, st));
     RJK_HIP(ctx, hipStreamSynchronize(st));
-    bool general = false;
+    bool general = false, low_rank = chol;
+    size_t ncol[2] = {0, 0};
     for (int s = 0; s < ns; ++s) {
+        const double* h_st = stats.data() + nstat * s;
         double asym = 0, amax = 0;
         for (unsigned q = 0; q < nblk; ++q) {
-            asym = std::max(asym, stats[2 * nblk * s + 2 * q]);
-            amax = std::max(amax, stats[2 * nblk * s + 2 * q + 1]);
+            asym = std::max(asym, h_st[2 * q]);
+            amax = std::max(amax, h_st[2 * q + 1]);
         }
         if (!std::isfinite(amax)) return fail(ctx, RJK_ERR_NONFINITE, "dm holds NaN/Inf");
         if (asym > kAsymTol * std::max(amax, 1e-300)) general = true;
+        if (chol) {
+            int rank = -1;
+            std::memcpy(&rank, h_st + 2 * nblk + 1, sizeof(int));
+            if (rank < 0 || !(h_st[2 * nblk] <= kCholTol * amax)) low_rank = false;
+            else ncol[s] = (size_t)rank;
+        }
     }
     if (general) return vk_dm_general(ctx, dm_dev, ns, scaling_factor, vk_dev);
+    if (low_rank) {
+        KPlan kp;
+        k_plan_cols(kp, nbf, ncol, ns, prec);
+        void *cocc, *sign, *m;
+        double* kpart;
+        rc = k_plan_ws(ctx, kp, ns, prec, &cocc, &sign, &kpart, &m);
+        if (rc) return rc;
+        if (kp.nk > 0)
+            RJK_HIP(ctx, launch_prep_factor(st, d_vec, nbf, n2, ncol, ns, kp, (double*)cocc, (double*)sign));
+        return k_run(ctx, kp, ns, prec, b, cocc, sign, kpart, m, scaling_factor, vk_dev);
+    }
+    ncol[0] = ncol[1] = 0;
     std::vector<double> lam(nbf);
     std::vector<int> sel_idx[2];
     std::vector<double> sel_lam[2];
-    size_t ncol[2] = {0, 0};
     for (int s = 0; s < ns; ++s) {
         RJK_HIP(ctx, launch_symmetrize(st, dm_dev + s * n2, nbf, d_vec + s * n2));
         rocblas_status rs = rocsolver_dsyevd(h, rocblas_evect_original, rocblas_fill_upper, (rocblas_int)nbf,

@@ -144,6 +144,8 @@ hipError_t launch_prep_cocc(hipStream_t st, int prec, const double* eigv, size_t
 hipError_t launch_prep_cocc_idx(hipStream_t st, int prec, const double* vecs, size_t nbf, const int* idx,
                                 const double* lam, size_t ncol, size_t col_off, const KPlan& kp, void* cocc,
                                 void* sign);
+hipError_t launch_prep_factor(hipStream_t st, const double* f, size_t nbf, size_t fs, const size_t* ncol, int nspin,
+                              const KPlan& kp, double* cocc, double* sign);
 hipError_t launch_khalf(hipStream_t st, int prec, const void* b, size_t ldb, size_t nbf, size_t P0, size_t Pc,
                         const KPlan& kp, const void* cocc, void* m);
 hipError_t launch_ksyrk(hipStream_t st, int prec, const void* m, size_t nbf, size_t Pc, const KPlan& kp, int nspin,
@@ -179,6 +181,12 @@ hipError_t launch_check_finite(hipStream_t st, const double* x, size_t n, int* f
 constexpr size_t kAsymBlocks = 256;
 unsigned asym_stats_blocks(size_t nbf);
 hipError_t launch_asym_stats(hipStream_t st, const double* dm, size_t nbf, double* out);
+// pivoted Cholesky factor of a symmetric positive semidefinite D, at most kmax columns L[k][nbf]; rank
+// (−1: not such a D, or more columns) and the largest element D leaves out, on the device.  diag: 2·nbf
+// doubles, blockmax: ceil(nbf / 32)² + 2
+constexpr size_t kCholMaxRank = 1024;
+hipError_t launch_pivot_chol(hipStream_t st, const double* dm, size_t nbf, size_t kmax, double cut, double* diag, double* L,
+                             int* rank, double* blockmax, double* residual);
 hipError_t launch_prep_general(hipStream_t st, const double* dm, size_t nbf, size_t nk, size_t nrow, double* cx,
                                double* cy);
 hipError_t launch_pack_upper(hipStream_t st, const double* g, size_t nbf, size_t ldg, double scale, double* vk);

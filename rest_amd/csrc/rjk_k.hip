@@ -144,6 +144,19 @@ __global__ void k_prep_cocc_idx(const double* __restrict__ vecs, int nbf, const 
     if (nu == 0) sign[col_off + q] = (T)((w > 0) ? 1.0 : ((w < 0) ? -1.0 : 0.0));
 }
 
+// C'[ν][c] from columns that are weights already (rows of f, spin s at f + s·fs): the Cholesky factor
+// of a density; padding columns and rows are zero
+__global__ void k_prep_factor(const double* __restrict__ f, int nbf, size_t fs, int n0, int n1, int off1, int nk,
+                              int nrow, double* __restrict__ cocc, double* __restrict__ sign) {
+    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (size_t)nrow * nk) return;
+    const int c = (int)(t % nk), nu = (int)(t / nk);
+    const bool in0 = c < n0, in1 = c >= off1 && c < off1 + n1;
+    const double* src = in0 ? f + (size_t)c * nbf : f + fs + (size_t)(c - off1) * nbf;
+    cocc[t] = (in0 || in1) && nu < nbf ? src[nu] : 0.0;
+    if (nu == 0) sign[c] = in0 || in1 ? 1.0 : 0.0;
+}
+
 template <typename T, int FM, int FN>
 hipError_t khalf_go(hipStream_t st, const T* b, size_t ldb, size_t nbf, size_t P0, size_t Pc, const KPlan& kp,
                     const T* cocc, T* m) {
@@ -242,6 +255,14 @@ hipError_t launch_prep_cocc_idx(hipStream_t st, int prec, const double* vecs, si
     else
         hipLaunchKernelGGL(k_prep_cocc_idx<float>, g, dim3(256), 0, st, vecs, (int)nbf, idx, lam, (int)ncol,
                            (int)col_off, (int)kp.nk, (int)kp.nbf_pad, (float*)cocc, (float*)sign);
+    return hipGetLastError();
+}
+
+hipError_t launch_prep_factor(hipStream_t st, const double* f, size_t nbf, size_t fs, const size_t* ncol, int nspin,
+                              const KPlan& kp, double* cocc, double* sign) {
+    const size_t n = kp.nbf_pad * kp.nk;
+    hipLaunchKernelGGL(k_prep_factor, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, f, (int)nbf, fs, (int)ncol[0],
+                       nspin == 2 ? (int)ncol[1] : 0, (int)kp.col_off[1], (int)kp.nk, (int)kp.nbf_pad, cocc, sign);
     return hipGetLastError();
 }
 

@@ -2,7 +2,7 @@
 // of full B columns (REST ri3fn) into the packed pair layout, padding of
 // compact packed columns to the device leading dimension, FP32 copies,
 // symmetrisation of D, a plain copy (counter calibration), a finite check and
-// the helpers of the density-only K on a general D.
+// the helpers of the density-only K (pivoted Cholesky factor; general D).
 #include <algorithm>
 
 #include "rjk_internal.hpp"
@@ -153,6 +153,266 @@ __global__ void k_pack_upper(const double* __restrict__ g, size_t nbf, size_t ld
     vk[p] = scale * g[i + j * ldg];
 }
 
+// Pivoted Cholesky factor of the symmetric part of a column-major nbf × nbf D: L[k][i], D ≈ Σ_k L_k L_kᵀ,
+// for the density-only K (an SCF density has rank nocc, and this finds it in nocc steps where an
+// eigensolver needs n).  One work-group: a step is a pivot search, one column of D and k products per
+// row, too little to spread over CUs; what bounds it is the chain of barriers and L2 latencies, about 2 us a
+// step (nbf 192, rank 40: 80 us against 3 ms for the eigenpairs).  The first columns of L stay in
+// LDS as well, the products of a row are split over 1024 / nbf threads.
+// Stops when the largest remaining diagonal is at most cut·max diag(D); rank -> out[0], or -1 if a
+// diagonal falls below −cut·max (D is not positive semidefinite) or kmax columns do not suffice.
+constexpr int kCholThreads = 1024;
+constexpr size_t kCholSmall = 256;   // largest nbf of the one-work-group kernel
+constexpr int kCholLds = 16384;   // doubles of L kept in LDS
+__global__ __launch_bounds__(kCholThreads) void k_pivot_chol(const double* __restrict__ dm, int n, int kmax, double cut,
+                                                             double* __restrict__ diag, double* __restrict__ L,
+                                                             int* __restrict__ out) {
+    extern __shared__ double sm[];
+    double* ls = sm;                        // [kCholLds]
+    double* part = sm + kCholLds;           // [kCholThreads]
+    double* lp = part + kCholThreads;       // [kmax] row p of L
+    __shared__ double wmax[16], wmin[16];
+    __shared__ int widx[16];
+    __shared__ double sh_max, sh_min;
+    __shared__ int sh_p;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int klds = kCholLds / n;          // columns of L kept in LDS
+    int G = 1;                              // threads that share a row's products
+    while (2 * G * n <= kCholThreads) G *= 2;
+    for (int i = tid; i < n; i += kCholThreads) diag[i] = dm[(size_t)i * n + i];
+    __syncthreads();
+    double d0 = 0.0;
+    int rank = -1;
+    for (int k = 0;; ++k) {
+        double mx = -INFINITY, mn = INFINITY;
+        int at = 0;
+        for (int i = tid; i < n; i += kCholThreads) {
+            const double d = diag[i];
+            if (d > mx) {
+                mx = d;
+                at = i;
+            }
+            mn = fmin(mn, d);
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const double m2 = __shfl_xor(mx, o, 64);
+            const int a2 = __shfl_xor(at, o, 64);
+            if (m2 > mx || (m2 == mx && a2 < at)) {
+                mx = m2;
+                at = a2;
+            }
+            mn = fmin(mn, __shfl_xor(mn, o, 64));
+        }
+        if (lane == 0) {
+            wmax[wave] = mx;
+            wmin[wave] = mn;
+            widx[wave] = at;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            for (int w = 1; w < 16; ++w) {
+                if (wmax[w] > wmax[0]) {
+                    wmax[0] = wmax[w];
+                    widx[0] = widx[w];
+                }
+                wmin[0] = fmin(wmin[0], wmin[w]);
+            }
+            sh_max = wmax[0];
+            sh_min = wmin[0];
+            sh_p = widx[0];
+        }
+        __syncthreads();
+        const double top = sh_max, low = sh_min;
+        const int p = sh_p;
+        if (k == 0) d0 = top;
+        if (low < -cut * d0 || !(top >= 0.0)) break;      // not positive semidefinite (or NaN)
+        if (top <= cut * d0) {
+            rank = k;
+            break;
+        }
+        if (k == kmax) break;
+        for (int j = tid; j < k; j += kCholThreads) lp[j] = j < klds ? ls[j * n + p] : L[(size_t)j * n + p];
+        __syncthreads();
+        const double inv = 1.0 / sqrt(top);
+        for (int i0 = 0; i0 < n; i0 += kCholThreads / G) {   // G > 1 only when one pass covers all rows
+            const int i = i0 + tid / G, q = tid % G;
+            double v = 0.0;
+            if (i < n) {
+                const int kl = min(k, klds);
+                int j = q;
+                for (; j < kl; j += G) v += ls[j * n + i] * lp[j];
+                for (; j + 7 * G < k; j += 8 * G) {   // eight loads in flight
+                    double x[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) x[u] = L[(size_t)(j + u * G) * n + i];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v += x[u] * lp[j + u * G];
+                }
+                for (; j < k; j += G) v += L[(size_t)j * n + i] * lp[j];
+                if (G == 1) v = (0.5 * (dm[(size_t)p * n + i] + dm[(size_t)i * n + p]) - v) * inv;
+            }
+            if (G > 1) {
+                part[tid] = v;
+                __syncthreads();
+                if (q == 0 && i < n) {
+                    for (int u = 1; u < G; ++u) v += part[tid + u];
+                    v = (0.5 * (dm[(size_t)p * n + i] + dm[(size_t)i * n + p]) - v) * inv;
+                }
+            }
+            if (q == 0 && i < n) {
+                const double l = i == p ? top * inv : v;
+                if (k < klds) ls[k * n + i] = l;
+                L[(size_t)k * n + i] = l;
+                diag[i] = i == p ? 0.0 : diag[i] - l * l;
+            }
+        }
+        __syncthreads();
+    }
+    if (tid == 0) out[0] = rank;
+}
+
+// Step k of the same factor for larger D, one launch a step and 64 rows a work-group: the row of products
+// is rank·nbf reads, 26 us a step at nbf 1536 on one CU.  Every work-group finds the pivot in diag[k % 2] by
+// itself and writes its rows' diagonals to the other half; out[k % 2] is the state launch k finds: −2 running,
+// else the verdict of an earlier launch, which it hands on.
+constexpr int kCholRows = 64;
+__global__ void k_chol_start(const double* __restrict__ dm, int n, double* __restrict__ diag, int* __restrict__ out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) diag[i] = dm[(size_t)i * n + i];
+    if (i == 0) out[0] = -2;
+    if (i == 1) out[1] = -2;
+}
+__global__ __launch_bounds__(256) void k_chol_step(const double* __restrict__ dm, int n, int k, int kmax, double cut,
+                                                   double* __restrict__ diag, double* __restrict__ top0,
+                                                   double* __restrict__ L, int* __restrict__ out) {
+    __shared__ double wmax[4], wmin[4], part[256], lp[kCholMaxRank];
+    __shared__ int widx[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (out[k & 1] != -2) {   // finished in an earlier launch (uniform): hand the verdict on
+        if (blockIdx.x == 0 && tid == 0) out[(k + 1) & 1] = out[k & 1];
+        return;
+    }
+    const double* __restrict__ din = diag + (size_t)(k & 1) * n;
+    double mx = -INFINITY, mn = INFINITY;
+    int at = 0;
+    for (int i = tid; i < n; i += 256) {
+        const double d = din[i];
+        if (d > mx) {
+            mx = d;
+            at = i;
+        }
+        mn = fmin(mn, d);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const double m2 = __shfl_xor(mx, o, 64);
+        const int a2 = __shfl_xor(at, o, 64);
+        if (m2 > mx || (m2 == mx && a2 < at)) {
+            mx = m2;
+            at = a2;
+        }
+        mn = fmin(mn, __shfl_xor(mn, o, 64));
+    }
+    if (lane == 0) {
+        wmax[wave] = mx;
+        wmin[wave] = mn;
+        widx[wave] = at;
+    }
+    __syncthreads();
+    double top = wmax[0], low = wmin[0];
+    int p = widx[0];
+    for (int w = 1; w < 4; ++w) {
+        if (wmax[w] > top) {
+            top = wmax[w];
+            p = widx[w];
+        }
+        low = fmin(low, wmin[w]);
+    }
+    const double d0 = k == 0 ? top : top0[0];
+    const bool bad = low < -cut * d0 || !(top >= 0.0), done = top <= cut * d0;
+    if (blockIdx.x == 0 && tid == 0) {
+        if (k == 0) top0[0] = top;
+        out[(k + 1) & 1] = bad ? -1 : (done ? k : (k == kmax ? -1 : -2));   // the next launch's state
+    }
+    if (bad || done || k == kmax) return;   // uniform over the grid
+    for (int j = tid; j < k; j += 256) lp[j] = L[(size_t)j * n + p];
+    __syncthreads();
+    const int i = blockIdx.x * kCholRows + lane;
+    double v = 0.0;
+    if (i < n) {
+        int j = wave;
+        for (; j + 28 < k; j += 32) {   // eight loads in flight
+            double x[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) x[u] = L[(size_t)(j + 4 * u) * n + i];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v += x[u] * lp[j + 4 * u];
+        }
+        for (; j < k; j += 4) v += L[(size_t)j * n + i] * lp[j];
+    }
+    part[tid] = v;
+    __syncthreads();
+    if (wave == 0 && i < n) {
+        v = (part[lane] + part[lane + 64]) + (part[lane + 128] + part[lane + 192]);
+        const double inv = 1.0 / sqrt(top);
+        const double l = i == p ? top * inv : (0.5 * (dm[(size_t)p * n + i] + dm[(size_t)i * n + p]) - v) * inv;
+        L[(size_t)k * n + i] = l;
+        diag[(size_t)((k + 1) & 1) * n + i] = i == p ? 0.0 : din[i] - l * l;
+    }
+}
+
+// Per-block maxima of |½(D + Dᵀ) − Σ_{k < rank} L_k L_kᵀ|: whether the factor holds all of D.  32 × 32 blocks.
+__global__ __launch_bounds__(256) void k_chol_residual(const double* __restrict__ dm, int n, const double* __restrict__ L,
+                                                       const int* __restrict__ rank_dev, double* __restrict__ out) {
+    __shared__ double la[32][33], lb[32][33], red[256];
+    const int rank = rank_dev[0];
+    const int bi = blockIdx.x * 32, bj = blockIdx.y * 32;
+    const int x = threadIdx.x & 31, y = threadIdx.x >> 5;   // element (bi + x, bj + y + 8 q)
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    if (bi <= bj)
+        for (int k0 = 0; k0 < rank; k0 += 32) {
+            for (int r = y; r < 32; r += 8) {
+                const int k = k0 + r;
+                la[r][x] = (k < rank && bi + x < n) ? L[(size_t)k * n + bi + x] : 0.0;
+                lb[r][x] = (k < rank && bj + x < n) ? L[(size_t)k * n + bj + x] : 0.0;
+            }
+            __syncthreads();
+#pragma unroll 8
+            for (int r = 0; r < 32; ++r)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[q] += la[r][x] * lb[r][y + 8 * q];
+            __syncthreads();
+        }
+    double m = 0.0;
+    if (bi <= bj)
+        for (int q = 0; q < 4; ++q) {
+            const int i = bi + x, j = bj + y + 8 * q;
+            if (i < n && j < n) m = fmax(m, fabs(0.5 * (dm[(size_t)j * n + i] + dm[(size_t)i * n + j]) - acc[q]));
+        }
+    red[threadIdx.x] = m;
+    __syncthreads();
+    for (int h = 128; h > 0; h >>= 1) {
+        if ((int)threadIdx.x < h) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + h]);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[blockIdx.y * gridDim.x + blockIdx.x] = red[0];
+}
+
+// out[0] = max of x[0 .. n)
+__global__ __launch_bounds__(256) void k_max(const double* __restrict__ x, int n, double* __restrict__ out) {
+    __shared__ double red[256];
+    double m = 0.0;
+    for (int i = threadIdx.x; i < n; i += 256) m = fmax(m, x[i]);
+    red[threadIdx.x] = m;
+    __syncthreads();
+    for (int h = 128; h > 0; h >>= 1) {
+        if ((int)threadIdx.x < h) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + h]);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[0] = red[0];
+}
+
 unsigned grid_for(size_t n) {
     size_t g = (n + 255) / 256;
     if (g > 65536) g = 65536;
@@ -191,6 +451,37 @@ hipError_t launch_copy(hipStream_t st, void* dst, const void* src, size_t bytes)
     if (rem)
         hipLaunchKernelGGL(k_copy1, dim3(1), dim3(256), 0, st, (const unsigned char*)src + n16 * 16,
                            (unsigned char*)dst + n16 * 16, rem);
+    return hipGetLastError();
+}
+size_t pivot_chol_lds(size_t kmax) { return (kCholLds + kCholThreads + kmax) * sizeof(double); }
+hipError_t launch_pivot_chol(hipStream_t st, const double* dm, size_t nbf, size_t kmax, double cut, double* diag, double* L,
+                             int* rank, double* blockmax, double* residual) {
+    const size_t lds = pivot_chol_lds(kmax);
+    const unsigned nb = (unsigned)((nbf + 31) / 32);
+    if (nbf > kCholSmall) {
+        int* state = (int*)(blockmax + (size_t)nb * nb);            // two ints
+        double* top0 = blockmax + (size_t)nb * nb + 1;
+        hipLaunchKernelGGL(k_chol_start, dim3((unsigned)((nbf + 255) / 256)), dim3(256), 0, st, dm, (int)nbf, diag, state);
+        const unsigned g = (unsigned)((nbf + kCholRows - 1) / kCholRows);
+        for (size_t k = 0; k <= kmax; ++k)
+            hipLaunchKernelGGL(k_chol_step, dim3(g), dim3(256), 0, st, dm, (int)nbf, (int)k, (int)kmax, cut, diag, top0,
+                               L, state);
+        const hipError_t e0 = hipGetLastError();
+        if (e0 != hipSuccess) return e0;
+        int* verdict = state + ((kmax + 1) & 1);
+        hipLaunchKernelGGL(k_chol_residual, dim3(nb, nb), dim3(256), 0, st, dm, (int)nbf, L, verdict, blockmax);
+        hipLaunchKernelGGL(k_max, dim3(1), dim3(256), 0, st, blockmax, (int)(nb * nb), residual);
+        hipLaunchKernelGGL(k_copy1, dim3(1), dim3(256), 0, st, (const unsigned char*)verdict, (unsigned char*)rank,
+                           sizeof(int));
+        return hipGetLastError();
+    }
+    // more LDS than a launch's default limit
+    const hipError_t e =
+        hipFuncSetAttribute((const void*)k_pivot_chol, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_pivot_chol, dim3(1), dim3(kCholThreads), lds, st, dm, (int)nbf, (int)kmax, cut, diag, L, rank);
+    hipLaunchKernelGGL(k_chol_residual, dim3(nb, nb), dim3(256), 0, st, dm, (int)nbf, L, rank, blockmax);
+    hipLaunchKernelGGL(k_max, dim3(1), dim3(256), 0, st, blockmax, (int)(nb * nb), residual);
     return hipGetLastError();
 }
 unsigned asym_stats_blocks(size_t nbf) {
