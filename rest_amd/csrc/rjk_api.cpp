@@ -520,7 +520,7 @@ void k_plan_cols(KPlan& kp, size_t nbf, const size_t* ncol, int ns, int prec) {
     kp.col_off[1] = kp.col_cnt[0];
     const size_t tot = kp.col_cnt[0] + kp.col_cnt[1];
     if (is_bf16(prec)) {
-        kp.nk = round_up(tot, kColPad);
+        kp.nk = tot;
     } else {
         kp.fn = k_tile_groups(tot / kTileK, prec);
         kp.nk = round_up(tot, (size_t)kp.fn * kTileK);
@@ -534,6 +534,13 @@ size_t k_slots(size_t naux, size_t chunk, size_t nsplit) {
         return Pc ? (Pc + pps - 1) / pps : 0;
     };
     return std::max<size_t>(1, std::max(filled(std::min(chunk, naux)), filled(naux % chunk)));
+}
+
+// occupied columns as padded for the split sizes and counted by the profiler: to 64 over all spins,
+// BF16 to 64 a spin
+size_t padded_cols(const KPlan& kp, int prec) {
+    if (is_bf16(prec)) return round_up(kp.col_cnt[0], kColPad) + round_up(kp.col_cnt[1], kColPad);
+    return round_up(kp.col_cnt[0] + kp.col_cnt[1], kColPad);
 }
 
 // chunking and split-K; carves [cocc | sign | kpart | M'] out of the workspace.
@@ -563,7 +570,7 @@ int k_plan_ws(rjk_ctx* ctx, KPlan& kp, int ns, int prec, void** cocc, void** sig
         // with naux.  Up to half the workspace goes to the partials.  The splits follow from the sizes
         // padded to 128 rows and 64 columns, not from the tiles chosen, so that no choice of
         // tile changes where an FP32 sum ends.
-        const size_t pad = round_up(ctx->nbf, kTileMN), nk = round_up(kp.nk ? kp.col_cnt[0] + kp.col_cnt[1] : 0, kColPad);
+        const size_t pad = round_up(ctx->nbf, kTileMN), nk = padded_cols(kp, prec);
         const size_t nt = pad / kTileMN, ntiles = nt * (nt + 1) / 2;
         const size_t slot_bytes = (size_t)ns * pad * pad * sizeof(double), perP_ = nk * pad * es;
         const size_t small = round_up(pad * nk * es, 256) + round_up(nk * es, 256);
@@ -606,7 +613,7 @@ int k_run(rjk_ctx* ctx, const KPlan& kp, int ns, int prec, const void* b, const 
         return RJK_OK;
     }
     const bool bf = is_bf16(prec);
-    const double work_nk = (double)round_up(kp.col_cnt[0] + kp.col_cnt[1], kColPad);   // profiler's column count
+    const double work_nk = (double)padded_cols(kp, prec);
     for (size_t P0 = 0; P0 < ctx->naux; P0 += kp.chunk) {
         size_t Pc = std::min(kp.chunk, ctx->naux - P0);
         const double nb = (double)ctx->nbf;
@@ -617,7 +624,7 @@ int k_run(rjk_ctx* ctx, const KPlan& kp, int ns, int prec, const void* b, const 
         }
         {
             PhaseScope ps(ctx, 3, prec, nb * (nb + 1.0) * work_nk * (double)Pc);
-            if (bf) RJK_HIP(ctx, launch_bf_ksyrk(st, prec, m, Pc, kp, ns, sign, P0 > 0 ? 1 : 0, kpart));
+            if (bf) RJK_HIP(ctx, launch_bf_ksyrk(st, prec, m, ctx->nbf, Pc, kp, ns, sign, P0 > 0 ? 1 : 0, kpart));
             else RJK_HIP(ctx, launch_ksyrk(st, prec, m, ctx->nbf, Pc, kp, ns, sign, P0 > 0 ? 1 : 0, kpart));
         }
     }

@@ -294,17 +294,6 @@ __device__ inline void split_to(double x, __bf16* out) {
     }
 }
 
-template <int S>
-__device__ inline void split_to_f(float x, __bf16* out) {
-    float r = x;
-#pragma unroll
-    for (int k = 0; k < S; ++k) {
-        const __bf16 h = (__bf16)r;
-        out[k] = h;
-        r -= (float)h;
-    }
-}
-
 // C'ᵀ planes (column c of C diag(sqrt|occ|) as a row, ν fastest) and sign masks
 template <int S>
 __global__ __launch_bounds__(256) void k_b_bf_prep(const BProb* __restrict__ pr, int np, Tables tb) {
@@ -427,7 +416,7 @@ __device__ __forceinline__ void bf_half_tile(__bf16* __restrict__ lds, const RJK
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 __bf16 h[S];
-                split_to_f<S>(rb[j][i], h);
+                split_f<S>(rb[j][i], h);
 #pragma unroll
                 for (int k = 0; k < S; ++k) v[k][i] = h[k];
             }
@@ -471,20 +460,11 @@ __device__ __forceinline__ void bf_half_tile(__bf16* __restrict__ lds, const RJK
         __builtin_amdgcn_s_setprio(0);
         __syncthreads();
     }
-    // M' planes: lane holds c = c0 + 16(wx FX + i) + 4(l/16) + r for μ = mu0 + 16(wy FY + j) + l%16
 #pragma unroll
     for (int i = 0; i < H::FX; ++i)
 #pragma unroll
-        for (int j = 0; j < H::FY; ++j) {
-            const int c = c0 + (wx * H::FX + i) * 16 + 4 * (lane >> 4);
-            const int mu = mu0 + (wy * H::FY + j) * 16 + l16;
-            __bf16 h[4][S];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) split_to_f<S>(acc[i][j][r] + acc2[i][j][r], h[r]);
-#pragma unroll
-            for (int k = 0; k < S; ++k)
-                *(RJK_GLB bft::bf4*)(mP + (size_t)k * pm + (size_t)mu * nk + c) = bft::bf4{h[0][k], h[1][k], h[2][k], h[3][k]};
-        }
+        for (int j = 0; j < H::FY; ++j)
+            store_m<S>(mP, pm, mu0 + (wy * H::FY + j) * 16, c0 + (wx * H::FX + i) * 16, nk, lane, acc[i][j] + acc2[i][j]);
 }
 
 // half-transform over the problems of one tile class: round_up(naux, 8) · ntm · ntc items per problem
@@ -510,6 +490,8 @@ __global__ __launch_bounds__(256) void k_b_bf_khalf(const BProb* __restrict__ pr
     }
 }
 
+__device__ inline int rup32(int n) { return (n + 31) / 32 * 32; }
+
 // SYRK over the problems of one tile class: nsplit · ntile2 items per problem (split s on XCD s % 8),
 // Kpart[split][ν][μ] = Σ_{P in split, c} sign_c M'_P[ν][c] M'_P[μ][c] on upper tile pairs
 template <class C>
@@ -529,25 +511,18 @@ __global__ __launch_bounds__(C::NT) void k_b_bf_ksyrk(const BProb* __restrict__ 
         size_t tm, tn;
         upper_tile(t, &tm, &tn);
         const int mu0 = (int)tm * C::WGY, nu0 = (int)tn * C::WGX;
-        const int ncb = (P.nocc + C::TK - 1) / C::TK;
         const int Pb = split * P.pps, Pe = min(P.naux, Pb + P.pps);
-        const int nq = (Pe > Pb ? Pe - Pb : 0) * ncb;
         const size_t mplane = (size_t)P.naux * P.nbf_pad * P.nk, mPs = (size_t)P.nbf_pad * P.nk;
         const RJK_GLB __bf16* mpl = glb((const __bf16*)P.m);
         const RJK_GLB unsigned short* smask = glb((const unsigned short*)P.sign);
         bft::f4 acc[C::FX][C::FY], acc2[C::FX][C::FY];   // leading product; corrections
-        bft::nt_tile2<C, true>(
-            lds, [&](int q) { return mpl + (Pb + q / ncb) * mPs + (size_t)nu0 * P.nk + (q % ncb) * C::TK; },
-            (size_t)P.nk, mplane,
-            [&](int q) { return mpl + (Pb + q / ncb) * mPs + (size_t)mu0 * P.nk + (q % ncb) * C::TK; },
-            (size_t)P.nk, mplane,
-            [&](int q, int pc) {
-                const RJK_GLB unsigned short* sm = smask + (q % ncb) * C::TK + pc;
-                return bft::u4{(unsigned)sm[0] | ((unsigned)sm[1] << 16), (unsigned)sm[2] | ((unsigned)sm[3] << 16),
-                               (unsigned)sm[4] | ((unsigned)sm[5] << 16), (unsigned)sm[6] | ((unsigned)sm[7] << 16)};
-            },
-            nq, acc, acc2);
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wx = wave % C::WX, wy = wave / C::WX;
+        const int wnu = nu0 + wx * C::FX * 16, wmu = mu0 + wy * C::FY * 16;
+        const bool live = wnu < P.nbf && wmu < P.nbf && wmu < wnu + C::FX * 16;   // else nothing of it is read
+        const auto base = mpl + (size_t)Pb * mPs;
+        bft::nt_tile2<C, true>(lds, base + (size_t)nu0 * P.nk, base + (size_t)mu0 * P.nk, (size_t)16 * P.nk, mplane, mPs,
+                               smask, max(0, Pe - Pb), rup32(P.nocc), live, acc, acc2);
+        if (!live) continue;
         RJK_GLB double* __restrict__ kp = glb(P.kpart) + (size_t)split * P.nbf_pad * P.nbf_pad;
 #pragma unroll
         for (int i = 0; i < C::FX; ++i)
@@ -594,7 +569,7 @@ BProb geometry(size_t nbf, size_t naux, size_t nocc, int prec) {
     if (is_bf(prec)) {
         P.nbf_pad = (int)rup(nbf, 64);     // the 64-wide BF16 tiles; 128-wide ones where nbf_pad % 128 == 0
         P.ncb = 0;
-        P.nk = (int)rup(nocc, kBfColGran);
+        P.nk = (int)rup(nocc, kColPad);
     } else {
         P.nbf_pad = (int)rup(nbf, kTileMN);
         P.ncb = (int)(rup(nocc, kTileK) / kTileK);
@@ -817,8 +792,8 @@ int enqueue_bf(rjk_batch* b, hipEvent_t* ev) {
     using H2 = BfHalf<S, 64, TK, 192>;
     using H3 = BfHalf<S, 128, TK, 64>;
     using H4 = BfHalf<S, 128, TK, 128>;
-    using Y0 = bft::Cfg<S, 64, 64, 2, 2, false, TK>;
-    using Y1 = bft::Cfg<S, 128, 128, 2, 4, false, TK>;
+    using Y0 = bft::Cfg<S, 64, 64, 2, 2, TK>;
+    using Y1 = bft::Cfg<S, 128, 128, 2, 4, TK>;
     const int np = (int)b->h.size();
     const Tables tb = tables(b);
     const hipStream_t st = b->stream;

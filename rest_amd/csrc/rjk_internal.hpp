@@ -21,7 +21,7 @@ constexpr int kNumPhases = 5;        // J-gamma, J-acc, K-half, K-syrk, K-other
 constexpr int kTileMN = 128;         // nbf padding for the K tiles
 constexpr int kTileK = 16;           // k-block of the K tiles
 constexpr int kColPad = 64;          // occupied-column padding of M (all spins)
-constexpr int kBfColGran = 64;       // BF16 K: per-spin column granule (the deepest SYRK k-block)
+constexpr int kBfColGran = 32;       // BF16 K: per-spin column granule (one MFMA deep)
 constexpr int kBfStoredPlanes = 3;   // BF16 planes kept per B element (RJK_STORE_BF16)
 constexpr int kNumPrec = RJK_NUM_PREC; // profile rows: one per RJK_PREC_* value
 
@@ -131,7 +131,7 @@ struct KPlan {
     size_t tile = kTileMN;   // SYRK tile rows (64 or 128; BF16: kTileMN)
     int fn = 4;              // FP64/FP32: 16-column groups of a half-transform tile
     size_t nbf_pad = 0;      // multiple of `tile`; BF16: of kTileMN
-    size_t nk = 0;           // padded occupied columns, all spins (multiple of 16·fn; BF16: of kColPad)
+    size_t nk = 0;           // padded occupied columns, all spins (multiple of 16·fn; BF16: of kBfColGran)
     size_t col_off[2] = {0, 0}, col_cnt[2] = {0, 0};   // per-spin column ranges (multiples of 16)
     size_t chunk = 0;        // P per chunk
     size_t nsplit = 0;       // split-K divisor of the SYRK: a chunk of Pc columns takes ceil(Pc / nsplit) a split
@@ -165,7 +165,7 @@ hipError_t launch_bf_prep_c_idx(hipStream_t st, int prec, const double* vecs, si
                                 void* smask);
 hipError_t launch_bf_khalf(hipStream_t st, int prec, const void* bpl, size_t naux, size_t nbf, size_t P0, size_t Pc,
                            const KPlan& kp, const void* ct, void* mpl);
-hipError_t launch_bf_ksyrk(hipStream_t st, int prec, const void* mpl, size_t Pc, const KPlan& kp, int nspin,
+hipError_t launch_bf_ksyrk(hipStream_t st, int prec, const void* mpl, size_t nbf, size_t Pc, const KPlan& kp, int nspin,
                            const void* smask, int beta, double* kpart);
 
 // util

@@ -10,16 +10,18 @@
 // A[l%16][8(l/16)+i] and B[8(l/16)+i][l%16]; register r of lane l receives
 // D[4(l/16)+r][l%16] (probed on gfx950).  Split-K partials join an FP64 sum.
 //
-// Layouts (BF16 planes, padding zero; nbf_pad a multiple of 128, nk of 64):
-//   B planes  [S][naux][nbf_pad][nbf_pad]  full symmetric squares (aligned 16-byte row pieces)
-//   C' planes [S][nk][nbf_pad]             C'ᵀ: column c of C' as a row, ν fastest
-//   M' planes [S][Pc][nbf_pad][nk]         c fastest, so both SYRK operands load as rows
-// Stage 1: M'_P[μ][c] = Σ_ν C'ᵀ[c][ν] B_P[ν][μ]                  (128 μ × 64 c tiles)
+// Layouts (BF16 planes as 16 × 32 fragments, rjk_bftile.hpp; padding zero; nbf_pad a multiple of
+// 128, nk of 32):
+//   B planes  [S][naux] of nbf_pad × nbf_pad   full symmetric squares
+//   C' planes [S] of nk × nbf_pad              C'ᵀ: column c of C' as a row
+//   M' planes [S][Pc] of nbf_pad × nk          c along the rows of a fragment: both SYRK operands
+// Stage 1: M'_P[μ][c] = Σ_ν C'ᵀ[c][ν] B_P[ν][μ]                  (128 μ × up to 160 c tiles)
 // Stage 2: Kpart[split][s][ν][μ] (+)= Σ_{P,c} sign_c M'_P[ν][c] M'_P[μ][c]  (128 × 128 upper tiles)
 // Stage 3: the FP64 split reduction of rjk_k.hip.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "rjk_bftile.hpp"
 #include "rjk_internal.hpp"
@@ -44,36 +46,41 @@ __device__ inline void split_d(double x, __bf16* out) {
     }
 }
 
-template <int S>
-__device__ inline void split_f(float x, __bf16* out) {
-    float r = x;
-#pragma unroll
-    for (int k = 0; k < S; ++k) {
-        const __bf16 h = (__bf16)r;
-        out[k] = h;
-        r -= (float)h;
-    }
-}
-
 // ---- conversions ---------------------------------------------------------------
 // B planes of auxiliary columns [P0, P0 + Pc) from the packed FP64 B (upper triangle,
 // element (i<=j) at j(j+1)/2 + i)
 template <int S>
 __global__ void k_bf_planes_b(const double* __restrict__ b64, size_t ldb, int nbf, int nbf_pad, size_t naux,
                               size_t P0, size_t Pc, __bf16* __restrict__ planes) {
-    const size_t sq = (size_t)nbf_pad * nbf_pad, total = Pc * sq;
-    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-        const size_t P = t / sq, e = t % sq;
-        const int mu = (int)(e / nbf_pad), nu = (int)(e % nbf_pad);
-        double x = 0.0;
-        if (mu < nbf && nu < nbf) {
-            const size_t lo = mu < nu ? mu : nu, hi = mu < nu ? nu : mu;
-            x = b64[(P0 + P) * ldb + tri_b(hi) + lo];
-        }
-        __bf16 h[S];
-        split_d<S>(x, h);
+    // A wave a fragment (nbf_pad²/512 of them, a multiple of the block's 4): read along the packed
+    // column, lanes on ν left of the diagonal and on μ beyond it, and turned through LDS.
+    __shared__ double tile[4][16][bft::KM + 1];
+    const size_t sq = (size_t)nbf_pad * nbf_pad, per = sq / bft::FRAG, total = Pc * per;
+    const int n32 = nbf_pad / bft::KM, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (size_t t0 = (size_t)blockIdx.x * 4; t0 < total; t0 += (size_t)gridDim.x * 4) {
+        const size_t P = (t0 + wave) / per;
+        const int f = (int)((t0 + wave) % per), mu0 = f / n32 * 16, nu0 = f % n32 * bft::KM;
+        const double* __restrict__ col = b64 + (P0 + P) * ldb;
+        const bool left = nu0 < mu0;
 #pragma unroll
-        for (int k = 0; k < S; ++k) planes[((size_t)k * naux + P0 + P) * sq + e] = h[k];
+        for (int i = 0; i < 8; ++i) {
+            const int e = i * 64 + lane, r = left ? e / bft::KM : e % 16, c = left ? e % bft::KM : e / 16;
+            const int mu = mu0 + r, nu = nu0 + c, lo = mu < nu ? mu : nu, hi = mu < nu ? nu : mu;
+            tile[wave][r][c] = hi < nbf ? col[tri_b(hi) + lo] : 0.0;
+        }
+        __syncthreads();
+        bft::bf8 v[S];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            __bf16 h[S];
+            split_d<S>(tile[wave][lane & 15][(lane >> 4) * 8 + i], h);
+#pragma unroll
+            for (int k = 0; k < S; ++k) v[k][i] = h[k];
+        }
+#pragma unroll
+        for (int k = 0; k < S; ++k)
+            *(bft::bf8*)(planes + ((size_t)k * naux + P0 + P) * sq + (size_t)f * bft::FRAG + lane * 8) = v[k];
+        __syncthreads();
     }
 }
 
@@ -101,7 +108,7 @@ __global__ void k_bf_prep_c(const double* __restrict__ eigv, int nbf, int nstate
         __bf16 h[S];
         split_d<S>(v, h);
 #pragma unroll
-        for (int k = 0; k < S; ++k) ct[(size_t)k * total + t] = h[k];
+        for (int k = 0; k < S; ++k) ct[(size_t)k * total + bft::frag_elem(c, nu, nbf_pad)] = h[k];
         if (nu == 0) smask[c] = w < 0 ? 0x8000 : 0;
     }
 }
@@ -119,88 +126,86 @@ __global__ void k_bf_prep_c_idx(const double* __restrict__ vecs, int nbf, const 
         const double v = nu < nbf ? vecs[(size_t)idx[q] * nbf + nu] * sqrt(fabs(w)) : 0.0;
         __bf16 h[S];
         split_d<S>(v, h);
-        const size_t e = (size_t)(col_off + q) * nbf_pad + nu;
+        const size_t e = bft::frag_elem(col_off + q, nu, nbf_pad);
 #pragma unroll
         for (int k = 0; k < S; ++k) ct[(size_t)k * plane + e] = h[k];
         if (nu == 0) smask[col_off + q] = w < 0 ? 0x8000 : 0;
     }
 }
 
-// Tile shapes from a sweep at nbf 1536, nk 320, 256 auxiliary columns per launch (executed
-// BF16 MFMA rate, accumulators in VGPRs, the conflict-free LDS swizzle of rjk_bftile.hpp), then
-// checked in the K build itself (about 1000 auxiliary columns per launch):
-//   half-transform, 2 planes: 64 c × 256 μ on 1 × 4 waves, 64-deep: 5.39 ms per launch in the
-//     build against 5.46 for 64 × 128 on 2 × 2 waves (the sweep, at a quarter of the columns,
-//     ranks them the other way: 747 against 857 TFLOP/s); needs nbf_pad % 256 == 0, else 64 × 128;
-//   half-transform, 3 planes: 64 c × 128 μ on 2 × 4 waves, 64-deep: 9.34 ms per 1024 columns
-//     (2 × 2 waves: 9.64; 64 × 256 on 2 × 4: 10.24);
-//   SYRK, 2 planes: 128 × 128 on 2 × 4 waves, 64-deep: 988 (2 × 2 waves: 951; in the build 2.66
-//     against 2.93 ms per launch);
-//   SYRK, 3 planes: 128 × 128 on 2 × 4 waves, 32-deep: 1110 (2 × 2 waves: 1077; 64-deep: 1043).
+// SYRK tiles, measured in the K build: two planes 128 × 128 on 2 × 4 waves, 64-deep (nbf 768, 160
+// columns: 1.20 ms; 32-deep 1.28, 2 × 2 waves 1.31); three planes the same 32-deep (nbf 900, 190
+// columns: 4.5 ms; 2 × 2 waves 5.9, 4 × 2 waves 5.3).  Both run at the rate that a large BF16 matrix
+// product reaches on this card, whose clock falls under that load (1.5 GHz in the two-plane SYRK).
 template <int S> struct KbfTiles;
 template <> struct KbfTiles<2> {
-    using Half = bft::Cfg<2, 64, 256, 1, 4, false, 64>;    // X = 64 c, Y = 256 μ
-    using HalfNarrow = bft::Cfg<2, 64, 128, 2, 2, false, 64>;
-    using Syrk = bft::Cfg<2, 128, 128, 2, 4, false, 64>;   // X = 128 ν, Y = 128 μ
+    using Syrk = bft::Cfg<2, 128, 128, 2, 4, 64>;   // X = 128 ν, Y = 128 μ
 };
 template <> struct KbfTiles<1> {
-    using Half = bft::Cfg<1, 64, 256, 1, 4, false, 64>;
-    using HalfNarrow = bft::Cfg<1, 64, 128, 2, 2, false, 64>;
-    using Syrk = bft::Cfg<1, 128, 128, 2, 4, false, 64>;
+    using Syrk = bft::Cfg<1, 128, 128, 2, 4, 64>;
 };
 template <> struct KbfTiles<3> {
-    using Half = bft::Cfg<3, 64, 128, 2, 4, false, 64>;
-    using Syrk = bft::Cfg<3, 128, 128, 2, 4, false, 32>;
+    using Syrk = bft::Cfg<3, 128, 128, 2, 4, 32>;
 };
 
 // ---- stage 1 -------------------------------------------------------------------
+// Y fragments from the B planes
+template <int S, int FM>
+struct PlaneRows {
+    struct Raw { bft::u4 v[S]; };
+    const __bf16* base;      // first fragment of the wave's rows, plane 0 (uniform)
+    size_t plane, row;       // elements between planes and row fragments
+    __device__ __forceinline__ void load(int s, Raw (&r)[FM]) const {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int k = 0; k < S; ++k)
+#pragma unroll
+            for (int j = 0; j < FM; ++j)
+                r[j].v[k] = bft::ld16(base + k * plane + j * row + (size_t)s * bft::FRAG + lane * 8);
+    }
+    __device__ __forceinline__ void frag(const Raw& r, bft::bf8 (&f)[S]) const {
+#pragma unroll
+        for (int k = 0; k < S; ++k) f[k] = __builtin_bit_cast(bft::bf8, r.v[k]);
+    }
+};
+
 // 1-D grid, XCD-aware: every tile of auxiliary column P runs on XCD P % 8 and the
 // column tiles of one μ tile are consecutive there, so they share B's rows in L2.
-template <class C>
-__global__ __launch_bounds__(C::NT) void k_bf_khalf(const __bf16* __restrict__ bpl, size_t naux, int nbf,
-                                                    int nbf_pad, size_t P0, int Pc, int ntm, int ntc,
-                                                    const __bf16* __restrict__ ct, int nk,
-                                                    __bf16* __restrict__ mpl) {
-    constexpr int S = C::S;
-    __shared__ __bf16 lds[C::LDS_ELEMS];
+template <class H>
+__global__ __launch_bounds__(H::NT, 2) void k_bf_khalf(const __bf16* __restrict__ bpl, size_t naux, int nbf,
+                                                       int nbf_pad, size_t P0, int Pc, int ntm, int ntc,
+                                                       const __bf16* __restrict__ ct, int nk,
+                                                       __bf16* __restrict__ mpl) {
+    constexpr int S = H::S;
+    __shared__ __bf16 lds[H::LDS_ELEMS];
     const int w = blockIdx.x, xcd = w % kXcdB, kq = w / kXcdB, per = ntm * ntc;
     const int Pl = (kq / per) * kXcdB + xcd;
     if (Pl >= Pc) return;   // padding work-groups (uniform exit)
-    const int rem = kq % per, mt = rem / ntc, ctile = rem % ntc;
-    const int mu0 = mt * C::WGY, c0 = ctile * C::WGX;
+    const int rem = kq % per, mt = rem / ntc, c0 = (rem % ntc) * H::TC;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int mu0 = mt * H::TMU + wave * 16 * H::FM;
     const size_t sq = (size_t)nbf_pad * nbf_pad;
-    const __bf16* __restrict__ bP = bpl + (P0 + Pl) * sq + (size_t)mu0 * nbf_pad;
-    const __bf16* __restrict__ cT = ct + (size_t)c0 * nbf_pad;
-    bft::f4 acc[C::FX][C::FY];
-    // D[c][μ] = Σ_ν C'ᵀ[c][ν] B[μ][ν]  (B_P symmetric; padding rows and columns are zero)
-    bft::nt_tile<C>(lds, [&](int q) { return cT + q * C::TK; }, (size_t)nbf_pad, (size_t)nk * nbf_pad,
-                    [&](int q) { return bP + q * C::TK; }, (size_t)nbf_pad, naux * sq,
-                    [](int, int) { return bft::u4{0, 0, 0, 0}; }, (nbf + C::TK - 1) / C::TK, acc);
-    // M' planes: lane holds c = cb + 4(l/16) + r for μ = mb + l%16
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wx = wave % C::WX, wy = wave / C::WX;
+    const PlaneRows<S, H::FM> y{bpl + (P0 + Pl) * sq + (size_t)mu0 * nbf_pad, naux * sq, (size_t)16 * nbf_pad};
+    bft::f4 acc[H::FX][H::FM];
+    // B_P symmetric; padding rows and columns are zero
+    bft::half_tile<H, false>(lds, ct, nk, nbf_pad / bft::KM, c0, (nbf + bft::KM - 1) / bft::KM, mu0 < nbf, y, acc, acc);
+    if (mu0 >= nbf_pad) return;
     const size_t mplane = (size_t)Pc * nbf_pad * nk;
     __bf16* __restrict__ mP = mpl + (size_t)Pl * nbf_pad * nk;
 #pragma unroll
-    for (int i = 0; i < C::FX; ++i)
+    for (int i = 0; i < H::FX; ++i) {
+        if (c0 + i * 16 >= nk) break;
 #pragma unroll
-        for (int j = 0; j < C::FY; ++j) {
-            const int c = c0 + (wx * C::FX + i) * 16 + 4 * (lane >> 4);
-            const int mu = mu0 + (wy * C::FY + j) * 16 + (lane & 15);
-            __bf16 h[4][S];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) split_f<S>(acc[i][j][r], h[r]);
-#pragma unroll
-            for (int k = 0; k < S; ++k)
-                *(bf4*)(mP + (size_t)k * mplane + (size_t)mu * nk + c) = bf4{h[0][k], h[1][k], h[2][k], h[3][k]};
-        }
+        for (int j = 0; j < H::FM; ++j) bft::store_m<S>(mP, mplane, mu0 + j * 16, c0 + i * 16, nk, lane, acc[i][j]);
+    }
 }
 
 // ---- stage 2 -------------------------------------------------------------------
 // 1-D grid of (nslot rounded up to 8) × nspin × ntile2 work-groups (split s
 // on XCD s % 8).  Upper tile pairs (μ tile <= ν tile) of 128 × 128.
 template <class C>
-__global__ __launch_bounds__(C::NT) void k_bf_ksyrk(const __bf16* __restrict__ mpl, int Pc, int nbf_pad,
-                                                    int nk, int ntile2, int nspin, int off0, int cnt0,
+__global__ __launch_bounds__(C::NT, 4) void k_bf_ksyrk(const __bf16* __restrict__ mpl, int Pc, int nbf,
+                                                    int nbf_pad, int nk, int ntile2, int nspin, int off0, int cnt0,
                                                     int off1, int cnt1,
                                                     const unsigned short* __restrict__ smask, int nslot,
                                                     int p_per_split, int beta, double* __restrict__ kpart,
@@ -217,22 +222,17 @@ __global__ __launch_bounds__(C::NT) void k_bf_ksyrk(const __bf16* __restrict__ m
     const size_t tm = t - tri_b(tn);
     const int mu0 = (int)tm * C::WGY, nu0 = (int)tn * C::WGX;
     const int cb = spin == 0 ? off0 : off1, cnt = spin == 0 ? cnt0 : cnt1;
-    const int ncb = (cnt + C::TK - 1) / C::TK;
-    const int nq = (Pe > Pb ? Pe - Pb : 0) * ncb;
     const size_t mplane = (size_t)Pc * nbf_pad * nk, mP = (size_t)nbf_pad * nk;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wx = wave % C::WX, wy = wave / C::WX;
+    // outputs of this wave: nothing of them is read beyond nbf or below the diagonal
+    const int wnu = nu0 + wx * C::FX * 16, wmu = mu0 + wy * C::FY * 16;
+    const bool live = wnu < nbf && wmu < nbf && wmu < wnu + C::FX * 16;
     bft::f4 acc[C::FX][C::FY];
     // D[ν][μ] = Σ_c sign_c M'[ν][c] M'[μ][c]
-    bft::nt_tile<C>(
-        lds, [&](int q) { return mpl + (Pb + q / ncb) * mP + (size_t)nu0 * nk + cb + (q % ncb) * C::TK; }, (size_t)nk,
-        mplane, [&](int q) { return mpl + (Pb + q / ncb) * mP + (size_t)mu0 * nk + cb + (q % ncb) * C::TK; },
-        (size_t)nk, mplane,
-        [&](int q, int pc) {
-            const unsigned short* sm = smask + cb + (q % ncb) * C::TK + pc;
-            return bft::u4{(unsigned)sm[0] | ((unsigned)sm[1] << 16), (unsigned)sm[2] | ((unsigned)sm[3] << 16),
-                           (unsigned)sm[4] | ((unsigned)sm[5] << 16), (unsigned)sm[6] | ((unsigned)sm[7] << 16)};
-        },
-        nq, acc);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wx = wave % C::WX, wy = wave / C::WX;
+    const __bf16* __restrict__ base = mpl + (size_t)Pb * mP + (size_t)(cb / bft::KM) * bft::FRAG;
+    bft::nt_tile<C>(lds, base + (size_t)nu0 * nk, base + (size_t)mu0 * nk, (size_t)16 * nk, mplane, mP, smask + cb,
+                    max(0, Pe - Pb), cnt, live, acc);
+    if (!live) return;
     double* __restrict__ kp = kpart + ((size_t)split * nspin + spin) * slot;
 #pragma unroll
     for (int i = 0; i < C::FX; ++i)
@@ -262,7 +262,7 @@ hipError_t launch_bf_planes_b(hipStream_t st, const double* b64, size_t ldb, siz
     const size_t sq = nbf_pad * nbf_pad, slab = std::max<size_t>(1, (size_t(1) << 28) / sq);
     for (size_t P0 = 0; P0 < naux; P0 += slab) {
         const size_t Pc = std::min(slab, naux - P0);
-        hipLaunchKernelGGL(k_bf_planes_b<kBfStoredPlanes>, dim3(gs_blocks(Pc * sq)), dim3(256), 0, st, b64, ldb,
+        hipLaunchKernelGGL(k_bf_planes_b<kBfStoredPlanes>, dim3(gs_blocks(Pc * sq / 8)), dim3(256), 0, st, b64, ldb,
                            (int)nbf, (int)nbf_pad, naux, P0, Pc, (__bf16*)planes);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -306,23 +306,49 @@ hipError_t launch_bf_prep_c_idx(hipStream_t st, int prec, const double* vecs, si
 
 namespace {
 
-template <class C>
+template <class H>
 hipError_t bf_khalf_t(hipStream_t st, const void* bpl, size_t naux, size_t nbf, size_t P0, size_t Pc, const KPlan& kp,
                       const void* ct, void* mpl) {
-    const int ntm = (int)(kp.nbf_pad / C::WGY), ntc = (int)(kp.nk / C::WGX);
+    const int ntm = (int)((kp.nbf_pad + H::TMU - 1) / H::TMU), ntc = (int)((kp.nk + H::TC - 1) / H::TC);
     const size_t nwg = ((Pc + kXcdB - 1) / kXcdB * kXcdB) * (size_t)ntm * ntc;
-    hipLaunchKernelGGL(k_bf_khalf<C>, dim3((unsigned)nwg), dim3(C::NT), 0, st, (const __bf16*)bpl, naux, (int)nbf,
+    hipLaunchKernelGGL(k_bf_khalf<H>, dim3((unsigned)nwg), dim3(H::NT), 0, st, (const __bf16*)bpl, naux, (int)nbf,
                        (int)kp.nbf_pad, P0, (int)Pc, ntm, ntc, (const __bf16*)ct, (int)kp.nk, (__bf16*)mpl);
     return hipGetLastError();
 }
 
+// Columns go in tiles of up to 12 fragments, all of one width.  12 against 10 (the columns then in two
+// tiles): nbf 768, 192 columns 2.33 against 2.59 ms with two planes, 3.98 against 4.16 with three; 16 is no
+// faster (nbf 900, 256 columns: 4.61 against 4.12 ms).  Eight waves share C'ᵀ where their 256 rows are
+// no great part of nbf and the tile is wide: nbf 645, 160 columns 2.36 against 2.58 ms with three planes,
+// nbf 768 two planes 2.09 against 2.16; four at nbf 300 (0.133 against 0.143 ms) and for 6 fragments
+// (nbf 900, three planes: 6.43 against 6.81 ms).
+template <int S>
+hipError_t bf_khalf_s(hipStream_t st, const void* bpl, size_t naux, size_t nbf, size_t P0, size_t Pc, const KPlan& kp,
+                      const void* ct, void* mpl) {
+    const size_t f = kp.nk / 16, tiles = (f + 11) / 12, fx = round_up((f + tiles - 1) / tiles, 2);
+    auto go = [&](auto fx_) -> hipError_t {
+        constexpr int FX = decltype(fx_)::value;
+        if constexpr (FX >= 8)
+            if (nbf > 512) return bf_khalf_t<bft::HalfCfg<S, FX, 2, 8>>(st, bpl, naux, nbf, P0, Pc, kp, ct, mpl);
+        return bf_khalf_t<bft::HalfCfg<S, FX, 2, 4>>(st, bpl, naux, nbf, P0, Pc, kp, ct, mpl);
+    };
+    switch (fx) {
+        case 2: return go(std::integral_constant<int, 2>{});
+        case 4: return go(std::integral_constant<int, 4>{});
+        case 6: return go(std::integral_constant<int, 6>{});
+        case 8: return go(std::integral_constant<int, 8>{});
+        case 10: return go(std::integral_constant<int, 10>{});
+        default: return go(std::integral_constant<int, 12>{});
+    }
+}
+
 template <class C>
-hipError_t bf_ksyrk_t(hipStream_t st, const void* mpl, size_t Pc, const KPlan& kp, int nspin, const void* smask,
+hipError_t bf_ksyrk_t(hipStream_t st, const void* mpl, size_t nbf, size_t Pc, const KPlan& kp, int nspin, const void* smask,
                       int beta, double* kpart) {
     const size_t nt = kp.nbf_pad / C::WGX, nt2 = nt * (nt + 1) / 2;
     const int pps = (int)((Pc + kp.nsplit - 1) / kp.nsplit);
     const size_t nwg = round_up(kp.nslot, kXcdB) * (size_t)nspin * nt2;
-    hipLaunchKernelGGL(k_bf_ksyrk<C>, dim3((unsigned)nwg), dim3(C::NT), 0, st, (const __bf16*)mpl, (int)Pc,
+    hipLaunchKernelGGL(k_bf_ksyrk<C>, dim3((unsigned)nwg), dim3(C::NT), 0, st, (const __bf16*)mpl, (int)Pc, (int)nbf,
                        (int)kp.nbf_pad, (int)kp.nk, (int)nt2, nspin, (int)kp.col_off[0], (int)kp.col_cnt[0],
                        (int)kp.col_off[1], (int)kp.col_cnt[1], (const unsigned short*)smask, (int)kp.nslot, pps, beta, kpart,
                        kp.nbf_pad * kp.nbf_pad);
@@ -331,27 +357,23 @@ hipError_t bf_ksyrk_t(hipStream_t st, const void* mpl, size_t Pc, const KPlan& k
 
 }  // namespace
 
-// Tile preconditions: nbf_pad a multiple of 128 (both SYRK tiles, the narrow half-transform
-// tile) or of 256 (the wide one, chosen only then); nk a multiple of 64 (the c tiles); every
-// spin's column count a multiple of kBfColGran = 64 (the deepest k-block).
+// Tile preconditions: nbf_pad a multiple of 128 (SYRK tiles; whole waves of half-transform rows), every
+// spin's column count a multiple of 32 (one MFMA deep).
 hipError_t launch_bf_khalf(hipStream_t st, int prec, const void* bpl, size_t naux, size_t nbf, size_t P0, size_t Pc,
                            const KPlan& kp, const void* ct, void* mpl) {
-    const int S = bf_planes(prec);
-    if (S == 3) return bf_khalf_t<KbfTiles<3>::Half>(st, bpl, naux, nbf, P0, Pc, kp, ct, mpl);
-    const bool wide = kp.nbf_pad % KbfTiles<2>::Half::WGY == 0;
-    if (S == 1)
-        return wide ? bf_khalf_t<KbfTiles<1>::Half>(st, bpl, naux, nbf, P0, Pc, kp, ct, mpl)
-                    : bf_khalf_t<KbfTiles<1>::HalfNarrow>(st, bpl, naux, nbf, P0, Pc, kp, ct, mpl);
-    return wide ? bf_khalf_t<KbfTiles<2>::Half>(st, bpl, naux, nbf, P0, Pc, kp, ct, mpl)
-                : bf_khalf_t<KbfTiles<2>::HalfNarrow>(st, bpl, naux, nbf, P0, Pc, kp, ct, mpl);
+    switch (bf_planes(prec)) {
+        case 3: return bf_khalf_s<3>(st, bpl, naux, nbf, P0, Pc, kp, ct, mpl);
+        case 1: return bf_khalf_s<1>(st, bpl, naux, nbf, P0, Pc, kp, ct, mpl);
+        default: return bf_khalf_s<2>(st, bpl, naux, nbf, P0, Pc, kp, ct, mpl);
+    }
 }
 
-hipError_t launch_bf_ksyrk(hipStream_t st, int prec, const void* mpl, size_t Pc, const KPlan& kp, int nspin,
+hipError_t launch_bf_ksyrk(hipStream_t st, int prec, const void* mpl, size_t nbf, size_t Pc, const KPlan& kp, int nspin,
                            const void* smask, int beta, double* kpart) {
     switch (bf_planes(prec)) {
-        case 3: return bf_ksyrk_t<KbfTiles<3>::Syrk>(st, mpl, Pc, kp, nspin, smask, beta, kpart);
-        case 1: return bf_ksyrk_t<KbfTiles<1>::Syrk>(st, mpl, Pc, kp, nspin, smask, beta, kpart);
-        default: return bf_ksyrk_t<KbfTiles<2>::Syrk>(st, mpl, Pc, kp, nspin, smask, beta, kpart);
+        case 3: return bf_ksyrk_t<KbfTiles<3>::Syrk>(st, mpl, nbf, Pc, kp, nspin, smask, beta, kpart);
+        case 1: return bf_ksyrk_t<KbfTiles<1>::Syrk>(st, mpl, nbf, Pc, kp, nspin, smask, beta, kpart);
+        default: return bf_ksyrk_t<KbfTiles<2>::Syrk>(st, mpl, nbf, Pc, kp, nspin, smask, beta, kpart);
     }
 }
 
