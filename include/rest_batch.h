@@ -42,7 +42,7 @@ extern "C" {
 typedef struct rjk_batch rjk_batch;
 
 /* Stages timed by rjk_batch_profile: 0 D weights, 1 γ, 2 J accumulation, 3 C' preparation,
- * 4 / 5 K half-transform (narrow / wide tile class), 6 / 7 K SYRK (narrow or, at FP64/FP32,
+ * 4 / 5 K half-transform (narrow / wide tile class; BF16: up to / above 32 columns a tile), 6 / 7 K SYRK (narrow or, at FP64/FP32,
  * every problem / wide), 8 split reduction. */
 #define RJK_BATCH_NUM_STAGES 9
 

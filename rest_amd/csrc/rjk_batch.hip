@@ -19,9 +19,9 @@
 // sums every kFp32Chain products).
 //
 // BF16 precisions (RJK_PREC_BF16X1/X2/X3): B is kept once, packed in FP32, and
-// J runs on it as at FP32.  The K half-transform reads the packed FP32 B and
-// splits every element into S BF16 planes while staging it into LDS (no plane
-// copy of B is stored), then runs the split products of rjk_kbf.hip on the
+// J runs on it as at FP32.  The K half-transform reads the packed FP32 B into
+// matrix-core fragments and splits every element into S BF16 planes there (no
+// plane copy of B is stored), then runs the split products of rjk_kbf.hip on the
 // BF16 matrix cores; M' and the SYRK are those of rjk_kbf.hip per problem.  Both
 // stages keep the leading product (plane 0 × plane 0) and the correction
 // products in separate FP32 accumulators, added at the end, so the corrections'
@@ -309,188 +309,127 @@ __global__ __launch_bounds__(256) void k_b_bf_prep(const BProb* __restrict__ pr,
         __bf16 h[S];
         split_to<S>(v, h);
 #pragma unroll
-        for (int k = 0; k < S; ++k) glb((__bf16*)P.cocc)[k * plane + e] = h[k];
+        for (int k = 0; k < S; ++k) glb((__bf16*)P.cocc)[k * plane + bft::frag_elem(c, nu, P.nbf_pad)] = h[k];
         if (nu == 0) glb((unsigned short*)P.sign)[c] = w < 0 ? 0x8000 : 0;
     }
 }
 
-// Half-transform tile D[c][μ] = Σ_ν C'ᵀ[c][ν] B[μ][ν] of TN c × TM μ on 2 × 2 waves, k-blocks of TK
-// ν.  B comes from the packed FP32 column (element (i<=j) at j(j+1)/2 + i); each thread stages
-// runs of 8 consecutive ν of one μ: along ν (contiguous in memory) when the tile lies wholly below
-// the diagonal, else one μ per lane (contiguous across lanes above the diagonal).  LDS rows are TK
-// BF16 values, 16-byte piece p of row r at p ^ sw(r) (the swizzle of rjk_bftile.hpp).
-template <int S, int TM, int TK, int TN = 64>
-struct BfHalf {
-    static constexpr int NT = 256, WX = 2, WY = 2, WGX = TN, WGY = TM, NPC = TK / 8;
-    static constexpr int FX = WGX / WX / 16, FY = WGY / WY / 16;
-    static constexpr int LX = WGX * NPC / NT, LY = WGY * NPC / NT;
-    static constexpr int LDS_ELEMS = S * (WGX + WGY) * TK;
-    static constexpr int S_ = S, TK_ = TK;
-    static_assert(LX >= 1 && LY >= 1 && LX * NT == WGX * NPC && LY * NT == WGY * NPC, "load shape");
-    __device__ static constexpr int sw(int r) { return NPC == 4 ? ((r >> 1) & 3) : ((r >> 1) & 7); }
-};
+__device__ inline int rup32(int n) { return (n + 31) / 32 * 32; }
 
 typedef float F4a __attribute__((ext_vector_type(4), aligned(4)));   // 4 floats at 4-byte alignment
 
-template <class H>
-__device__ __forceinline__ void bf_half_tile(__bf16* __restrict__ lds, const RJK_GLB float* __restrict__ bcol, int nbf,
-                                             int mu0, int c0, const RJK_GLB __bf16* __restrict__ ct, size_t pct,
-                                             int nbf_pad, int nk, RJK_GLB __bf16* __restrict__ mP, size_t pm) {
-    using namespace bft;
-    constexpr int S = H::S_, NP = npairs<S>(), TK = H::TK_, NPC = H::NPC;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wx = wave % H::WX, wy = wave / H::WX, l16 = lane & 15;
-    auto at = [](int r, int p) { return r * TK + ((p ^ H::sw(r)) << 3); };
-    auto Xs = [&](int k) { return lds + (size_t)k * (H::WGX + H::WGY) * TK; };
-    auto Ys = [&](int k) { return lds + ((size_t)k * (H::WGX + H::WGY) + H::WGX) * TK; };
-    f4 acc[H::FX][H::FY], acc2[H::FX][H::FY];   // leading product; corrections (added at the end)
-#pragma unroll
-    for (int i = 0; i < H::FX; ++i)
-#pragma unroll
-        for (int j = 0; j < H::FY; ++j) {
-            acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-            acc2[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-        }
-    u4 rx[S][H::LX];
-    float rb[H::LY][8];
-    bool below = false;
-    auto task_rp = [&](int j, int* r, int* p) {   // row (μ offset) and piece of B task j
-        const int e = tid + j * H::NT;
-        if (below) {
-            *r = e / NPC;
-            *p = e % NPC;
-        } else {
-            *r = e % H::WGY;
-            *p = e / H::WGY;
-        }
+// Fragments of B_P for rjk_bftile.hpp's half-transform, from the packed FP32 column (element (i <= j) at
+// j(j+1)/2 + i) straight into the lane that needs them; split into planes as the MFMAs take them.
+// Left of the diagonal a lane's 8 ν are consecutive (two 16-byte loads at 4-byte alignment), beyond it
+// 16 lanes' μ are (a load a ν); across it and at the edges every element finds its place.
+template <int S, int FM>
+struct PackedRows {
+    struct Raw {
+        float v[8];
+        unsigned ok;   // edge fragments: which of the 8 lie inside nbf
+        bool edge;
     };
-    auto fetch = [&](int nu0) {
+    const RJK_GLB float* col;
+    int nbf, mu0;
+    __device__ __forceinline__ void load(int s, Raw (&r)[FM]) const {
+        const int lane = threadIdx.x & 63, nu0 = s * bft::KM;
 #pragma unroll
-        for (int k = 0; k < S; ++k)
-#pragma unroll
-            for (int j = 0; j < H::LX; ++j) {
-                const int e = tid + j * H::NT;
-                rx[k][j] = ld16(ct + k * pct + (size_t)(c0 + e / NPC) * nbf_pad + nu0 + (e % NPC) * 8);
-            }
-        below = mu0 >= nu0 + TK - 1;
-#pragma unroll
-        for (int j = 0; j < H::LY; ++j) {
-            int r, p;
-            task_rp(j, &r, &p);
-            const int mu = mu0 + r, nub = nu0 + p * 8;
-            if (below) {
-                // 8 consecutive ν of row μ: two 16-byte loads at the row's 4-byte alignment
-                const size_t base = mu < nbf ? tri((size_t)mu) + nub : 0;
-                const RJK_GLB F4a* src = (const RJK_GLB F4a*)(bcol + base);
+        for (int j = 0; j < FM; ++j) {
+            const int m0 = mu0 + j * 16, mu = m0 + (lane & 15), nu = nu0 + (lane >> 4) * 8;
+            const bool in = m0 + 15 < nbf && nu0 + 31 < nbf;
+            r[j].edge = false;
+            if (in && nu0 + 31 <= m0) {
+                const RJK_GLB F4a* src = (const RJK_GLB F4a*)(col + tri((size_t)mu) + nu);
                 const F4a lo = src[0], hi = src[1];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    rb[j][i] = mu < nbf ? lo[i] : 0.f;
-                    rb[j][4 + i] = mu < nbf ? hi[i] : 0.f;
+                    r[j].v[i] = lo[i];
+                    r[j].v[4 + i] = hi[i];
                 }
-            } else {
+            } else if (in && nu0 >= m0 + 15) {
+                unsigned off = (unsigned)(nu * (nu + 1) / 2 + mu);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
-                    const int nu = nub + i;
-                    const bool ok = mu < nbf && nu < nbf;
-                    const int lo = mu < nu ? mu : nu, hi = mu < nu ? nu : mu;
-                    const float v = bcol[ok ? tri((size_t)hi) + lo : 0];
-                    rb[j][i] = ok ? v : 0.f;
+                    r[j].v[i] = col[off];
+                    off += (unsigned)(nu + i + 1);
+                }
+            } else {
+                r[j].edge = true;
+                r[j].ok = 0;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int lo = min(mu, nu + i), hi = max(mu, nu + i);
+                    r[j].ok |= (unsigned)(hi < nbf) << i;
+                    r[j].v[i] = col[hi < nbf ? (unsigned)(hi * (hi + 1) / 2 + lo) : 0u];
                 }
             }
         }
-    };
-    auto stash = [&]() {
-#pragma unroll
-        for (int k = 0; k < S; ++k)
-#pragma unroll
-            for (int j = 0; j < H::LX; ++j) {
-                const int e = tid + j * H::NT;
-                *(u4*)(Xs(k) + at(e / NPC, e % NPC)) = rx[k][j];
-            }
-#pragma unroll
-        for (int j = 0; j < H::LY; ++j) {
-            int r, p;
-            task_rp(j, &r, &p);
-            bf8 v[S];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                __bf16 h[S];
-                split_f<S>(rb[j][i], h);
-#pragma unroll
-                for (int k = 0; k < S; ++k) v[k][i] = h[k];
-            }
-#pragma unroll
-            for (int k = 0; k < S; ++k) *(bf8*)(Ys(k) + at(r, p)) = v[k];
-        }
-    };
-    auto compute = [&]() {
-#pragma unroll
-        for (int ks = 0; ks < TK / KM; ++ks) {
-            const int pr = ks * 4 + (lane >> 4);
-            bf8 fx[H::FX][S], fy[H::FY][S];
-#pragma unroll
-            for (int k = 0; k < S; ++k) {
-#pragma unroll
-                for (int i = 0; i < H::FX; ++i) fx[i][k] = *(const bf8*)(Xs(k) + at((wx * H::FX + i) * 16 + l16, pr));
-#pragma unroll
-                for (int j = 0; j < H::FY; ++j) fy[j][k] = *(const bf8*)(Ys(k) + at((wy * H::FY + j) * 16 + l16, pr));
-            }
-#pragma unroll
-            for (int p = 0; p < NP; ++p)
-#pragma unroll
-                for (int i = 0; i < H::FX; ++i)
-#pragma unroll
-                    for (int j = 0; j < H::FY; ++j) {
-                        if (p > 0)
-                            acc2[i][j] = mfma(fx[i][pa<S>(p)], fy[j][pb<S>(p)], acc2[i][j]);
-                        else
-                            acc[i][j] = mfma(fx[i][pa<S>(p)], fy[j][pb<S>(p)], acc[i][j]);
-                    }
-        }
-    };
-    const int nq = (nbf + TK - 1) / TK;
-    fetch(0);
-    for (int q = 0; q < nq; ++q) {
-        stash();
-        __syncthreads();
-        if (q + 1 < nq) fetch((q + 1) * TK);
-        __builtin_amdgcn_s_setprio(1);   // MFMA phase first (batch of 512 clusters: 874 -> 853 ms at BF16X3)
-        compute();
-        __builtin_amdgcn_s_setprio(0);
-        __syncthreads();
     }
+    __device__ __forceinline__ void frag(const Raw& r, bft::bf8 (&f)[S]) const {
+        float v[8];
 #pragma unroll
-    for (int i = 0; i < H::FX; ++i)
+        for (int i = 0; i < 8; ++i) v[i] = r.v[i];
+        if (r.edge) {
 #pragma unroll
-        for (int j = 0; j < H::FY; ++j)
-            store_m<S>(mP, pm, mu0 + (wy * H::FY + j) * 16, c0 + (wx * H::FX + i) * 16, nk, lane, acc[i][j] + acc2[i][j]);
-}
+            for (int i = 0; i < 8; ++i) v[i] = r.ok >> i & 1 ? v[i] : 0.f;
+        }
+        bft::u4 p[S];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            unsigned w[S];
+            bft::split_pair<S>(v[2 * i], v[2 * i + 1], w);
+#pragma unroll
+            for (int k = 0; k < S; ++k) p[k][i] = w[k];
+        }
+#pragma unroll
+        for (int k = 0; k < S; ++k) f[k] = __builtin_bit_cast(bft::bf8, p[k]);
+    }
+};
 
-// half-transform over the problems of one tile class: round_up(naux, 8) · ntm · ntc items per problem
-template <class H>
-__global__ __launch_bounds__(256) void k_b_bf_khalf(const BProb* __restrict__ pr, const int* __restrict__ sub,
-                                                    const size_t* __restrict__ off, int nsub) {
+constexpr int kHalfRows = 32;     // μ rows of a wave in the BF16 half-transform
+constexpr int kHalfWaves = 4;
+
+// Half-transform over the problems whose columns take tiles of 16·FX.  A wave's unit is 32 rows μ of one
+// auxiliary column; a work-group's four waves take consecutive units, of one column or of two, since all
+// they share is C'ᵀ.  XCD x holds the columns P % 8 == x.  24 clusters of 48 to 384 functions (2.4 TFLOP with
+// three planes): 7.16 ms through LDS tiles of 64 or 128 rows and 64-column granules, 3.71 now (650 TFLOP/s),
+// bound by its own waits: 218 registers leave two waves a SIMD.  16 rows a wave 4.08 ms, eight waves 3.78,
+// three waves a SIMD (spilling) 6.3.
+template <int S, int FX>
+__global__ __launch_bounds__(kHalfWaves * 64, 2) void k_b_bf_khalf(const BProb* __restrict__ pr,
+                                                                   const int* __restrict__ sub,
+                                                                   const size_t* __restrict__ off, int nsub) {
+    using H = bft::HalfCfg<S, FX, kHalfRows / 16, kHalfWaves>;
     __shared__ __bf16 lds[H::LDS_ELEMS];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const size_t total = off[nsub];
     for (size_t it = blockIdx.x; it < total; it += gridDim.x) {
         const int j = find_prob(off, nsub, it);
         const BProb& P = pr[sub[j]];
         if (!P.active) continue;
-        const size_t local = it - off[j];
-        const int ntm = P.nbf_pad / H::WGY, ntc = P.nk / H::WGX, per = ntm * ntc;
-        const size_t xcd = local % kXcd, kq = local / kXcd;
-        const int Pl = (int)((kq / per) * kXcd + xcd);
-        if (Pl >= P.naux) continue;   // padding items (uniform per work-group)
-        const int rem = (int)(kq % per), mt = rem / ntc, ctile = rem % ntc;
-        const size_t pm = (size_t)P.naux * P.nbf_pad * P.nk;
-        bf_half_tile<H>(lds, glb((const float*)P.b) + (size_t)Pl * P.ldb, P.nbf, mt * H::WGY, ctile * H::WGX,
-                        glb((const __bf16*)P.cocc), (size_t)P.nk * P.nbf_pad, P.nbf_pad, P.nk,
-                        glb((__bf16*)P.m) + (size_t)Pl * P.nbf_pad * P.nk, pm);
+        const unsigned local = (unsigned)(it - off[j]), xcd = local % kXcd, kq = local / kXcd;
+        const unsigned nrb = (P.nbf + kHalfRows - 1) / kHalfRows, ntc = (rup32(P.nocc) + H::TC - 1) / H::TC;
+        const unsigned unit = kq / ntc * kHalfWaves + wave;
+        const int c0 = (int)(kq % ntc) * H::TC, Pl = (int)(unit / nrb * kXcd + xcd), mu0 = (int)(unit % nrb) * kHalfRows;
+        const bool live = Pl < P.naux;
+        const PackedRows<S, H::FM> y{glb((const float*)P.b) + (size_t)(live ? Pl : 0) * P.ldb, P.nbf, mu0};
+        bft::f4 acc[FX][H::FM], acc2[FX][H::FM];   // leading product; corrections (added at the end)
+        bft::half_tile<H, true>(lds, glb((const __bf16*)P.cocc), P.nk, P.nbf_pad / bft::KM, c0,
+                                (P.nbf + bft::KM - 1) / bft::KM, live, y, acc, acc2);
+        if (live) {
+            const size_t pm = (size_t)P.naux * P.nbf_pad * P.nk;
+            const auto mP = glb((__bf16*)P.m) + (size_t)Pl * P.nbf_pad * P.nk;
+#pragma unroll
+            for (int i = 0; i < FX; ++i) {
+                if (c0 + i * 16 >= P.nk) break;
+#pragma unroll
+                for (int jj = 0; jj < H::FM; ++jj)
+                    bft::store_m<S>(mP, pm, mu0 + jj * 16, c0 + i * 16, P.nk, lane, acc[i][jj] + acc2[i][jj]);
+            }
+        }
+        __syncthreads();   // the next item's C'ᵀ overwrites the LDS buffers
     }
 }
-
-__device__ inline int rup32(int n) { return (n + 31) / 32 * 32; }
 
 // SYRK over the problems of one tile class: nsplit · ntile2 items per problem (split s on XCD s % 8),
 // Kpart[split][ν][μ] = Σ_{P in split, c} sign_c M'_P[ν][c] M'_P[μ][c] on upper tile pairs
@@ -608,12 +547,16 @@ size_t prob_bytes(const BProb& P, int prec) {
 
 bool valid_prec(int prec) { return prec == RJK_PREC_FP64 || prec == RJK_PREC_FP32 || is_bf(prec); }
 
-// Half-transform groups: (μ rows, c columns) of the tile.  BF16 uses all five (one c tile covers
-// every occupied column up to 192 at 64 rows, 128 at 128 rows, so each B element is staged once);
-// FP64/FP32 use 0 and 3 (rjk_ktiles.hpp's 64 × 64 and 128 × 64 tiles).
-constexpr int kHalfGroups = 5;
-constexpr int kGroupTM[kHalfGroups] = {64, 64, 64, 128, 128};
-constexpr int kGroupTN[kHalfGroups] = {64, 128, 192, 64, 128};
+// Half-transform groups, a launch each.  BF16: column tiles of 2, 4 or 6 fragments, one tile for up to 96
+// occupied columns (each B element is then read and split once).  FP64/FP32: 64 × 64 and 128 × 64 tiles of
+// rjk_ktiles.hpp (0 and 1).
+constexpr int kHalfGroups = 3;
+
+// 16-column fragments of a BF16 problem's column tiles: as few tiles of at most 6 as hold them, of one width
+size_t half_frags(size_t nocc) {
+    const size_t f = (nocc + 31) / 32, tiles = (f + 2) / 3;   // in pairs: the SYRK takes 32 columns at a time
+    return (f + tiles - 1) / tiles * 2;
+}
 
 bool valid_shape(size_t nbf, size_t naux, size_t nocc) {
     return nbf != 0 && naux != 0 && nocc != 0 && nocc <= nbf && nbf <= 32768 && naux <= (1u << 24);
@@ -684,17 +627,21 @@ Tables tables(const rjk_batch* b) {
 }
 
 // Tile class of a problem under the current cut: 0 = narrow (FP: 64 × 64 half-transform tiles;
-// BF16: 64-wide half-transform and SYRK tiles), 1 = wide (128); BF16 needs nbf_pad % 128 == 0 for 1.
+// BF16: 64-wide SYRK tiles), 1 = wide (128); BF16 needs nbf_pad % 128 == 0 for 1.
 int tile_class(const rjk_batch* b, const BProb& P) {
     if (P.nbf_pad < b->khalf_cut) return 0;
     return (is_bf(b->prec) && P.nbf_pad % 128) ? 0 : 1;
 }
 
 int half_group(const rjk_batch* b, const BProb& P) {
-    const int v = tile_class(b, P);
-    if (!is_bf(b->prec)) return v == 0 ? 0 : 3;
-    if (v == 0) return P.nk == 128 ? 1 : (P.nk == 192 ? 2 : 0);
-    return P.nk == 128 ? 4 : 3;
+    return is_bf(b->prec) ? (int)half_frags(P.nocc) / 2 - 1 : tile_class(b, P);
+}
+
+// work items of a problem's half-transform
+size_t half_items(const rjk_batch* b, const BProb& P) {
+    if (!is_bf(b->prec)) return rup(P.naux, 8) * (size_t)(P.nbf_pad / (tile_class(b, P) ? 128 : 64)) * (P.nk / 64);
+    const size_t units = rup(P.naux, 8) / 8 * ((P.nbf + kHalfRows - 1) / kHalfRows), tc = 16 * half_frags(P.nocc);
+    return 8 * ((units + kHalfWaves - 1) / kHalfWaves) * ((rup(P.nocc, 32) + tc - 1) / tc);
 }
 
 int build_subsets(rjk_batch* b) {
@@ -706,9 +653,9 @@ int build_subsets(rjk_batch* b) {
     for (int v = 0; v < 2; ++v) soff[v].push_back(0);
     for (int q = 0; q < np; ++q) {
         const BProb& P = b->h[q];
-        const int g = half_group(b, P), TM = kGroupTM[g], TN = kGroupTN[g];
+        const int g = half_group(b, P);
         sub[g].push_back(q);
-        off[g].push_back(off[g].back() + rup(P.naux, 8) * (size_t)(P.nbf_pad / TM) * (P.nk / TN));
+        off[g].push_back(off[g].back() + half_items(b, P));
         if (bf) {
             const int v = tile_class(b, P);
             const size_t nt = (size_t)P.nbf_pad / (v == 0 ? 64 : 128);
@@ -770,9 +717,9 @@ int enqueue_fp(rjk_batch* b, hipEvent_t* ev) {
         hipLaunchKernelGGL((k_b_khalf<T, 1, 4>), dim3(grid_items(b, b->t_sub_items[0], b->waves)), dim3(kBlock), 0,
                            st, b->d_prob, b->d_sub, b->d_suboff, b->t_sub_n[0]);
     mark(5);
-    if (b->t_sub_items[3])
-        hipLaunchKernelGGL((k_b_khalf<T, 2, 4>), dim3(grid_items(b, b->t_sub_items[3], b->waves)), dim3(kBlock), 0,
-                           st, b->d_prob, b->d_sub + 3 * np, b->d_suboff + 3 * (np + 1), b->t_sub_n[3]);
+    if (b->t_sub_items[1])
+        hipLaunchKernelGGL((k_b_khalf<T, 2, 4>), dim3(grid_items(b, b->t_sub_items[1], b->waves)), dim3(kBlock), 0,
+                           st, b->d_prob, b->d_sub + np, b->d_suboff + (np + 1), b->t_sub_n[1]);
     mark(6);
     hipLaunchKernelGGL((k_b_ksyrk<T, 4>), dim3(grid_items(b, b->t_syrk.back(), b->waves)), dim3(kBlock), 0, st,
                        b->d_prob, np, tb);
@@ -787,11 +734,6 @@ int enqueue_fp(rjk_batch* b, hipEvent_t* ev) {
 template <int S>
 int enqueue_bf(rjk_batch* b, hipEvent_t* ev) {
     constexpr int TK = S == 3 ? 32 : 64;
-    using H0 = BfHalf<S, 64, TK, 64>;
-    using H1 = BfHalf<S, 64, TK, 128>;
-    using H2 = BfHalf<S, 64, TK, 192>;
-    using H3 = BfHalf<S, 128, TK, 64>;
-    using H4 = BfHalf<S, 128, TK, 128>;
     using Y0 = bft::Cfg<S, 64, 64, 2, 2, TK>;
     using Y1 = bft::Cfg<S, 128, 128, 2, 4, TK>;
     const int np = (int)b->h.size();
@@ -813,15 +755,13 @@ int enqueue_bf(rjk_batch* b, hipEvent_t* ev) {
     mark(4);
     auto half = [&](auto kern, int g) {
         if (b->t_sub_items[g])
-            hipLaunchKernelGGL(kern, dim3(grid_items(b, b->t_sub_items[g], b->waves)), dim3(256), 0, st, b->d_prob,
-                               b->d_sub + g * np, b->d_suboff + g * (np + 1), b->t_sub_n[g]);
+            hipLaunchKernelGGL(kern, dim3(grid_items(b, b->t_sub_items[g], b->waves)), dim3(kHalfWaves * 64), 0, st,
+                               b->d_prob, b->d_sub + g * np, b->d_suboff + g * (np + 1), b->t_sub_n[g]);
     };
-    half(k_b_bf_khalf<H0>, 0);
-    half(k_b_bf_khalf<H1>, 1);
-    half(k_b_bf_khalf<H2>, 2);
+    half(k_b_bf_khalf<S, 2>, 0);
     mark(5);
-    half(k_b_bf_khalf<H3>, 3);
-    half(k_b_bf_khalf<H4>, 4);
+    half(k_b_bf_khalf<S, 4>, 1);
+    half(k_b_bf_khalf<S, 6>, 2);
     mark(6);
     if (b->t_syrk_items[0])
         hipLaunchKernelGGL(k_b_bf_ksyrk<Y0>, dim3(grid_items(b, b->t_syrk_items[0], b->waves)), dim3(Y0::NT), 0, st,

@@ -17,8 +17,9 @@ namespace rjk {
 namespace bft {
 
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
 constexpr int KM = 32;        // one MFMA deep
@@ -69,8 +70,8 @@ __device__ __host__ inline size_t frag_elem(size_t row, size_t col, size_t ncol)
 __device__ const u4* pm_vec(const unsigned short*);   // the vector pointer of a mask pointer's address space
 __device__ const __attribute__((address_space(1))) u4* pm_vec(const __attribute__((address_space(1))) unsigned short*);
 
-__device__ bf4* bf4_ptr(__bf16*);
-__device__ __attribute__((address_space(1))) bf4* bf4_ptr(__attribute__((address_space(1))) __bf16*);
+__device__ u2* u2_ptr(__bf16*);
+__device__ __attribute__((address_space(1))) u2* u2_ptr(__attribute__((address_space(1))) __bf16*);
 
 // SYRK tile: D[ν][μ] over the np auxiliary columns of a split and ncol columns of M' each.
 // Their fragment columns ("runs" of 32) follow each other and TK/32 make a k-block, so neither a
@@ -205,26 +206,29 @@ __device__ __forceinline__ void nt_tile(__bf16* __restrict__ lds, PX x, PX y, si
     nt_tile2<C, false>(lds, x, y, rowst, pl, ps, mask, np, ncol, live, acc, acc);
 }
 
+// Planes of two values, packed (a in the low half).  One conversion instruction a plane; the empty asm keeps
+// the compiler from joining the pairs into a wider vector conversion, which it can place in the
+// registers of its own sources and order so that it overwrites them before they are read (clang of ROCm 7.2).
 template <int S>
-__device__ inline void split_f(float x, __bf16* out) {
-    float r = x;
+__device__ __forceinline__ void split_pair(float a, float b, unsigned (&w)[S]) {
 #pragma unroll
     for (int k = 0; k < S; ++k) {
-        const __bf16 h = (__bf16)r;
-        out[k] = h;
-        r -= (float)h;
+        w[k] = __builtin_bit_cast(unsigned, bf2{(__bf16)a, (__bf16)b});
+        asm("" : "+v"(w[k]));
+        a -= __builtin_bit_cast(float, w[k] << 16);
+        b -= __builtin_bit_cast(float, w[k] & 0xffff0000u);
     }
 }
 
 // one accumulator fragment into the M' planes: lane holds columns c0 + 4(l/16) + r of row mu0 + l%16
 template <int S, class P>
 __device__ __forceinline__ void store_m(P m, size_t plane, int mu0, int c0, int nk, int lane, f4 a) {
-    __bf16 h[4][S];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) split_f<S>(a[r], h[r]);
+    unsigned lo[S], hi[S];
+    split_pair<S>(a[0], a[1], lo);
+    split_pair<S>(a[2], a[3], hi);
     const size_t e = frag_elem(mu0, c0, nk) + (lane >> 5) * 128 + (lane & 15) * 8 + (lane >> 4 & 1) * 4;
 #pragma unroll
-    for (int k = 0; k < S; ++k) *(decltype(bf4_ptr(m)))(m + k * plane + e) = bf4{h[0][k], h[1][k], h[2][k], h[3][k]};
+    for (int k = 0; k < S; ++k) *(decltype(u2_ptr(m)))(m + k * plane + e) = u2{lo[k], hi[k]};
 }
 
 // ---------------------------------------------------------------------------

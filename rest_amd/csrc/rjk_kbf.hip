@@ -29,8 +29,6 @@
 namespace rjk {
 namespace {
 
-typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
-
 constexpr int kXcdB = 8;
 
 __device__ inline size_t tri_b(size_t j) { return j * (j + 1) / 2; }
@@ -69,17 +67,22 @@ __global__ void k_bf_planes_b(const double* __restrict__ b64, size_t ldb, int nb
             tile[wave][r][c] = hi < nbf ? col[tri_b(hi) + lo] : 0.0;
         }
         __syncthreads();
-        bft::bf8 v[S];
+        bft::u4 v[S];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            __bf16 h[S];
-            split_d<S>(tile[wave][lane & 15][(lane >> 4) * 8 + i], h);
+        for (int i = 0; i < 4; ++i) {
+            double a = tile[wave][lane & 15][(lane >> 4) * 8 + 2 * i], b = tile[wave][lane & 15][(lane >> 4) * 8 + 2 * i + 1];
 #pragma unroll
-            for (int k = 0; k < S; ++k) v[k][i] = h[k];
+            for (int k = 0; k < S; ++k) {   // as bft::split_pair, with the remainders in FP64
+                unsigned w = __builtin_bit_cast(unsigned, bft::bf2{(__bf16)(float)a, (__bf16)(float)b});
+                asm("" : "+v"(w));
+                v[k][i] = w;
+                a -= (double)__builtin_bit_cast(float, w << 16);
+                b -= (double)__builtin_bit_cast(float, w & 0xffff0000u);
+            }
         }
 #pragma unroll
         for (int k = 0; k < S; ++k)
-            *(bft::bf8*)(planes + ((size_t)k * naux + P0 + P) * sq + (size_t)f * bft::FRAG + lane * 8) = v[k];
+            *(bft::u4*)(planes + ((size_t)k * naux + P0 + P) * sq + (size_t)f * bft::FRAG + lane * 8) = v[k];
         __syncthreads();
     }
 }
