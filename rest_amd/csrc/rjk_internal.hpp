@@ -187,6 +187,18 @@ hipError_t launch_asym_stats(hipStream_t st, const double* dm, size_t nbf, doubl
 constexpr size_t kCholMaxRank = 1024;
 hipError_t launch_pivot_chol(hipStream_t st, const double* dm, size_t nbf, size_t kmax, double cut, double* diag, double* L,
                              int* rank, double* blockmax, double* residual);
+// Eigenpairs of a symmetric A (upper triangle, column-major) of at most kEigMax functions (rjk_eig.hip):
+// eigenvalues w ascending, vectors the columns of Z.  ws: eig_ws(n) doubles, which start with T's diagonal [n]
+// and off-diagonal [n].  *bad: the pairs are not good enough; eigenvectors of T in Z then become A's by
+// launch_eig_back.
+constexpr size_t kEigMax = 192;
+// The SCF's smaller problems, free atoms among them, stay with dsyevd: an atom's shells are exactly
+// degenerate, so these kernels would hand most of them on, and which way an open shell points, hence the
+// guess made of it, is whichever vectors the solver gives.
+constexpr size_t kEigMin = 40;
+size_t eig_ws(size_t n);
+hipError_t launch_eig(hipStream_t st, const double* A, size_t n, double* w, double* Z, double* ws, int* bad);
+hipError_t launch_eig_back(hipStream_t st, double* Z, size_t n, const double* ws);
 hipError_t launch_prep_general(hipStream_t st, const double* dm, size_t nbf, size_t nk, size_t nrow, double* cx,
                                double* cy);
 hipError_t launch_pack_upper(hipStream_t st, const double* g, size_t nbf, size_t ldg, double scale, double* vk);

@@ -2,7 +2,7 @@
 //
 // One J/K build per iteration through the context's resident B; Fock,
 // energy, DIIS and the density in HBM (FP64, rocBLAS GEMMs and small
-// kernels); F C = S C ε through X = S^{-1/2} and rocSOLVER dsyevd.  Mirrors REST's scf()
+// kernels); F C = S C ε through X = S^{-1/2} and rjk_eig.hip or rocSOLVER.  Mirrors REST's scf()
 // (src/scf_io/mod.rs:3190-3268) with prepare_next_input (:2947-3091),
 // generate_diis_error_vector (:3094-3136), diis_solver (:3138-3188) and
 // check_scf_convergence (:1875-1951).
@@ -432,6 +432,7 @@ int scf_core(rjk_ctx* ctx, const char* who, const double* S_h, const double* H_h
     double* T2 = mem.get(ctx, n2, &rc);
     double* Dt = mem.get(ctx, n2, &rc);     // total density for J (UHF)
     double* Ework = mem.get(ctx, n, &rc);
+    double* eigws = n > rjk::kEigMin && n <= rjk::kEigMax ? mem.get(ctx, rjk::eig_ws(n), &rc) : nullptr;
     double* vj = mem.get(ctx, npair, &rc);
     double* partial = mem.get(ctx, kRedBlocks, &rc);
     double* info_d = mem.get(ctx, 1, &rc);
@@ -531,8 +532,27 @@ int scf_core(rjk_ctx* ctx, const char* who, const double* S_h, const double* H_h
         eps[s].assign(n, 0.0);
         eps_prev[s].assign(n, 0.0);
     }
+    // Eigenpairs of M (kEigMin < n <= kEigMax: the kernels of rjk_eig.hip, vectors in T1, info_d non-zero where eigenvalues are
+    // too close for them; else rocSOLVER, vectors in place), and then again by divide and conquer on
+    // the same tridiagonal matrix.  dsyevd at n 192: 3863 us, here 702 (1880 with divide and conquer).
+    auto eigen = [&](double* M, double* w, double** vec) -> int {
+        *vec = eigws ? T1 : M;
+        if (eigws) SCF_HIP(rjk::launch_eig(st, M, n, w, T1, eigws, (int*)info_d));
+        else
+            SCF_BLAS(rocsolver_dsyevd(h, rocblas_evect_original, rocblas_fill_upper, (rocblas_int)n, M, (rocblas_int)n, w,
+                                      Ework, (rocblas_int*)info_d));
+        return RJK_OK;
+    };
+    auto eigen_again = [&](double* w, double* vec) -> int {
+        SCF_HIP(hipMemcpyAsync(w, eigws, n * sizeof(double), hipMemcpyDeviceToDevice, st));
+        SCF_HIP(hipMemcpyAsync(Ework, eigws + n, n * sizeof(double), hipMemcpyDeviceToDevice, st));
+        SCF_BLAS(rocsolver_dstedc(h, rocblas_evect_tridiagonal, (rocblas_int)n, w, Ework, vec, (rocblas_int)n,
+                                  (rocblas_int*)info_d));
+        SCF_HIP(rjk::launch_eig_back(st, vec, n, eigws));
+        return RJK_OK;
+    };
     // Orthogonaliser X = S^{-1/2} = U s^{-1/2} Uᵀ, once: every F C = S C ε then becomes
-    // F' = X F X (two GEMMs), F' C' = C' ε (rocSOLVER dsyevd), C = X C' (one GEMM).
+    // F' = X F X (two GEMMs), F' C' = C' ε, C = X C' (one GEMM).
     // Same eigenpairs as REST's generalised solver (dspgvx, src/scf_io/mod.rs:1851),
     // without re-factorising S in every iteration.
     // X cached on the context for the same S (the guess step and the SCF of one molecule share it)
@@ -548,22 +568,28 @@ int scf_core(rjk_ctx* ctx, const char* who, const double* S_h, const double* H_h
     }
     if (ctx->scf_s.empty()) {
         SCF_HIP(hipMemcpyAsync(Bw, S, n2 * sizeof(double), hipMemcpyDeviceToDevice, st));
-        SCF_BLAS(rocsolver_dsyevd(h, rocblas_evect_original, rocblas_fill_upper, (rocblas_int)n, Bw, (rocblas_int)n,
-                                  W[0], Ework, (rocblas_int*)info_d));
+        double* U = nullptr;
         int info = 0;
         std::vector<double> sv(n);
+        SCF_RC(eigen(Bw, W[0], &U));
         SCF_HIP(hipMemcpyAsync(&info, info_d, sizeof(int), hipMemcpyDeviceToHost, st));
         SCF_HIP(hipMemcpyAsync(sv.data(), W[0], n * sizeof(double), hipMemcpyDeviceToHost, st));
         SCF_HIP(hipStreamSynchronize(st));
+        if (info != 0 && eigws) {
+            SCF_RC(eigen_again(W[0], U));
+            SCF_HIP(hipMemcpyAsync(&info, info_d, sizeof(int), hipMemcpyDeviceToHost, st));
+            SCF_HIP(hipMemcpyAsync(sv.data(), W[0], n * sizeof(double), hipMemcpyDeviceToHost, st));
+            SCF_HIP(hipStreamSynchronize(st));
+        }
         if (info != 0) return rjk::fail(ctx, RJK_ERR_NOSOLVER, "rocsolver_dsyevd(S) info = " + std::to_string(info));
         if (!(sv[0] > 0.0))
             return rjk::fail(ctx, RJK_ERR_ARG, std::string(who) + ": the overlap matrix is not positive definite");
         for (double& v : sv) v = 1.0 / std::sqrt(v);
         SCF_HIP(hipMemcpyAsync(W[0], sv.data(), n * sizeof(double), hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(k_scale_columns, g2, b256, 0, st, Bw, W[0], n, T1);   // T1 = U s^{-1/2}
+        hipLaunchKernelGGL(k_scale_columns, g2, b256, 0, st, U, W[0], n, T2);   // T2 = U s^{-1/2}
         SCF_HIP(hipGetLastError());
         SCF_BLAS(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_transpose, (rocblas_int)n, (rocblas_int)n,
-                               (rocblas_int)n, &one, T1, (rocblas_int)n, Bw, (rocblas_int)n, &zero, X,
+                               (rocblas_int)n, &one, T2, (rocblas_int)n, U, (rocblas_int)n, &zero, X,
                                (rocblas_int)n));
         SCF_HIP(hipStreamSynchronize(st));   // sv is a host temporary
         ctx->scf_s.assign(S_h, S_h + n2);
@@ -578,16 +604,20 @@ int scf_core(rjk_ctx* ctx, const char* who, const double* S_h, const double* H_h
         SCF_BLAS(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, (rocblas_int)n, (rocblas_int)n,
                                (rocblas_int)n, &one, X, (rocblas_int)n, T1, (rocblas_int)n, &zero, Bw,
                                (rocblas_int)n));
-        SCF_BLAS(rocsolver_dsyevd(h, rocblas_evect_original, rocblas_fill_upper, (rocblas_int)n, Bw, (rocblas_int)n,
-                                  W[s], Ework, (rocblas_int*)info_d));
-        SCF_BLAS(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, (rocblas_int)n, (rocblas_int)n,
-                               (rocblas_int)n, &one, X, (rocblas_int)n, Bw, (rocblas_int)n, &zero, A[s],
-                               (rocblas_int)n));
+        double* U = nullptr;
         int info = 0;
-        SCF_HIP(hipMemcpyAsync(&info, info_d, sizeof(int), hipMemcpyDeviceToHost, st));
-        SCF_HIP(hipMemcpyAsync(eps[s].data(), W[s], n * sizeof(double), hipMemcpyDeviceToHost, st));
-        SCF_HIP(hipStreamSynchronize(st));
-        if (info != 0) return rjk::fail(ctx, RJK_ERR_NOSOLVER, "rocsolver_dsyevd info = " + std::to_string(info));
+        for (bool again = false;; again = true) {
+            if (again) SCF_RC(eigen_again(W[s], U));
+            else SCF_RC(eigen(Bw, W[s], &U));
+            SCF_BLAS(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, (rocblas_int)n, (rocblas_int)n,
+                                   (rocblas_int)n, &one, X, (rocblas_int)n, U, (rocblas_int)n, &zero, A[s],
+                                   (rocblas_int)n));
+            SCF_HIP(hipMemcpyAsync(&info, info_d, sizeof(int), hipMemcpyDeviceToHost, st));
+            SCF_HIP(hipMemcpyAsync(eps[s].data(), W[s], n * sizeof(double), hipMemcpyDeviceToHost, st));
+            SCF_HIP(hipStreamSynchronize(st));
+            if (info == 0 || again || !eigws) break;
+        }
+        if (info != 0) return rjk::fail(ctx, RJK_ERR_NOSOLVER, "eigensolver info = " + std::to_string(info));
         t_diag += now() - t0;
         return RJK_OK;
     };
