@@ -3,13 +3,13 @@
 //   2. eigenvalues by Sturm counts, a wave an eigenvalue, 64 points a round;
 //   3. eigenvectors of the tridiagonal, a wave a vector, from its twisted factors (Parlett and Dhillon,
 //      Linear Algebra Appl. 267, 247 (1997));
-//   4. two Newton–Schulz steps Z ← Z (3 I − ZᵀZ)/2, which make the vectors of close eigenvalues orthogonal
+//   4. one or two Newton–Schulz steps Z ← Z (3 I − ZᵀZ)/2, which make the vectors of close eigenvalues orthogonal
 //      again: a gap g leaves them eps ‖T‖/g from it, and mixing them costs a residual of eps ‖T‖;
 //   5. the residuals and ZᵀZ decide whether the pairs are good: equal eigenvalues (a gap below about
 //      1e-11 ‖T‖) have no such vectors, and the caller then takes divide and conquer on the same T;
 //   6. the vectors transformed back, a wave a vector.
 // rocSOLVER's dsyevd spends n² / 2 dependent small launches on the reduction and merges on one
-// work-group: n 192 702 us here against 3863, n 64 189 against 1331, with smaller residuals.
+// work-group: n 192 526 us here against 3863, n 64 143 against 1316, with smaller residuals.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -35,20 +35,34 @@ __device__ __forceinline__ double dpp(double x) {
 }
 constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kHalfMirror = 0x141, kRor8 = 0x128;   // lanes l^1, l^2, 7−l of 8, l^8
 
+// x: rows of 16 lanes (32 lanes) 1, 3 exchanged for rows 0, 2 of y; x + y then holds x's sums over a pair of
+// rows in the even ones and y's in the odd ones
+template <int BIT>
+__device__ __forceinline__ double pair_sum(double x, double y) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    u2 a = __builtin_bit_cast(u2, x), b = __builtin_bit_cast(u2, y);
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        const auto r = BIT == 16 ? __builtin_amdgcn_permlane16_swap(a[w], b[w], false, false)
+                                 : __builtin_amdgcn_permlane32_swap(a[w], b[w], false, false);
+        a[w] = r[0];
+        b[w] = r[1];
+    }
+    return __builtin_bit_cast(double, a) + __builtin_bit_cast(double, b);
+}
+
 __device__ __forceinline__ double wave_sum(double x) {
     x += dpp<kXor1>(x);
     x += dpp<kXor2>(x);
     x += dpp<kHalfMirror>(x);
     x += dpp<kRor8>(x);
-    x += __shfl_xor(x, 16, 64);
-    x += __shfl_xor(x, 32, 64);
-    return x;
+    x = pair_sum<16>(x, x);
+    return pair_sum<32>(x, x);
 }
 
 template <int BIT>
 __device__ __forceinline__ double from_partner(double x) {
-    if constexpr (BIT == 16) return __shfl_xor(x, 16, 64);
-    else if constexpr (BIT == 8) return dpp<kRor8>(x);
+    if constexpr (BIT == 8) return dpp<kRor8>(x);
     else if constexpr (BIT == 4) return dpp<kHalfMirror>(x);
     else if constexpr (BIT == 2) return dpp<kXor2>(x);
     else return dpp<kXor1>(x);
@@ -65,9 +79,12 @@ __device__ __forceinline__ double half_wave_sums(const double (&s)[M], int lane,
 #pragma unroll
         for (int q = 0; q < H; ++q) {
             const double hi = q + H < M ? s[q + H < M ? q + H : 0] : 0.0;
-            t[q] = (up ? hi : s[q]) + from_partner<BIT>(up ? s[q] : hi);
+            if constexpr (BIT == 16) t[q] = pair_sum<16>(s[q], hi);
+            else t[q] = (up ? hi : s[q]) + from_partner<BIT>(up ? s[q] : hi);
         }
         if (up) *at += H;
+    } else if constexpr (BIT == 16) {
+        t[0] = pair_sum<16>(s[0], s[0]);
     } else {
         t[0] = s[0] + from_partner<BIT>(s[0]);
     }
@@ -75,16 +92,29 @@ __device__ __forceinline__ double half_wave_sums(const double (&s)[M], int lane,
     else return t[0];
 }
 
-// A (upper triangle, column-major) -> T = Qᵀ A Q, Q = H_0 H_1 .., H_k = I − tau_k v_k v_kᵀ with v_k zero up to k
-// and one at k + 1 (rows of Hv).  The matrix stays in registers, both halves of it: thread (x, y) of
+__device__ __forceinline__ double recip(double q) {   // 1/q to an ulp or two
+    double r = __builtin_amdgcn_rcp(q);
+    r = fma(r, fma(-q, r, 1.0), r);
+    return fma(r, fma(-q, r, 1.0), r);
+}
+
+__device__ __forceinline__ double recip_sqrt(double q) {   // 1/sqrt(q) likewise, q > 0
+    double r = __builtin_amdgcn_rsq(q);
+    r = fma(0.5 * r, fma(-q * r, r, 1.0), r);
+    return fma(0.5 * r, fma(-q * r, r, 1.0), r);
+}
+
+// A (upper triangle, column-major) -> T = Qᵀ A Q, Q = H_0 H_1 .., H_k = I − tau_k u_k u_kᵀ with u_k (row k of Hv)
+// zero up to k, beyond k + 1 the column itself.  The matrix stays in registers, both halves of it: thread (x, y) of
 // TX × 32 holds elements (x + TX r, y + 32 c).  A column then costs its own broadcast through LDS,
 // A v as sums over half waves, and the rank-two update: two barriers; every wave forms the norms and
 // scalars by itself.  Blocks of 32 columns behind column k drop out of the products.  Bound by the
-// waves' instructions: n 192 428 us with TX 16, 498 with 32 (which spills), 528 with 8.
+// chain of a column's sums and barriers and by the waves' instructions: n 192 319 us; before the permlane
+// sums and selects instead of branches 428 with TX 16, 498 with 32 (which spills), 528 with 8.
 template <int NB, int TX>
 __global__ __launch_bounds__(TX * 32) void k_tridiag(const double* __restrict__ A, int n, double* __restrict__ d,
                                                      double* __restrict__ e, double* __restrict__ Hv,
-                                                     double* __restrict__ tau_out) {
+                                                     double* __restrict__ tau_out, int* __restrict__ bad) {
     constexpr int NP = NB * 32, NQ = (NB + 1) / 2, NR = NP / TX;
     __shared__ double xs[2][NQ * 64], ps[NQ * 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ty = lane & 31, tx = 2 * wave + (lane >> 5);
@@ -96,6 +126,13 @@ __global__ __launch_bounds__(TX * 32) void k_tridiag(const double* __restrict__ 
             const int i = tx + TX * r, j = ty + 32 * c, lo = min(i, j), hi = max(i, j);
             a[r][c] = hi < n ? A[(size_t)hi * n + lo] : 0.0;
         }
+    // the elements have arrived: otherwise the loop waits for memory, and so for its own stores, on every column
+    // (n 192: 392 us against 319)
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+        for (int c = 0; c < NB; ++c) asm volatile("" : "+v"(a[r][c]));
+    if (tid == 0) bad[0] = 0;
     if (NP < NQ * 64 && tid < 32) {   // entries no row has
         xs[0][NP + tid] = xs[1][NP + tid] = 0.0;
         ps[NP + tid] = 0.0;
@@ -109,33 +146,38 @@ __global__ __launch_bounds__(TX * 32) void k_tridiag(const double* __restrict__ 
                 double* const x = xs[kk & 1];
                 if (ty == kk)
 #pragma unroll
-                    for (int r = R0; r < NR; ++r) x[tx + TX * r] = a[r][kc];
+                    for (int r = R0; r < NR; ++r) {
+                        const int i = tx + TX * r;
+                        x[i] = i > k ? a[r][kc] : 0.0;
+                        if (i == k) d[k] = a[r][kc];
+                    }
                 __syncthreads();
                 double xq[NQ], nrm = 0.0;
 #pragma unroll
                 for (int q = 0; q < NQ; ++q) {
-                    const int i = lane + 64 * q;
-                    xq[q] = i > k + 1 ? x[i] : 0.0;
-                    nrm += xq[q] * xq[q];
+                    xq[q] = lane + 64 * q < R0 * TX ? 0.0 : x[lane + 64 * q];
+                    nrm += lane + 64 * q == k + 1 ? 0.0 : xq[q] * xq[q];
                 }
                 const double alpha = x[k + 1];
+                double uc[MC];
+#pragma unroll
+                for (int c = 0; c < MC; ++c) uc[c] = x[ty + 32 * (kc + c)];
                 nrm = wave_sum(nrm);
-                double beta = alpha, tau = 0.0, sc = 0.0;
-                if (nrm != 0.0) {
-                    const double len = sqrt(alpha * alpha + nrm);
+                // u = column − beta e_{k+1}, tau = 2/uᵀu = 1/(|beta| (|beta| + |alpha|))
+                double beta = alpha, tau = 0.0;
+                if (nrm > 1e-280) {   // less is no part of any matrix whose products are normal numbers
+                    const double s2 = fma(alpha, alpha, nrm), len = s2 * recip_sqrt(s2);
                     beta = alpha >= 0.0 ? -len : len;
-                    tau = (beta - alpha) / beta;
-                    sc = 1.0 / (alpha - beta);
+                    tau = recip(len * (len + fabs(alpha)));
                 }
-                const auto v = [&](int i) { return i > k + 1 ? x[i] * sc : (i == k + 1 ? 1.0 : 0.0); };
+                const double u1 = alpha - beta;   // u at k + 1
 #pragma unroll
                 for (int q = 0; q < NQ; ++q) {
                     const int i = lane + 64 * q;
-                    xq[q] = i == k + 1 ? 1.0 : xq[q] * sc;   // v from here on
+                    xq[q] = i == k + 1 ? u1 : xq[q];
                     if (wave == q && i < n) Hv[(size_t)k * n + i] = xq[q];
                 }
                 if (tid == 0) {
-                    d[k] = x[k];
                     e[k] = beta;
                     tau_out[k] = tau;
                 }
@@ -144,31 +186,33 @@ __global__ __launch_bounds__(TX * 32) void k_tridiag(const double* __restrict__ 
                 for (int r = 0; r < MR; ++r) s[r] = 0.0;
 #pragma unroll
                 for (int c = 0; c < MC; ++c) {
-                    const double vc = v(ty + 32 * (kc + c));
+                    uc[c] = ty + 32 * (kc + c) == k + 1 ? u1 : uc[c];
 #pragma unroll
-                    for (int r = 0; r < MR; ++r) s[r] += a[R0 + r][kc + c] * vc;
+                    for (int r = 0; r < MR; ++r) s[r] += a[R0 + r][kc + c] * uc[c];
                 }
                 int at = 0;
                 const double y = half_wave_sums<MR, 16>(s, lane, &at);
                 if (at < MR) ps[tx + TX * (R0 + at)] = y;   // lanes that share a value write the same
                 __syncthreads();
+                // w = tau y − K u, K = tau² yᵀu / 2; what this does to rows and columns up to k is never read
                 double dot = 0.0;
 #pragma unroll
-                for (int q = 0; q < NQ; ++q) dot += lane + 64 * q > k ? ps[lane + 64 * q] * xq[q] : 0.0;
-                const double K = 0.5 * tau * tau * wave_sum(dot);
-                double vr[MR], wr[MR];   // v and w = tau y − K v of this thread's rows; its columns' one at a time
+                for (int q = 0; q < NQ; ++q) dot += lane + 64 * q < R0 * TX ? 0.0 : ps[lane + 64 * q] * xq[q];
+                double ur[MR], wr[MR];
 #pragma unroll
                 for (int r = 0; r < MR; ++r) {
                     const int i = tx + TX * (R0 + r);
-                    vr[r] = v(i);
-                    wr[r] = i > k ? tau * ps[i] - K * vr[r] : 0.0;
+                    ur[r] = i == k + 1 ? u1 : x[i];
+                    wr[r] = ps[i];
                 }
+                const double K = 0.5 * tau * tau * wave_sum(dot);
+#pragma unroll
+                for (int r = 0; r < MR; ++r) wr[r] = tau * wr[r] - K * ur[r];
 #pragma unroll
                 for (int c = 0; c < MC; ++c) {
-                    const int j = ty + 32 * (kc + c);
-                    const double vc = v(j), wc = j > k ? tau * ps[j] - K * vc : 0.0;
+                    const double wc = tau * ps[ty + 32 * (kc + c)] - K * uc[c];
 #pragma unroll
-                    for (int r = 0; r < MR; ++r) a[R0 + r][kc + c] -= vr[r] * wc + wr[r] * vc;
+                    for (int r = 0; r < MR; ++r) a[R0 + r][kc + c] -= ur[r] * wc + wr[r] * uc[c];
                 }
             }
         },
@@ -181,12 +225,6 @@ __global__ __launch_bounds__(TX * 32) void k_tridiag(const double* __restrict__ 
             if (i == j && i < n && i >= n - 2) d[i] = a[r][c];
             if (i == n - 1 && j == n - 2) e[j] = a[r][c];
         }
-}
-
-__device__ __forceinline__ double recip(double q) {   // 1/q to an ulp or two
-    double r = __builtin_amdgcn_rcp(q);
-    r = fma(r, fma(-q, r, 1.0), r);
-    return fma(r, fma(-q, r, 1.0), r);
 }
 
 __device__ __forceinline__ double wave_max(double x) {
@@ -228,7 +266,9 @@ __global__ __launch_bounds__(64) void k_tri_values(const double* __restrict__ d,
             if (fabs(q) < piv) q = -piv;
             cnt += q < 0.0;
             if (i == n) break;
-            q = ds[i] - x - es[i - 1] * es[i - 1] * recip(q);
+            double r = __builtin_amdgcn_rcp(q);   // one step: to a few ulps, which perturb e² by as much
+            r = fma(r, fma(-q, r, 1.0), r);
+            q = ds[i] - x - es[i - 1] * es[i - 1] * r;
         }
         const unsigned long long above = __ballot(cnt > k);   // points with more than k eigenvalues below them
         const int m = above ? __builtin_ctzll(above) : 64;
@@ -312,17 +352,35 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 
 // T = (3 I − ZᵀZ)/2 (GRAM; part: maxima of |ZᵀZ − I|) or out = Z T, 32 × 32 outputs a work-group, 16 × 16 a
 // wave straight from memory: the operands are in L2, and 36 work-groups leave nothing to gain from LDS.
+// The second step (`first`: the first one's maxima) has nothing to do where those are within kEigOrth: then
+// T stays and out = Z.
+constexpr double kEigRes = 2e-15, kEigOrth = 1e-8;
 template <bool GRAM>
 __global__ __launch_bounds__(256) void k_eig_mul(const double* __restrict__ Z, const double* __restrict__ T, int n,
-                                                 double* __restrict__ out, double* __restrict__ part) {
+                                                 double* __restrict__ out, double* __restrict__ part,
+                                                 const double* __restrict__ first) {
     __shared__ double red[4];
+    if (first) {
+        const int np = (int)(gridDim.x * gridDim.y), q = threadIdx.x & 63;   // np <= 36
+        if (__all(q >= np || first[q] <= kEigOrth)) {                        // the same in every wave
+            if (GRAM) {
+                if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = 0.0;
+                return;
+            }
+            for (int e = threadIdx.x; e < 1024; e += 256) {
+                const int i = blockIdx.x * 32 + (e & 31), j = blockIdx.y * 32 + (e >> 5);
+                if (i < n && j < n) out[(size_t)j * n + i] = Z[(size_t)j * n + i];
+            }
+            return;
+        }
+    }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
     const int i0 = blockIdx.x * 32 + (wave & 1) * 16, j0 = blockIdx.y * 32 + (wave >> 1) * 16;
     const int i = min(i0 + l16, n - 1), j = min(j0 + l16, n - 1);
     const double* __restrict__ pa = GRAM ? Z + (size_t)i * n : Z + i;
     const double* __restrict__ pb = (GRAM ? Z : T) + (size_t)j * n;
     d4 acc = {0.0, 0.0, 0.0, 0.0};
-    constexpr int U = 12;
+    constexpr int U = 24;   // two rounds of loads at n 192
     for (int k0 = 0; k0 < n; k0 += 4 * U) {
         double a[U], b[U];
 #pragma unroll
@@ -361,48 +419,29 @@ __global__ __launch_bounds__(256) void k_eig_mul(const double* __restrict__ Z, c
     part[blockIdx.y * gridDim.x + blockIdx.x] = m;
 }
 
-// bad = 1 unless every residual |T z − w z| is within kEigRes of |T| and ZᵀZ was within kEigOrth of one
+// bad (zero beforehand) = 1 unless every residual |T z − w z| is within kEigRes of |T| and ZᵀZ was within kEigOrth of one
 // before the last step
-constexpr double kEigRes = 2e-15, kEigOrth = 1e-8;
 template <int NQ>
-__global__ __launch_bounds__(1024) void k_tri_check(const double* __restrict__ d, const double* __restrict__ e, int n,
-                                                    const double* __restrict__ w, const double* __restrict__ Z,
-                                                    const double* __restrict__ part, int np, double* __restrict__ dev,
-                                                    int* __restrict__ bad) {
-    __shared__ double ds[NQ * 64], es[NQ * 64], red[16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+__global__ __launch_bounds__(256) void k_tri_check(const double* __restrict__ d, const double* __restrict__ e, int n,
+                                                   const double* __restrict__ w, const double* __restrict__ Z,
+                                                   const double* __restrict__ part, int np, int* __restrict__ bad) {
+    __shared__ double ds[NQ * 64], es[NQ * 64];
+    const int lane = threadIdx.x & 63, k = blockIdx.x * 4 + (threadIdx.x >> 6);
     const double t = load_t<NQ>(d, e, n, ds, es);
-    double m = 0.0, o = 0.0;
-    for (int k = wave; k < n; k += 16) {
-        const double* __restrict__ z = Z + (size_t)k * n;
-        const double x = w[k];
+    if (k >= n) return;
+    const double* __restrict__ z = Z + (size_t)k * n;
+    const double x = w[k];
+    bool ok = lane >= np || part[lane] <= kEigOrth;   // np <= 36
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const int i = lane + 64 * q;
-            if (i >= n) continue;
-            double v = (ds[i] - x) * z[i];
-            if (i > 0) v += es[i - 1] * z[i - 1];
-            if (i < n - 1) v += es[i] * z[i + 1];
-            m = fabs(v) <= m ? m : fabs(v);
-        }
+    for (int q = 0; q < NQ; ++q) {
+        const int i = lane + 64 * q;
+        if (i >= n) continue;
+        double v = (ds[i] - x) * z[i];
+        if (i > 0) v += es[i - 1] * z[i - 1];
+        if (i < n - 1) v += es[i] * z[i + 1];
+        ok = ok && fabs(v) <= kEigRes * t;
     }
-    for (int q = threadIdx.x; q < np; q += 1024) o = part[q] <= o ? o : part[q];
-    for (int s = 32; s > 0; s >>= 1) {
-        const double m2 = __shfl_xor(m, s, 64), o2 = __shfl_xor(o, s, 64);
-        m = m2 <= m ? m : m2;
-        o = o2 <= o ? o : o2;
-    }
-    const bool ok = m <= kEigRes * t && o <= kEigOrth;
-    if (lane == 0) red[wave] = ok ? 0.0 : 1.0;
-    if (threadIdx.x == 0) {
-        dev[0] = m / t;
-        dev[1] = o;
-    }
-    __syncthreads();
-    if (threadIdx.x) return;
-    double any = 0.0;
-    for (int q = 0; q < 16; ++q) any += red[q];
-    bad[0] = any != 0.0;
+    if (!__all(ok) && lane == 0) bad[0] = 1;
 }
 
 // Columns of Z <- H_0 .. H_{n−3} Z, a wave a column: n − 2 dot products of n in registers, eight reflectors
@@ -452,21 +491,22 @@ hipError_t eig_run(hipStream_t st, const double* A, int n, double* w, double* Z,
     const dim3 tiles((unsigned)((n + 31) / 32), (unsigned)((n + 31) / 32)), waves((unsigned)n), w64(64), w256(256);
     const int np = (int)(tiles.x * tiles.y);
     constexpr int TX = 16;
-    hipLaunchKernelGGL((k_tridiag<NB, TX>), dim3(1), dim3(TX * 32), 0, st, A, n, d, e, Hv, tau);
+    hipLaunchKernelGGL((k_tridiag<NB, TX>), dim3(1), dim3(TX * 32), 0, st, A, n, d, e, Hv, tau, bad);
     hipLaunchKernelGGL(k_tri_values<NQ>, waves, w64, 0, st, d, e, n, w);
     hipLaunchKernelGGL(k_tri_vectors<NQ>, waves, w64, 0, st, d, e, n, w, Z);
-    hipLaunchKernelGGL(k_eig_mul<true>, tiles, w256, 0, st, Z, (const double*)nullptr, n, T, part);
-    hipLaunchKernelGGL(k_eig_mul<false>, tiles, w256, 0, st, Z, T, n, Z1, part);
-    hipLaunchKernelGGL(k_eig_mul<true>, tiles, w256, 0, st, Z1, (const double*)nullptr, n, T, part);
-    hipLaunchKernelGGL(k_eig_mul<false>, tiles, w256, 0, st, Z1, T, n, Z, part);
-    hipLaunchKernelGGL(k_tri_check<NQ>, dim3(1), dim3(1024), 0, st, d, e, n, w, Z, part, np, part + np, bad);
+    const double *none = nullptr;
+    hipLaunchKernelGGL(k_eig_mul<true>, tiles, w256, 0, st, Z, none, n, T, part, none);
+    hipLaunchKernelGGL(k_eig_mul<false>, tiles, w256, 0, st, Z, T, n, Z1, part, none);
+    hipLaunchKernelGGL(k_eig_mul<true>, tiles, w256, 0, st, Z1, none, n, T, part + np, part);
+    hipLaunchKernelGGL(k_eig_mul<false>, tiles, w256, 0, st, Z1, T, n, Z, part + np, part);
+    hipLaunchKernelGGL(k_tri_check<NQ>, dim3((unsigned)(n + 3) / 4), w256, 0, st, d, e, n, w, Z, part + np, np, bad);
     if (n > 2) hipLaunchKernelGGL(k_back<NQ>, waves, w64, 0, st, Z, n, Hv, tau);
     return hipGetLastError();
 }
 
 }  // namespace
 
-size_t eig_ws(size_t n) { return 3 * n + 3 * n * n + 64; }
+size_t eig_ws(size_t n) { return 3 * n + 3 * n * n + 72; }
 
 hipError_t launch_eig(hipStream_t st, const double* A, size_t n, double* w, double* Z, double* ws, int* bad) {
     if (n <= 64) return eig_run<2>(st, A, (int)n, w, Z, ws, bad);
