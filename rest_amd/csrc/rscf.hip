@@ -205,6 +205,21 @@ __global__ void k_sumsq_diff(const double* __restrict__ A, const double* __restr
     if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
+// partial[k·kDotBlocks + b] = Σ x y_k over the block's elements, for every y at once: DIIS takes a row of its
+// matrix from one launch and one copy (as dot products one by one, 8 of them with a wait each, 150 us)
+constexpr int kDotBlocks = 64;
+struct Vecs {
+    const double* y[16];
+};
+__global__ __launch_bounds__(256) void k_dots(const double* __restrict__ x, Vecs v, size_t len,
+                                              double* __restrict__ partial) {
+    const double* __restrict__ y = v.y[blockIdx.y];
+    double acc = 0.0;
+    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < len; t += kDotBlocks * 256) acc += x[t] * y[t];
+    const double s = block_sum(acc);
+    if (threadIdx.x == 0) partial[blockIdx.y * kDotBlocks + blockIdx.x] = s;
+}
+
 struct Coefs {
     double c[16];
     const double* f[16];
@@ -435,6 +450,7 @@ int scf_core(rjk_ctx* ctx, const char* who, const double* S_h, const double* H_h
     double* eigws = n > rjk::kEigMin && n <= rjk::kEigMax ? mem.get(ctx, rjk::eig_ws(n), &rc) : nullptr;
     double* vj = mem.get(ctx, npair, &rc);
     double* partial = mem.get(ctx, kRedBlocks, &rc);
+    double* dots = mem.get(ctx, 16 * kDotBlocks, &rc);   // num_max_diis <= 16
     double* info_d = mem.get(ctx, 1, &rc);
     // per spin: Fock, extrapolated Fock, eigenvectors, densities (current, previous,
     // mixed), eigenvalues, occupations, exchange
@@ -913,6 +929,22 @@ int scf_core(rjk_ctx* ctx, const char* who, const double* S_h, const double* H_h
     int nvec = 0, head = 0;   // DIIS ring: vectors [head, head+nvec) mod nd
     bool shift_pending = false;   // first FP64 build after the switch: shift the stored vectors
     std::vector<double> Bmat((size_t)nd * nd, 0.0);
+    // row i of Bmat up to its diagonal: error vector i with the vectors before it
+    auto diis_row = [&](int i) -> int {
+        Vecs v = {};
+        for (int j = 0; j <= i; ++j) v.y[j] = ering + (size_t)((head + j) % nd) * ev_len;
+        double p[16 * kDotBlocks];
+        hipLaunchKernelGGL(k_dots, dim3(kDotBlocks, (unsigned)(i + 1)), b256, 0, st, v.y[i], v, ev_len, dots);
+        SCF_HIP(hipGetLastError());
+        SCF_HIP(hipMemcpyAsync(p, dots, (size_t)(i + 1) * kDotBlocks * sizeof(double), hipMemcpyDeviceToHost, st));
+        SCF_HIP(hipStreamSynchronize(st));
+        for (int j = 0; j <= i; ++j) {
+            double dot = 0.0;
+            for (int b = 0; b < kDotBlocks; ++b) dot += p[j * kDotBlocks + b];
+            Bmat[(size_t)i * nd + j] = Bmat[(size_t)j * nd + i] = dot;
+        }
+        return RJK_OK;
+    };
     bool converged = false;
     // REST's energy_records / prev_hamiltonian (src/scf_io/mod.rs:2850-2851, :3002-3057):
     // energies recorded by the DIIS steps, and a list of at most two slots of Fock matrices
@@ -982,13 +1014,7 @@ int scf_core(rjk_ctx* ctx, const char* who, const double* S_h, const double* H_h
                         SCF_HIP(hipGetLastError());
                     }
                 }
-                for (int i = 0; i < nvec; ++i)
-                    for (int j = 0; j <= i; ++j) {
-                        double dot = 0.0;
-                        SCF_BLAS(rocblas_ddot(h, (rocblas_int)ev_len, ering + (size_t)((head + i) % nd) * ev_len, 1,
-                                              ering + (size_t)((head + j) % nd) * ev_len, 1, &dot));
-                        Bmat[(size_t)i * nd + j] = Bmat[(size_t)j * nd + i] = dot;
-                    }
+                for (int i = 0; i < nvec; ++i) SCF_RC(diis_row(i));
             }
             shift_pending = false;
             // error vector e_s = F_s D_s S − S D_s F_s, spins back to back, into the ring slot
@@ -1018,12 +1044,7 @@ int scf_core(rjk_ctx* ctx, const char* who, const double* S_h, const double* H_h
                                        hipMemcpyDeviceToDevice, st));
             }
             ++nvec;
-            for (int k = 0; k < nvec; ++k) {
-                double dot = 0.0;
-                SCF_BLAS(rocblas_ddot(h, (rocblas_int)ev_len, e_new, 1, ering + (size_t)((head + k) % nd) * ev_len, 1,
-                                      &dot));
-                Bmat[(size_t)(nvec - 1) * nd + k] = Bmat[(size_t)k * nd + (nvec - 1)] = dot;
-            }
+            SCF_RC(diis_row(nvec - 1));
             std::vector<double> bm((size_t)nvec * nvec), inv;
             for (int i = 0; i < nvec; ++i)
                 for (int j = 0; j < nvec; ++j) bm[(size_t)i * nvec + j] = Bmat[(size_t)i * nd + j];
