@@ -1,5 +1,6 @@
-// rjk_eig.hip — eigenpairs of a small symmetric FP64 matrix (n <= 192), nine launches:
-//   1. tridiagonal reduction by one work-group with the matrix in its registers;
+// rjk_eig.hip — eigenpairs of a symmetric FP64 matrix of at most 1024 rows:
+//   1. tridiagonal reduction, up to 192 by one work-group with the matrix in its registers, beyond with
+//      one launch a column;
 //   2. eigenvalues by Sturm counts, a wave an eigenvalue, 64 points a round;
 //   3. eigenvectors of the tridiagonal, a wave a vector, from its twisted factors (Parlett and Dhillon,
 //      Linear Algebra Appl. 267, 247 (1997));
@@ -9,7 +10,8 @@
 //      1e-11 ‖T‖) have no such vectors, and the caller then takes divide and conquer on the same T;
 //   6. the vectors transformed back, a wave a vector.
 // rocSOLVER's dsyevd spends n² / 2 dependent small launches on the reduction and merges on one
-// work-group: n 192 526 us here against 3863, n 64 143 against 1316, with smaller residuals.
+// work-group: n 192 526 us here against 3863, n 64 143 against 1316, n 336 2185 against 7028, n 1024 10.2 ms
+// against 22.7, with smaller residuals.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -227,6 +229,129 @@ __global__ __launch_bounds__(TX * 32) void k_tridiag(const double* __restrict__ 
         }
 }
 
+// The reduction for n > 192, one launch a column: what a column needs of all rows (the dot product that makes
+// w of y = A u, the next column, its norm) every work-group computes from y for itself, and one pass over
+// its own rows applies the rank-two update and multiplies by the new u.  A: full square, rows
+// contiguous; Y and C: [2][n] by parity of k, y_k and the entries of column k + 1 before update k.
+// A launch is 4 to 5 us and the pass over the rows, in L2, hides in it.
+constexpr int kStepRows = 2;   // of a wave
+__global__ __launch_bounds__(256) void k_step_start(const double* __restrict__ A, int n, double* __restrict__ F,
+                                                    double* __restrict__ C, int* __restrict__ bad) {
+    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (t == 0) bad[0] = 0;
+    if (t >= (size_t)n * n) return;
+    const int i = (int)(t / n), j = (int)(t % n);
+    const double x = A[(size_t)max(i, j) * n + min(i, j)];
+    F[t] = x;
+    if (i == 0) C[n + j] = x;
+}
+
+template <int NQ>
+__global__ __launch_bounds__(256) void k_step(double* __restrict__ F, int n, int k, double* __restrict__ d,
+                                              double* __restrict__ e, double* __restrict__ tau_out,
+                                              double* __restrict__ Hv, double* __restrict__ Y, double* __restrict__ C) {
+    __shared__ double vs[NQ * 64], ws[NQ * 64], us[NQ * 64], red[2][4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int i0 = k + 1 + (blockIdx.x * 4 + wave) * kStepRows, q0 = (k + 1) / 64;
+    double a[kStepRows][NQ];
+#pragma unroll
+    for (int r = 0; r < kStepRows; ++r)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const int j = lane + 64 * q;
+            a[r][q] = q >= q0 && i0 + r < n && j < n ? F[(size_t)(i0 + r) * n + j] : 0.0;
+        }
+    const double* __restrict__ yk = Y + (size_t)((k + 1) & 1) * n;
+    const double* __restrict__ ck = C + (size_t)((k + 1) & 1) * n;
+    const double tau0 = k ? tau_out[k - 1] : 0.0;
+    constexpr int NT = (NQ * 64 + 255) / 256;
+    double y[NT], v[NT], x[NT], dot = 0.0;
+#pragma unroll
+    for (int m = 0; m < NT; ++m) {
+        const int i = tid + 256 * m;
+        const bool in = i >= k && i < n;
+        y[m] = in && k ? yk[i] : 0.0;
+        v[m] = in && k ? Hv[(size_t)(k - 1) * n + i] : 0.0;
+        x[m] = in ? ck[i] : 0.0;
+        dot += y[m] * v[m];
+    }
+    dot = wave_sum(dot);
+    if (lane == 0) red[0][wave] = dot;
+    __syncthreads();
+    const double K = 0.5 * tau0 * tau0 * ((red[0][0] + red[0][1]) + (red[0][2] + red[0][3]));
+#pragma unroll
+    for (int m = 0; m < NT; ++m) {
+        const int i = tid + 256 * m;
+        if (i < NQ * 64) {
+            vs[i] = v[m];
+            ws[i] = y[m] = tau0 * y[m] - K * v[m];   // y: w from here on
+        }
+    }
+    __syncthreads();
+    const double vk = vs[k], wk = ws[k];
+    double nrm = 0.0;
+#pragma unroll
+    for (int m = 0; m < NT; ++m) {
+        const int i = tid + 256 * m;
+        x[m] -= v[m] * wk + y[m] * vk;
+        if (i < NQ * 64) us[i] = i > k ? x[m] : 0.0;
+        if (i > k + 1) nrm += x[m] * x[m];
+        if (i == k && blockIdx.x == 0) d[k] = x[m];
+    }
+    nrm = wave_sum(nrm);
+    if (lane == 0) red[1][wave] = nrm;
+    __syncthreads();
+    nrm = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+    const double alpha = us[k + 1];
+    double beta = alpha, tau = 0.0;
+    if (nrm > 1e-280) {   // as in k_tridiag
+        const double s2 = fma(alpha, alpha, nrm), len = s2 * recip_sqrt(s2);
+        beta = alpha >= 0.0 ? -len : len;
+        tau = recip(len * (len + fabs(alpha)));
+    }
+    const double u1 = alpha - beta;
+    if (blockIdx.x == 0) {
+#pragma unroll
+        for (int m = 0; m < NT; ++m) {
+            const int i = tid + 256 * m;
+            if (i < n) Hv[(size_t)k * n + i] = i == k + 1 ? u1 : us[i];
+        }
+        if (tid == 0) {
+            e[k] = beta;
+            tau_out[k] = tau;
+        }
+    }
+    double s[kStepRows];
+#pragma unroll
+    for (int r = 0; r < kStepRows; ++r) s[r] = 0.0;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        if (q < q0) continue;
+        const int j = lane + 64 * q;
+        const double vj = vs[j], wj = ws[j], uj = j == k + 1 ? u1 : us[j];
+#pragma unroll
+        for (int r = 0; r < kStepRows; ++r) {
+            const int i = min(i0 + r, n - 1);
+            a[r][q] -= vs[i] * wj + ws[i] * vj;
+            s[r] += a[r][q] * uj;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kStepRows; ++r) {
+        const int i = i0 + r;
+        const double yi = wave_sum(s[r]);
+        if (i >= n) continue;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const int j = lane + 64 * q;
+            if (q >= q0 && j < n) F[(size_t)i * n + j] = a[r][q];
+            if (j == k + 1) C[(size_t)(k & 1) * n + i] = a[r][q];
+            if (i == n - 1 && j == n - 1 && k == n - 2) d[i] = a[r][q];
+        }
+        if (lane == 0) Y[(size_t)(k & 1) * n + i] = yi;
+    }
+}
+
 __device__ __forceinline__ double wave_max(double x) {
     for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o, 64));
     return x;
@@ -351,18 +476,22 @@ __global__ __launch_bounds__(64) void k_tri_vectors(const double* __restrict__ d
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 // T = (3 I − ZᵀZ)/2 (GRAM; part: maxima of |ZᵀZ − I|) or out = Z T, 32 × 32 outputs a work-group, 16 × 16 a
-// wave straight from memory: the operands are in L2, and 36 work-groups leave nothing to gain from LDS.
+// wave straight from memory: the operands are in L2, and a hundred work-groups leave little to gain from LDS.
 // The second step (`first`: the first one's maxima) has nothing to do where those are within kEigOrth: then
 // T stays and out = Z.
 constexpr double kEigRes = 2e-15, kEigOrth = 1e-8;
+__device__ __forceinline__ bool within(const double* __restrict__ x, int n, double bound) {   // by a whole wave
+    bool ok = true;
+    for (int q = threadIdx.x & 63; q < n; q += 64) ok = ok && x[q] <= bound;
+    return __all(ok);
+}
 template <bool GRAM>
 __global__ __launch_bounds__(256) void k_eig_mul(const double* __restrict__ Z, const double* __restrict__ T, int n,
                                                  double* __restrict__ out, double* __restrict__ part,
                                                  const double* __restrict__ first) {
     __shared__ double red[4];
     if (first) {
-        const int np = (int)(gridDim.x * gridDim.y), q = threadIdx.x & 63;   // np <= 36
-        if (__all(q >= np || first[q] <= kEigOrth)) {                        // the same in every wave
+        if (within(first, (int)(gridDim.x * gridDim.y), kEigOrth)) {   // the same in every wave
             if (GRAM) {
                 if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = 0.0;
                 return;
@@ -431,7 +560,7 @@ __global__ __launch_bounds__(256) void k_tri_check(const double* __restrict__ d,
     if (k >= n) return;
     const double* __restrict__ z = Z + (size_t)k * n;
     const double x = w[k];
-    bool ok = lane >= np || part[lane] <= kEigOrth;   // np <= 36
+    bool ok = within(part, np, kEigOrth);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         const int i = lane + 64 * q;
@@ -444,12 +573,12 @@ __global__ __launch_bounds__(256) void k_tri_check(const double* __restrict__ d,
     if (!__all(ok) && lane == 0) bad[0] = 1;
 }
 
-// Columns of Z <- H_0 .. H_{n−3} Z, a wave a column: n − 2 dot products of n in registers, eight reflectors
-// loaded ahead.
+// Columns of Z <- H_0 .. H_{n−3} Z, a wave a column: n − 2 dot products of n in registers, four or eight
+// reflectors loaded ahead.
 template <int NQ>
 __global__ __launch_bounds__(64) void k_back(double* __restrict__ Z, int n, const double* __restrict__ Hv,
                                              const double* __restrict__ tau) {
-    constexpr int U = 8;
+    constexpr int U = NQ > 3 ? 4 : 8;
     const int lane = threadIdx.x;
     double* __restrict__ zc = Z + (size_t)blockIdx.x * n;
     double z[NQ], v[U][NQ], t[U];
@@ -483,15 +612,23 @@ __global__ __launch_bounds__(64) void k_back(double* __restrict__ Z, int n, cons
 
 namespace {
 
-template <int NB>
+// NB: register blocks of the reduction, 0 for a launch a column; NQ: elements a lane of a wave's vector
+template <int NB, int NQ>
 hipError_t eig_run(hipStream_t st, const double* A, int n, double* w, double* Z, double* ws, int* bad) {
-    constexpr int NQ = (NB + 1) / 2;
     const size_t n2 = (size_t)n * n;
     double *d = ws, *e = ws + n, *tau = ws + 2 * n, *Hv = ws + 3 * n, *Z1 = Hv + n2, *T = Z1 + n2, *part = T + n2;
     const dim3 tiles((unsigned)((n + 31) / 32), (unsigned)((n + 31) / 32)), waves((unsigned)n), w64(64), w256(256);
     const int np = (int)(tiles.x * tiles.y);
-    constexpr int TX = 16;
-    hipLaunchKernelGGL((k_tridiag<NB, TX>), dim3(1), dim3(TX * 32), 0, st, A, n, d, e, Hv, tau, bad);
+    if constexpr (NB > 0) {
+        constexpr int TX = 16;
+        hipLaunchKernelGGL((k_tridiag<NB, TX>), dim3(1), dim3(TX * 32), 0, st, A, n, d, e, Hv, tau, bad);
+    } else {
+        double *Y = T, *C = T + 2 * n;   // the working square in Z1
+        hipLaunchKernelGGL(k_step_start, dim3((unsigned)((n2 + 255) / 256)), w256, 0, st, A, n, Z1, C, bad);
+        for (int k = 0; k <= n - 2; ++k)
+            hipLaunchKernelGGL(k_step<NQ>, dim3((unsigned)((n - 1 - k + 4 * kStepRows - 1) / (4 * kStepRows))), w256, 0, st, Z1,
+                               n, k, d, e, tau, Hv, Y, C);
+    }
     hipLaunchKernelGGL(k_tri_values<NQ>, waves, w64, 0, st, d, e, n, w);
     hipLaunchKernelGGL(k_tri_vectors<NQ>, waves, w64, 0, st, d, e, n, w, Z);
     const double *none = nullptr;
@@ -506,12 +643,15 @@ hipError_t eig_run(hipStream_t st, const double* A, int n, double* w, double* Z,
 
 }  // namespace
 
-size_t eig_ws(size_t n) { return 3 * n + 3 * n * n + 72; }
+size_t eig_ws(size_t n) { return 3 * n + 3 * n * n + 2 * ((n + 31) / 32) * ((n + 31) / 32); }
 
 hipError_t launch_eig(hipStream_t st, const double* A, size_t n, double* w, double* Z, double* ws, int* bad) {
-    if (n <= 64) return eig_run<2>(st, A, (int)n, w, Z, ws, bad);
-    if (n <= 128) return eig_run<4>(st, A, (int)n, w, Z, ws, bad);
-    return eig_run<6>(st, A, (int)n, w, Z, ws, bad);
+    if (n <= 64) return eig_run<2, 1>(st, A, (int)n, w, Z, ws, bad);
+    if (n <= 128) return eig_run<4, 2>(st, A, (int)n, w, Z, ws, bad);
+    if (n <= 192) return eig_run<6, 3>(st, A, (int)n, w, Z, ws, bad);
+    if (n <= 320) return eig_run<0, 5>(st, A, (int)n, w, Z, ws, bad);
+    if (n <= 512) return eig_run<0, 8>(st, A, (int)n, w, Z, ws, bad);
+    return eig_run<0, 16>(st, A, (int)n, w, Z, ws, bad);
 }
 
 hipError_t launch_eig_back(hipStream_t st, double* Z, size_t n, const double* ws) {
@@ -523,7 +663,10 @@ hipError_t launch_eig_back(hipStream_t st, double* Z, size_t n, const double* ws
     };
     if (n <= 64) return go(k_back<1>);
     if (n <= 128) return go(k_back<2>);
-    return go(k_back<3>);
+    if (n <= 192) return go(k_back<3>);
+    if (n <= 320) return go(k_back<5>);
+    if (n <= 512) return go(k_back<8>);
+    return go(k_back<16>);
 }
 
 }  // namespace rjk

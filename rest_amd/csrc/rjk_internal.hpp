@@ -191,7 +191,7 @@ hipError_t launch_pivot_chol(hipStream_t st, const double* dm, size_t nbf, size_
 // eigenvalues w ascending, vectors the columns of Z.  ws: eig_ws(n) doubles, which start with T's diagonal [n]
 // and off-diagonal [n].  *bad: the pairs are not good enough; eigenvectors of T in Z then become A's by
 // launch_eig_back.
-constexpr size_t kEigMax = 192;
+constexpr size_t kEigMax = 1024;
 // The SCF's smaller problems, free atoms among them, stay with dsyevd: an atom's shells are exactly
 // degenerate, so these kernels would hand most of them on, and which way an open shell points, hence the
 // guess made of it, is whichever vectors the solver gives.

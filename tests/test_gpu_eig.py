@@ -1,5 +1,5 @@
 """The eigensolver of the SCF at the edges of its sizes: 40 / 41 (rocSOLVER below), 64 / 65, 128 / 129 (register
-blocks), 192 / 193 (rocSOLVER above); and spectra with clusters: gaps of 1e-7 (orthogonalised), exact
+blocks), 192 / 193 (a launch a column above), 320 / 321, 512 / 513, 1024 / 1025 (rocSOLVER above); and spectra with clusters: gaps of 1e-7 (orthogonalised), exact
 fourfold degeneracy (divide and conquer on the same tridiagonal).  With B = 0 the Fock matrix of a guess
 step is H, so its orbitals solve H C = S C eps.  Bounds: an eigensolver's backward error of n eps |F'|,
 with F' = S^(-1/2) H S^(-1/2) and S within a factor 3 of one: 10 n eps |H| on H C - S C eps and 10 n eps on
@@ -23,7 +23,8 @@ def spectrum(kind, n, rng):
 
 @pytest.mark.parametrize("n,kind", [(40, "random"), (41, "random"), (64, "random"), (65, "random"), (96, "close"),
                                     (128, "random"), (129, "fourfold"), (191, "close"), (192, "random"),
-                                    (192, "fourfold"), (193, "random")])
+                                    (192, "fourfold"), (193, "random"), (256, "close"), (320, "random"), (321, "fourfold"),
+                                    (512, "random"), (513, "close"), (1024, "random"), (1025, "random")])
 def test_guess_step_eigenpairs(n, kind):
     print(f"[gpu-case] eigenpairs n={n} {kind}", flush=True)
     rng = np.random.default_rng(n)
