@@ -156,8 +156,8 @@ __global__ void k_pack_upper(const double* __restrict__ g, size_t nbf, size_t ld
 // Pivoted Cholesky factor of the symmetric part of a column-major nbf × nbf D: L[k][i], D ≈ Σ_k L_k L_kᵀ,
 // for the density-only K (an SCF density has rank nocc, and this finds it in nocc steps where an
 // eigensolver needs n).  One work-group: a step is a pivot search, one column of D and k products per
-// row, too little to spread over CUs; what bounds it is the chain of barriers and L2 latencies, about 2 us a
-// step (nbf 192, rank 40: 80 us against 3 ms for the eigenpairs).  The first columns of L stay in
+// row, too little to spread over CUs; what bounds it is the chain of barriers and L2 latencies, about 4 us a
+// step (nbf 192, rank 40: 154 us against 3 ms for the eigenpairs).  The first columns of L stay in
 // LDS as well, the products of a row are split over 1024 / nbf threads.
 // Stops when the largest remaining diagonal is at most cut·max diag(D); rank -> out[0], or -1 if a
 // diagonal falls below −cut·max (D is not positive semidefinite) or kmax columns do not suffice.
@@ -165,21 +165,19 @@ constexpr int kCholThreads = 1024;
 constexpr size_t kCholSmall = 256;   // largest nbf of the one-work-group kernel
 constexpr int kCholLds = 16384;   // doubles of L kept in LDS
 __global__ __launch_bounds__(kCholThreads) void k_pivot_chol(const double* __restrict__ dm, int n, int kmax, double cut,
-                                                             double* __restrict__ diag, double* __restrict__ L,
-                                                             int* __restrict__ out) {
+                                                             double* __restrict__ L, int* __restrict__ out) {
     extern __shared__ double sm[];
     double* ls = sm;                        // [kCholLds]
     double* part = sm + kCholLds;           // [kCholThreads]
     double* lp = part + kCholThreads;       // [kmax] row p of L
-    __shared__ double wmax[16], wmin[16];
-    __shared__ int widx[16];
-    __shared__ double sh_max, sh_min;
-    __shared__ int sh_p;
+    __shared__ double wmax[2][16], wmin[2][16], dg[kCholSmall];   // dg: the remaining diagonal
+    __shared__ int widx[2][16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int klds = kCholLds / n;          // columns of L kept in LDS
-    int G = 1;                              // threads that share a row's products
+    int G = 1;                              // threads that share a row's products: all rows at once (n <= kCholSmall)
     while (2 * G * n <= kCholThreads) G *= 2;
-    for (int i = tid; i < n; i += kCholThreads) diag[i] = dm[(size_t)i * n + i];
+    const int row = tid / G, q = tid % G;
+    for (int i = tid; i < n; i += kCholThreads) dg[i] = dm[(size_t)i * n + i];
     __syncthreads();
     double d0 = 0.0;
     int rank = -1;
@@ -187,7 +185,7 @@ __global__ __launch_bounds__(kCholThreads) void k_pivot_chol(const double* __res
         double mx = -INFINITY, mn = INFINITY;
         int at = 0;
         for (int i = tid; i < n; i += kCholThreads) {
-            const double d = diag[i];
+            const double d = dg[i];
             if (d > mx) {
                 mx = d;
                 at = i;
@@ -205,26 +203,26 @@ __global__ __launch_bounds__(kCholThreads) void k_pivot_chol(const double* __res
             mn = fmin(mn, __shfl_xor(mn, o, 64));
         }
         if (lane == 0) {
-            wmax[wave] = mx;
-            wmin[wave] = mn;
-            widx[wave] = at;
+            wmax[k & 1][wave] = mx;
+            wmin[k & 1][wave] = mn;
+            widx[k & 1][wave] = at;
         }
         __syncthreads();
-        if (tid == 0) {
-            for (int w = 1; w < 16; ++w) {
-                if (wmax[w] > wmax[0]) {
-                    wmax[0] = wmax[w];
-                    widx[0] = widx[w];
-                }
-                wmin[0] = fmin(wmin[0], wmin[w]);
+        mx = wmax[k & 1][lane & 15];   // every wave finishes for itself
+        mn = wmin[k & 1][lane & 15];
+        at = widx[k & 1][lane & 15];
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) {
+            const double m2 = __shfl_xor(mx, o, 64);
+            const int a2 = __shfl_xor(at, o, 64);
+            if (m2 > mx || (m2 == mx && a2 < at)) {
+                mx = m2;
+                at = a2;
             }
-            sh_max = wmax[0];
-            sh_min = wmin[0];
-            sh_p = widx[0];
+            mn = fmin(mn, __shfl_xor(mn, o, 64));
         }
-        __syncthreads();
-        const double top = sh_max, low = sh_min;
-        const int p = sh_p;
+        const double top = mx, low = mn;
+        const int p = at;
         if (k == 0) d0 = top;
         if (low < -cut * d0 || !(top >= 0.0)) break;      // not positive semidefinite (or NaN)
         if (top <= cut * d0) {
@@ -232,40 +230,33 @@ __global__ __launch_bounds__(kCholThreads) void k_pivot_chol(const double* __res
             break;
         }
         if (k == kmax) break;
+        // D's column is on its way while row p of L is gathered and multiplied
+        const double dcol = q == 0 && row < n ? 0.5 * (dm[(size_t)p * n + row] + dm[(size_t)row * n + p]) : 0.0;
         for (int j = tid; j < k; j += kCholThreads) lp[j] = j < klds ? ls[j * n + p] : L[(size_t)j * n + p];
         __syncthreads();
-        const double inv = 1.0 / sqrt(top);
-        for (int i0 = 0; i0 < n; i0 += kCholThreads / G) {   // G > 1 only when one pass covers all rows
-            const int i = i0 + tid / G, q = tid % G;
-            double v = 0.0;
-            if (i < n) {
-                const int kl = min(k, klds);
-                int j = q;
-                for (; j < kl; j += G) v += ls[j * n + i] * lp[j];
-                for (; j + 7 * G < k; j += 8 * G) {   // eight loads in flight
-                    double x[8];
+        double v = 0.0;
+        if (row < n) {
+            const int kl = min(k, klds);
+            int j = q;
+            for (; j < kl; j += G) v += ls[j * n + row] * lp[j];
+            for (; j + 7 * G < k; j += 8 * G) {   // eight loads in flight
+                double x[8];
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) x[u] = L[(size_t)(j + u * G) * n + i];
+                for (int u = 0; u < 8; ++u) x[u] = L[(size_t)(j + u * G) * n + row];
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) v += x[u] * lp[j + u * G];
-                }
-                for (; j < k; j += G) v += L[(size_t)j * n + i] * lp[j];
-                if (G == 1) v = (0.5 * (dm[(size_t)p * n + i] + dm[(size_t)i * n + p]) - v) * inv;
+                for (int u = 0; u < 8; ++u) v += x[u] * lp[j + u * G];
             }
-            if (G > 1) {
-                part[tid] = v;
-                __syncthreads();
-                if (q == 0 && i < n) {
-                    for (int u = 1; u < G; ++u) v += part[tid + u];
-                    v = (0.5 * (dm[(size_t)p * n + i] + dm[(size_t)i * n + p]) - v) * inv;
-                }
-            }
-            if (q == 0 && i < n) {
-                const double l = i == p ? top * inv : v;
-                if (k < klds) ls[k * n + i] = l;
-                L[(size_t)k * n + i] = l;
-                diag[i] = i == p ? 0.0 : diag[i] - l * l;
-            }
+            for (; j < k; j += G) v += L[(size_t)j * n + row] * lp[j];
+        }
+        part[tid] = v;
+        __syncthreads();
+        if (q == 0 && row < n) {
+            for (int u = 1; u < G; ++u) v += part[tid + u];
+            const double inv = 1.0 / sqrt(top);
+            const double l = row == p ? top * inv : (dcol - v) * inv;
+            if (k < klds) ls[k * n + row] = l;
+            L[(size_t)k * n + row] = l;
+            dg[row] = row == p ? 0.0 : dg[row] - l * l;
         }
         __syncthreads();
     }
@@ -479,7 +470,7 @@ hipError_t launch_pivot_chol(hipStream_t st, const double* dm, size_t nbf, size_
     const hipError_t e =
         hipFuncSetAttribute((const void*)k_pivot_chol, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pivot_chol, dim3(1), dim3(kCholThreads), lds, st, dm, (int)nbf, (int)kmax, cut, diag, L, rank);
+    hipLaunchKernelGGL(k_pivot_chol, dim3(1), dim3(kCholThreads), lds, st, dm, (int)nbf, (int)kmax, cut, L, rank);
     hipLaunchKernelGGL(k_chol_residual, dim3(nb, nb), dim3(256), 0, st, dm, (int)nbf, L, rank, blockmax);
     hipLaunchKernelGGL(k_max, dim3(1), dim3(256), 0, st, blockmax, (int)(nb * nb), residual);
     return hipGetLastError();
