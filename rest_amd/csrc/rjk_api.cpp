@@ -360,27 +360,38 @@ int j_run(rjk_ctx* ctx, const void* b, int prec, const double* dm_dev, int ns, d
     double* gamma = (double*)(base + L.cv.off[L.iG]);
     double* jpart = (double*)(base + L.cv.off[L.ij]);
     hipStream_t st = ctx->stream;
+    const double sb = prec == RJK_PREC_FP64 ? 8.0 : 4.0;
+    const double jpass = (double)ctx->npair * ctx->naux * sb + 8.0 * ns * ctx->npair;   // one pass over B
+    if (j_small(ctx->ldb, ctx->naux)) {
+        for (int pass = 0; pass < 2; ++pass) {
+            PhaseScope ps(ctx, pass, prec, jpass, timed);
+            RJK_HIP(ctx, launch_j_small(st, prec, b, ctx->ldb, ctx->naux, ctx->nbf, ctx->npair, ns, dm_dev, full_dm, scale,
+                                        gamma, vj_dev, pass));
+        }
+        return RJK_OK;
+    }
+    const size_t nsplit = j_splits(ctx->ldb, prec, L.nsplit);
     {
         PhaseScope ps(ctx, 4, 0, 0.0, timed);
         RJK_HIP(ctx, launch_dm_weights(st, dm_dev, ctx->nbf, ctx->npair, ctx->ldb, ns, full_dm, w));
     }
-    const double sb = prec == RJK_PREC_FP64 ? 8.0 : 4.0;
-    const double jpass = (double)ctx->npair * ctx->naux * sb + 8.0 * ns * ctx->npair;   // one pass over B
     {
         PhaseScope ps(ctx, 0, prec, jpass, timed);
         RJK_HIP(ctx, launch_jgamma(st, prec, b, ctx->ldb, ctx->naux, ns, w, L.nchunk, gpart));
     }
-    {
+    if (L.nchunk == 1) {
+        gamma = gpart;   // the sum of one
+    } else {
         PhaseScope ps(ctx, 4, 0, 0.0, timed);
         RJK_HIP(ctx, launch_gamma_reduce(st, gpart, L.nchunk, ns, ctx->naux, gamma));
     }
     {
         PhaseScope ps(ctx, 1, prec, jpass, timed);
-        RJK_HIP(ctx, launch_jacc(st, prec, b, ctx->ldb, ctx->naux, ns, gamma, L.nsplit, jpart));
+        RJK_HIP(ctx, launch_jacc(st, prec, b, ctx->ldb, ctx->naux, ns, gamma, nsplit, jpart));
     }
     {
         PhaseScope ps(ctx, 4, 0, 0.0, timed);
-        RJK_HIP(ctx, launch_jreduce(st, jpart, L.nsplit, ns, ctx->ldb, ctx->npair, scale, vj_dev));
+        RJK_HIP(ctx, launch_jreduce(st, jpart, nsplit, ns, ctx->ldb, ctx->npair, scale, vj_dev));
     }
     return RJK_OK;
 }
@@ -764,7 +775,7 @@ int vk_dm_general(rjk_ctx* ctx, const double* dm_dev, int ns, double scale, doub
 // columns, per call:
 //   FP64, nbf <= 4096, D positive semidefinite of low rank (an SCF density has rank nocc):
 //     the pivoted Cholesky factor, unless it leaves out more than kCholTol·max|D| (nbf 192, rank
-//     40: 0.08 ms against 3 ms for the eigenpairs; nbf 1536, rank 320: 3 against 38);
+//     40: 0.15 ms against 3 ms for the eigenpairs; nbf 1536, rank 320: 3 against 38);
 //   else the eigenpairs with |λ| > kEigRelCut·max|λ| (rocSOLVER dsyevd), weights λ.
 // The lower precisions keep the eigenpairs: their K depends on the columns at its own rounding.
 int vk_dm_device(rjk_ctx* ctx, const void* b, const double* dm_dev, size_t spin_channel, double scaling_factor,

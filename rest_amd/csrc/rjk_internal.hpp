@@ -114,6 +114,10 @@ struct PhaseScope {
 
 // ---- launchers (return hipError_t of the launch) ------------------------
 // J
+bool j_small(size_t ldb, size_t naux);
+hipError_t launch_j_small(hipStream_t st, int prec, const void* b, size_t ldb, size_t naux, size_t nbf, size_t npair,
+                          int nspin, const double* dm, int full_dm, double scale, double* gamma, double* vj, int pass);
+size_t j_splits(size_t ldb, int prec, size_t nsplit);
 hipError_t launch_dm_weights(hipStream_t st, const double* dm, size_t nbf, size_t npair, size_t ldb,
                              int nspin, int full_dm, double* w);
 hipError_t launch_jgamma(hipStream_t st, int prec, const void* b, size_t ldb, size_t naux, int nspin,

@@ -32,6 +32,7 @@ template <> struct V16<float> { using T = f4; static constexpr int N = 4; };
 
 constexpr int kJBlock = 256;
 constexpr int kGammaCols = 8;
+constexpr size_t kJSmallLd = 2048, kJSmallAux = 1024;
 
 __device__ inline double wave_sum(double v) {
 #pragma unroll
@@ -48,6 +49,15 @@ __device__ inline void unpair(size_t p, size_t* i, size_t* j) {
     *i = p - jj * (jj + 1) / 2;
 }
 
+// weight of pair p
+__device__ inline double pair_weight(const double* __restrict__ d, size_t nbf, size_t p, int full_dm) {
+    size_t i, j;
+    unpair(p, &i, &j);
+    if (i == j) return d[i + j * nbf];
+    if (full_dm) return d[i + j * nbf] + d[j + i * nbf];   // Σ_{kl} over both triangles
+    return 2.0 * d[i + j * nbf];                           // upper triangle only
+}
+
 __global__ __launch_bounds__(256) void k_dm_weights(const double* __restrict__ dm, size_t nbf, size_t npair,
                                                     size_t ldb, int nspin, int full_dm, double* __restrict__ w) {
     size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -56,16 +66,7 @@ __global__ __launch_bounds__(256) void k_dm_weights(const double* __restrict__ d
         for (int s = 0; s < nspin; ++s) w[s * ldb + p] = 0.0;
         return;
     }
-    size_t i, j;
-    unpair(p, &i, &j);
-    for (int s = 0; s < nspin; ++s) {
-        const double* d = dm + (size_t)s * nbf * nbf;
-        double v;
-        if (i == j) v = d[i + j * nbf];
-        else if (full_dm) v = d[i + j * nbf] + d[j + i * nbf];   // Σ_{kl} over both triangles
-        else v = 2.0 * d[i + j * nbf];                         // upper triangle only
-        w[s * ldb + p] = v;
-    }
+    for (int s = 0; s < nspin; ++s) w[s * ldb + p] = pair_weight(dm + (size_t)s * nbf * nbf, nbf, p, full_dm);
 }
 
 template <typename BT, int NS, int G>
@@ -218,15 +219,117 @@ __global__ __launch_bounds__(kJBlock) void k_jacc(const BT* __restrict__ b, size
     }
 }
 
-__global__ void k_jreduce(const double* __restrict__ jpart, int nsplit, int nspin, size_t ldb, size_t npair,
-                          double scale, double* __restrict__ vj) {
-    size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npair) return;
+// Four threads a pair, four loads in flight each: one thread for all of 56 splits took 15 us at nbf 192.
+__global__ __launch_bounds__(256) void k_jreduce(const double* __restrict__ jpart, int nsplit, int nspin, size_t ldb,
+                                                 size_t npair, double scale, double* __restrict__ vj) {
+    __shared__ double sh[4][64];
+    const int x = threadIdx.x & 63, g = threadIdx.x >> 6;
+    const size_t p = (size_t)blockIdx.x * 64 + x;
     for (int s = 0; s < nspin; ++s) {
+        const double* __restrict__ src = jpart + (size_t)s * ldb + p;
+        const size_t step = (size_t)nspin * ldb;
         double acc = 0;
-        for (int q = 0; q < nsplit; ++q) acc += jpart[((size_t)q * nspin + s) * ldb + p];
-        vj[(size_t)s * npair + p] = acc * scale;
+        if (p < npair) {
+            int q = g;
+            for (; q + 12 < nsplit; q += 16)
+                acc += (src[q * step] + src[(q + 4) * step]) + (src[(q + 8) * step] + src[(q + 12) * step]);
+            for (; q < nsplit; q += 4) acc += src[q * step];
+        }
+        sh[g][x] = acc;
+        __syncthreads();
+        if (g == 0 && p < npair) vj[(size_t)s * npair + p] = ((sh[0][x] + sh[1][x]) + (sh[2][x] + sh[3][x])) * scale;
+        __syncthreads();
     }
+}
+
+// J of a small problem (j_small) in two launches instead of five, each of which is its few microseconds of
+// launch: γ with the weights formed in LDS by every work-group, and J straight from γ.  nbf 24, naux
+// 113: 81 us for the J and K host calls together against 86, where copies and waits take most.
+template <typename BT, int NS>
+__global__ __launch_bounds__(256) void k_jgamma_small(const BT* __restrict__ b, size_t ldb, int naux,
+                                                      const double* __restrict__ dm, size_t nbf, size_t npair,
+                                                      int full_dm, double* __restrict__ gamma) {
+    using VT = typename V16<BT>::T;
+    constexpr int N = V16<BT>::N;
+    __shared__ double ws[NS][kJSmallLd];
+    for (size_t p = threadIdx.x; p < ldb; p += 256)
+#pragma unroll
+        for (int s = 0; s < NS; ++s) ws[s][p] = p < npair ? pair_weight(dm + s * nbf * nbf, nbf, p, full_dm) : 0.0;
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nvec = (int)(ldb / N);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int P = blockIdx.x * 8 + wave * 2 + c;
+        if (P >= naux) continue;
+        const VT* __restrict__ bp = reinterpret_cast<const VT*>(b) + (size_t)P * nvec;
+        double acc[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) acc[s] = 0.0;
+        for (int v = lane; v < nvec; v += 64) {
+            const VT x = bp[v];
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+#pragma unroll
+                for (int e = 0; e < N; ++e) acc[s] = fma((double)x[e], ws[s][v * N + e], acc[s]);
+        }
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const double t = wave_sum(acc[s]);
+            if (lane == 0) gamma[(size_t)s * naux + P] = t;
+        }
+    }
+}
+
+template <typename BT, int NS>
+__global__ __launch_bounds__(256) void k_jacc_small(const BT* __restrict__ b, size_t ldb, int naux,
+                                                    const double* __restrict__ gamma, size_t npair, double scale,
+                                                    double* __restrict__ vj) {
+    using VT = typename V16<BT>::T;
+    constexpr int N = V16<BT>::N;
+    __shared__ double sh[NS][16][16 * N + 1];
+    const int x = threadIdx.x & 15, y = threadIdx.x >> 4, nvec = (int)(ldb / N), v = blockIdx.x * 16 + x;
+    double acc[NS][N];
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int e = 0; e < N; ++e) acc[s][e] = 0.0;
+    if (v < nvec)
+#pragma unroll 4
+        for (int P = y; P < naux; P += 16) {
+            const VT t = *(reinterpret_cast<const VT*>(b) + (size_t)P * nvec + v);
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                const double g = gamma[(size_t)s * naux + P];
+#pragma unroll
+                for (int e = 0; e < N; ++e) acc[s][e] = fma((double)t[e], g, acc[s][e]);
+            }
+        }
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int e = 0; e < N; ++e) sh[s][y][x * N + e] = acc[s][e];
+    __syncthreads();
+    const int c = threadIdx.x & 63, s = threadIdx.x >> 6;   // 16·N <= 64 pairs, NS <= 4 spins
+    const size_t p = (size_t)blockIdx.x * 16 * N + c;
+    if (c < 16 * N && s < NS && p < npair) {
+        double t = 0;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) t += sh[s][q][c];
+        vj[(size_t)s * npair + p] = t * scale;
+    }
+}
+
+template <typename BT, int NS>
+hipError_t jsmall_t(hipStream_t st, const BT* b, size_t ldb, size_t naux, size_t nbf, size_t npair, const double* dm,
+                    int full_dm, double scale, double* gamma, double* vj, int pass) {
+    constexpr size_t per = 16 * V16<BT>::N;
+    if (pass == 0)
+        hipLaunchKernelGGL((k_jgamma_small<BT, NS>), dim3((unsigned)((naux + 7) / 8)), dim3(256), 0, st, b, ldb, (int)naux,
+                           dm, nbf, npair, full_dm, gamma);
+    else
+        hipLaunchKernelGGL((k_jacc_small<BT, NS>), dim3((unsigned)((npair + per - 1) / per)), dim3(256), 0, st, b, ldb,
+                           (int)naux, gamma, npair, scale, vj);
+    return hipGetLastError();
 }
 
 template <typename BT>
@@ -275,6 +378,26 @@ void j_plan(size_t ldb, size_t naux, int prec, size_t* nchunk, size_t* nsplit) {
     *nsplit = std::min(std::max<size_t>(sp, 1), smax);
 }
 
+// Up to 2048 pairs (the weights of two spins in LDS) and 1024 auxiliary functions (64 columns a thread)
+bool j_small(size_t ldb, size_t naux) { return ldb <= kJSmallLd && naux <= kJSmallAux; }
+
+hipError_t launch_j_small(hipStream_t st, int prec, const void* b, size_t ldb, size_t naux, size_t nbf, size_t npair,
+                          int nspin, const double* dm, int full_dm, double scale, double* gamma, double* vj, int pass) {
+    if (prec == RJK_PREC_FP64)
+        return nspin == 1 ? jsmall_t<double, 1>(st, (const double*)b, ldb, naux, nbf, npair, dm, full_dm, scale, gamma, vj, pass)
+                          : jsmall_t<double, 2>(st, (const double*)b, ldb, naux, nbf, npair, dm, full_dm, scale, gamma, vj, pass);
+    return nspin == 1 ? jsmall_t<float, 1>(st, (const float*)b, ldb, naux, nbf, npair, dm, full_dm, scale, gamma, vj, pass)
+                      : jsmall_t<float, 2>(st, (const float*)b, ldb, naux, nbf, npair, dm, full_dm, scale, gamma, vj, pass);
+}
+
+// Splits that a J accumulation uses of the j_plan's: enough work-groups for four a CU, since the partial sums of
+// every split are written and read again (nbf 768, FP32 B: J accumulation 668 us against 706 with a target of
+// 4096 and 691 with 2048; 512: 706)
+size_t j_splits(size_t ldb, int prec, size_t nsplit) {
+    const size_t bx = (ldb / (prec == RJK_PREC_FP64 ? 2 : 4) + kJBlock - 1) / kJBlock;
+    return std::min(nsplit, std::max<size_t>(1, (1024 + bx - 1) / bx));
+}
+
 hipError_t launch_dm_weights(hipStream_t st, const double* dm, size_t nbf, size_t npair, size_t ldb, int nspin,
                              int full_dm, double* w) {
     hipLaunchKernelGGL(k_dm_weights, dim3((unsigned)((ldb + 255) / 256)), dim3(256), 0, st, dm, nbf, npair, ldb,
@@ -305,7 +428,7 @@ hipError_t launch_jacc(hipStream_t st, int prec, const void* b, size_t ldb, size
 
 hipError_t launch_jreduce(hipStream_t st, const double* jpart, size_t nsplit, int nspin, size_t ldb, size_t npair,
                           double scale, double* vj) {
-    hipLaunchKernelGGL(k_jreduce, dim3((unsigned)((npair + 255) / 256)), dim3(256), 0, st, jpart, (int)nsplit, nspin,
+    hipLaunchKernelGGL(k_jreduce, dim3((unsigned)((npair + 63) / 64)), dim3(256), 0, st, jpart, (int)nsplit, nspin,
                        ldb, npair, scale, vj);
     return hipGetLastError();
 }
