@@ -53,6 +53,7 @@ struct rjk_ctx {
     size_t ws_size = 0;
     void* io = nullptr;       // grow-only staging of the host-pointer entry points (inputs, outputs)
     size_t io_size = 0;
+    void* pin = nullptr;      // kPinBytes of pinned host memory between small host arrays and io
     void* aux = nullptr;      // grow-only scratch of the density-only route (eigenpairs, statistics)
     size_t aux_size = 0;
     void* scratch = nullptr;  // this device's allocation-free J scratch (address from hipGetSymbolAddress)

@@ -34,3 +34,26 @@ def test_j_small_edges(nbf, naux, ns):
             assert np.abs(ri.vj(ds, ns, 0.7) - up).max() <= 1e-12 * nbf * big
         assert np.abs(ri.vj(ds, ns, 0.7, full_dm=True) - full).max() <= 1e-12 * nbf * big
         assert np.abs(ri.vj(ds, ns, 0.7, prec=jk.PREC_FP32) - up).max() <= 1e-6 * nbf * big
+
+
+@pytest.mark.parametrize("nbf", [24, 181, 182])
+def test_host_calls_on_both_sides_of_the_pinned_size(nbf):
+    """Densities of 181 x 181 pass through 256 KiB of pinned memory, of 182 x 182 directly; J, both K routes and two
+    contexts in turn must each return their own results."""
+    rng = np.random.default_rng(nbf)
+    naux, nocc = 19, 5
+    npair = nbf * (nbf + 1) // 2
+    b = [rng.standard_normal((npair, naux)) / np.sqrt(naux) for _ in range(2)]
+    with jk.DeviceRI(nbf, naux) as r0, jk.DeviceRI(nbf, naux) as r1:
+        for r, x in zip((r0, r1), b):
+            r.set_rimatr(x)
+        for it in range(3):
+            for r, x in zip((r0, r1), b):
+                c = rng.standard_normal((nbf, nocc)) / np.sqrt(nbf)
+                occ = rng.uniform(0.5, 2.0, nocc)
+                d = (c * occ) @ c.T
+                j, k = orc.vj_upper_rimatr(x, [d], 1, 1.0), orc.vk_upper_occ(x, True, [c], [nocc - 1], [occ], 1, -0.5)
+                big = max(np.abs(j).max(), np.abs(k).max())
+                assert np.abs(r.vj([d], 1) - j).max() <= 1e-12 * nbf * big
+                assert np.abs(r.vk_occ([c], [nocc - 1], [occ], 1, -0.5) - k).max() <= 1e-12 * nbf * big
+                assert np.abs(r.vk_dm([d], 1, -0.5) - k).max() <= 1e-12 * nbf * big
