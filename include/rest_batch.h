@@ -42,8 +42,7 @@ extern "C" {
 typedef struct rjk_batch rjk_batch;
 
 /* Stages timed by rjk_batch_profile: 0 D weights, 1 γ, 2 J accumulation, 3 C' preparation,
- * 4 / 5 K half-transform (narrow / wide tile class; BF16: up to / above 32 columns a tile), 6 / 7 K SYRK (narrow or, at FP64/FP32,
- * every problem / wide), 8 split reduction. */
+ * 4 / 5 K half-transform (narrow / wide tile class; BF16: up to / above 32 columns a tile), 6 / 7 K SYRK (narrow / wide: 64- / 128-row tiles), 8 split reduction. */
 #define RJK_BATCH_NUM_STAGES 9
 
 /* Device bytes rjk_batch_create allocates for these problems at precision prec (B, inputs,
@@ -93,9 +92,9 @@ int rjk_batch_synchronize(rjk_batch* batch);
 int rjk_batch_profile(rjk_batch* batch, double scale_j, double scale_k, double* stage_ms);
 /* Time every candidate configuration `reps` times, keep the fastest; best_ms (may be NULL) receives its time. */
 int rjk_batch_autotune(rjk_batch* batch, int reps, double* best_ms);
-/* Current configuration: problems with nbf_pad < khalf_cut use the narrow tiles (FP64/FP32: 64×64
- * half-transform tiles, else 128×64; BF16: 64-wide half-transform and SYRK tiles, else 128-wide
- * where nbf_pad is a multiple of 128); waves_per_cu persistent work-groups per CU for the tile kernels. */
+/* Current configuration: problems with nbf_pad < khalf_cut use the narrow tiles (FP64/FP32: 64-row
+ * half-transform tiles, else 128; BF16: 64-wide SYRK tiles, else 128-wide where nbf_pad is a
+ * multiple of 128); waves_per_cu persistent work-groups per CU for the tile kernels. */
 int rjk_batch_config(const rjk_batch* batch, int* khalf_cut, int* waves_per_cu);
 int rjk_batch_set_config(rjk_batch* batch, int khalf_cut, int waves_per_cu);
 

@@ -67,7 +67,6 @@ struct Tables {
     const size_t* cols;    // Σ ceil(naux / kGammaGroup): γ work items
     const size_t* jseg;    // Σ J-accumulation segments
     const size_t* prep;    // Σ nbf_pad·nk
-    const size_t* syrk;    // Σ nsplit·ntile2
 };
 
 __device__ inline int find_prob(const size_t* __restrict__ off, int n, size_t x) {
@@ -223,7 +222,8 @@ __global__ __launch_bounds__(256) void k_b_prep(const BProb* __restrict__ pr, in
 }
 
 // half-transform over the problems of one tile variant: items of problem j
-// (subset order) start at off[j]; round_up(naux, 8) · ntm · ntc items each
+// (subset order) start at off[j]; round_up(naux, 8) · ntm · ntc items each, tiles that hold a row below
+// nbf and a column below nocc
 template <typename T, int FM, int FN>
 __global__ __launch_bounds__(kBlock) void k_b_khalf(const BProb* __restrict__ pr, const int* __restrict__ sub,
                                                     const size_t* __restrict__ off, int nsub) {
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kBlock) void k_b_khalf(const BProb* __restrict__ pr
         const BProb& P = pr[sub[j]];
         if (!P.active) continue;
         const size_t local = it - off[j];
-        const int ntm = P.nbf_pad / TM, ntc = P.nk / TN, per = ntm * ntc;
+        const int ntm = (P.nbf + TM - 1) / TM, ntc = (P.ncb * kTileK + TN - 1) / TN, per = ntm * ntc;
         const size_t xcd = local % kXcd, kq = local / kXcd;
         const int Pl = (int)((kq / per) * kXcd + xcd);
         if (Pl >= P.naux) continue;   // padding items (uniform per work-group)
@@ -244,16 +244,18 @@ __global__ __launch_bounds__(kBlock) void k_b_khalf(const BProb* __restrict__ pr
     }
 }
 
+// SYRK over the problems of one tile class (tiles of 32·F): nsplit · ntile2 items per problem
 template <typename T, int F>
-__global__ __launch_bounds__(kBlock) void k_b_ksyrk(const BProb* __restrict__ pr, int np, Tables tb) {
+__global__ __launch_bounds__(kBlock) void k_b_ksyrk(const BProb* __restrict__ pr, const int* __restrict__ sub,
+                                                    const size_t* __restrict__ off, int nsub) {
     constexpr int Tt = 32 * F;
-    const size_t total = tb.syrk[np];
+    const size_t total = off[nsub];
     for (size_t it = blockIdx.x; it < total; it += gridDim.x) {
-        const int q = find_prob(tb.syrk, np, it);
-        const BProb& P = pr[q];
+        const int q = find_prob(off, nsub, it);
+        const BProb& P = pr[sub[q]];
         if (!P.active) continue;
-        const size_t local = it - tb.syrk[q];
-        const size_t nt = (size_t)P.nbf_pad / Tt, nt2 = nt * (nt + 1) / 2;
+        const size_t local = it - off[q];
+        const size_t nt = ((size_t)P.nbf + Tt - 1) / Tt, nt2 = nt * (nt + 1) / 2;
         const size_t xcd = local % kXcd, kq = local / kXcd;
         const size_t t = kq % nt2;
         const int split = (int)((kq / nt2) * kXcd + xcd);
@@ -548,9 +550,23 @@ size_t prob_bytes(const BProb& P, int prec) {
 bool valid_prec(int prec) { return prec == RJK_PREC_FP64 || prec == RJK_PREC_FP32 || is_bf(prec); }
 
 // Half-transform groups, a launch each.  BF16: column tiles of 2, 4 or 6 fragments, one tile for up to 96
-// occupied columns (each B element is then read and split once).  FP64/FP32: 64 × 64 and 128 × 64 tiles of
-// rjk_ktiles.hpp (0 and 1).
-constexpr int kHalfGroups = 3;
+// occupied columns (each B element is then read and split once).  FP64/FP32: 64- or 128-row tiles (tile class 0
+// or 1) of rjk_ktiles.hpp by 2, 4 or 5 groups of 16 columns, groups 0-2 and 3-5.
+constexpr int kHalfGroups = 6;
+constexpr int kFpGroups[3] = {2, 4, 5};
+
+// index into kFpGroups, as rjk_api.cpp's k_tile_groups: the fewest columns, a tile costing about one group more
+// than its own, within the 64-column padding of M' (24 clusters of 10 to 80 occupied orbitals in 64-column
+// tiles: FP64 10.8 ms, FP32 6.5; fitted 7.8 and 4.5)
+int fp_group(int ncb) {
+    int best = 1;
+    for (int g = 0; g < 3; ++g) {
+        const int fn = kFpGroups[g], tiles = (ncb + fn - 1) / fn;
+        const int bfn = kFpGroups[best], btiles = (ncb + bfn - 1) / bfn;
+        if (tiles * fn <= (ncb + 3) / 4 * 4 && tiles * (fn + 1) < btiles * (bfn + 1)) best = g;
+    }
+    return best;
+}
 
 // 16-column fragments of a BF16 problem's column tiles: as few tiles of at most 6 as hold them, of one width
 size_t half_frags(size_t nocc) {
@@ -572,12 +588,12 @@ struct rjk_batch {
     hipStream_t own = nullptr, stream = nullptr;
     std::vector<BProb> h;            // host copy of the problem table
     BProb* d_prob = nullptr;
-    size_t* d_tab = nullptr;         // the five prefix tables back to back
+    size_t* d_tab = nullptr;         // the four prefix tables back to back
     int* d_sub = nullptr;            // [kHalfGroups][nprob] problem lists of the half-transform groups
     size_t* d_suboff = nullptr;      // [kHalfGroups][nprob + 1] their item offsets
-    int* d_ssub = nullptr;           // [2][nprob] problem lists of the two SYRK tile classes (BF16)
+    int* d_ssub = nullptr;           // [2][nprob] problem lists of the two SYRK tile classes
     size_t* d_syrkoff = nullptr;     // [2][nprob + 1] their item offsets
-    std::vector<size_t> t_pairs, t_cols, t_jseg, t_prep, t_syrk;
+    std::vector<size_t> t_pairs, t_cols, t_jseg, t_prep;
     std::vector<void*> allocs;
     double* scratch = nullptr;       // FP64 staging for uploads / the synthetic fill
     size_t scratch_elems = 0;
@@ -622,24 +638,33 @@ Tables tables(const rjk_batch* b) {
     t.cols = b->d_tab + n1;
     t.jseg = b->d_tab + 2 * n1;
     t.prep = b->d_tab + 3 * n1;
-    t.syrk = b->d_tab + 4 * n1;
     return t;
 }
 
-// Tile class of a problem under the current cut: 0 = narrow (FP: 64 × 64 half-transform tiles;
+// Tile class of a problem under the current cut: 0 = narrow (FP: 64-row half-transform tiles;
 // BF16: 64-wide SYRK tiles), 1 = wide (128); BF16 needs nbf_pad % 128 == 0 for 1.
 int tile_class(const rjk_batch* b, const BProb& P) {
     if (P.nbf_pad < b->khalf_cut) return 0;
     return (is_bf(b->prec) && P.nbf_pad % 128) ? 0 : 1;
 }
 
+// SYRK tile class: 64 or 128 rows.  FP64 takes 128 beyond 640 functions, FP32 64 throughout (as the
+// single-problem K, for its reasons).
+int syrk_class(const rjk_batch* b, const BProb& P) {
+    if (is_bf(b->prec)) return tile_class(b, P);
+    return b->prec == RJK_PREC_FP64 && P.nbf > 640 ? 1 : 0;
+}
+
 int half_group(const rjk_batch* b, const BProb& P) {
-    return is_bf(b->prec) ? (int)half_frags(P.nocc) / 2 - 1 : tile_class(b, P);
+    return is_bf(b->prec) ? (int)half_frags(P.nocc) / 2 - 1 : 3 * tile_class(b, P) + fp_group(P.ncb);
 }
 
 // work items of a problem's half-transform
 size_t half_items(const rjk_batch* b, const BProb& P) {
-    if (!is_bf(b->prec)) return rup(P.naux, 8) * (size_t)(P.nbf_pad / (tile_class(b, P) ? 128 : 64)) * (P.nk / 64);
+    if (!is_bf(b->prec)) {
+        const int tm = tile_class(b, P) ? 128 : 64, fn = kFpGroups[fp_group(P.ncb)];
+        return rup(P.naux, 8) * (size_t)((P.nbf + tm - 1) / tm) * (size_t)((P.ncb + fn - 1) / fn);
+    }
     const size_t units = rup(P.naux, 8) / 8 * ((P.nbf + kHalfRows - 1) / kHalfRows), tc = 16 * half_frags(P.nocc);
     return 8 * ((units + kHalfWaves - 1) / kHalfWaves) * ((rup(P.nocc, 32) + tc - 1) / tc);
 }
@@ -656,12 +681,10 @@ int build_subsets(rjk_batch* b) {
         const int g = half_group(b, P);
         sub[g].push_back(q);
         off[g].push_back(off[g].back() + half_items(b, P));
-        if (bf) {
-            const int v = tile_class(b, P);
-            const size_t nt = (size_t)P.nbf_pad / (v == 0 ? 64 : 128);
-            ssub[v].push_back(q);
-            soff[v].push_back(soff[v].back() + (size_t)P.nsplit * (nt * (nt + 1) / 2));
-        }
+        const int v = syrk_class(b, P);
+        const size_t tile = v == 0 ? 64 : 128, nt = bf ? (size_t)P.nbf_pad / tile : ((size_t)P.nbf + tile - 1) / tile;
+        ssub[v].push_back(q);
+        soff[v].push_back(soff[v].back() + (size_t)P.nsplit * (nt * (nt + 1) / 2));
     }
     // entries past a list's end stay zero (never searched: its length bounds the search)
     std::vector<int> hs(kHalfGroups * np, 0), hss(2 * np, 0);
@@ -693,8 +716,8 @@ unsigned grid_items(const rjk_batch* b, size_t items, int per_cu) {
 }
 
 // Records ev[k] before stage k and ev[kStages] after the last (ev may be null).  Stages: 0 weights,
-// 1 γ, 2 J accumulation, 3 C' preparation, 4-5 half-transform (narrow, wide), 6-7 SYRK (narrow /
-// all for FP, wide), 8 split reduction.
+// 1 γ, 2 J accumulation, 3 C' preparation, 4-5 half-transform (narrow, wide), 6-7 SYRK (narrow,
+// wide), 8 split reduction.
 template <typename T>
 int enqueue_fp(rjk_batch* b, hipEvent_t* ev) {
     const int np = (int)b->h.size();
@@ -713,17 +736,25 @@ int enqueue_fp(rjk_batch* b, hipEvent_t* ev) {
     mark(3);
     hipLaunchKernelGGL(k_b_prep<T>, dim3(grid_elem(b->t_prep.back())), dim3(256), 0, st, b->d_prob, np, tb);
     mark(4);
-    if (b->t_sub_items[0])
-        hipLaunchKernelGGL((k_b_khalf<T, 1, 4>), dim3(grid_items(b, b->t_sub_items[0], b->waves)), dim3(kBlock), 0,
-                           st, b->d_prob, b->d_sub, b->d_suboff, b->t_sub_n[0]);
+    auto tiles = [&](auto kern, size_t items, const int* sub, const size_t* off, int nsub) {
+        if (items)
+            hipLaunchKernelGGL(kern, dim3(grid_items(b, items, b->waves)), dim3(kBlock), 0, st, b->d_prob, sub, off, nsub);
+    };
+    auto half = [&](auto kern, int g) {
+        tiles(kern, b->t_sub_items[g], b->d_sub + g * np, b->d_suboff + g * (np + 1), b->t_sub_n[g]);
+    };
+    half(k_b_khalf<T, 1, 2>, 0);
+    half(k_b_khalf<T, 1, 4>, 1);
+    half(k_b_khalf<T, 1, 5>, 2);
     mark(5);
-    if (b->t_sub_items[1])
-        hipLaunchKernelGGL((k_b_khalf<T, 2, 4>), dim3(grid_items(b, b->t_sub_items[1], b->waves)), dim3(kBlock), 0,
-                           st, b->d_prob, b->d_sub + np, b->d_suboff + (np + 1), b->t_sub_n[1]);
+    half(k_b_khalf<T, 2, 2>, 3);
+    half(k_b_khalf<T, 2, 4>, 4);
+    half(k_b_khalf<T, 2, 5>, 5);
     mark(6);
-    hipLaunchKernelGGL((k_b_ksyrk<T, 4>), dim3(grid_items(b, b->t_syrk.back(), b->waves)), dim3(kBlock), 0, st,
-                       b->d_prob, np, tb);
+    tiles(k_b_ksyrk<T, 2>, b->t_syrk_items[0], b->d_ssub, b->d_syrkoff, b->t_ssub_n[0]);
     mark(7);
+    if constexpr (sizeof(T) == 8)
+        tiles(k_b_ksyrk<T, 4>, b->t_syrk_items[1], b->d_ssub + np, b->d_syrkoff + (np + 1), b->t_ssub_n[1]);
     mark(8);
     hipLaunchKernelGGL(k_b_kreduce, dim3(grid_elem(b->t_pairs.back())), dim3(256), 0, st, b->d_prob, np, tb, b->sk);
     mark(9);
@@ -945,12 +976,8 @@ int rjk_batch_create(int device, size_t nprob, const size_t* nbf, const size_t* 
     prefix(b->t_cols, [](const BProb& P) { return (size_t)(P.naux + kGammaGroup - 1) / kGammaGroup; });
     prefix(b->t_jseg, [&](const BProb& P) { return (P.ldb + 256 * (16 / es) - 1) / (256 * (16 / es)); });
     prefix(b->t_prep, [](const BProb& P) { return (size_t)P.nbf_pad * P.nk; });
-    prefix(b->t_syrk, [](const BProb& P) {
-        const size_t nt = (size_t)P.nbf_pad / 128;
-        return (size_t)P.nsplit * (nt * (nt + 1) / 2);
-    });
     std::vector<size_t> tab;
-    for (auto* t : {&b->t_pairs, &b->t_cols, &b->t_jseg, &b->t_prep, &b->t_syrk}) tab.insert(tab.end(), t->begin(), t->end());
+    for (auto* t : {&b->t_pairs, &b->t_cols, &b->t_jseg, &b->t_prep}) tab.insert(tab.end(), t->begin(), t->end());
     if (hipMalloc((void**)&b->d_prob, nprob * sizeof(BProb)) != hipSuccess ||
         hipMalloc((void**)&b->d_tab, tab.size() * sizeof(size_t)) != hipSuccess ||
         hipMalloc((void**)&b->d_sub, kHalfGroups * nprob * sizeof(int)) != hipSuccess ||
