@@ -168,7 +168,8 @@ int rjk_vk_upper_occ_dev(rjk_ctx* ctx, const double* eigv_dev, size_t num_state,
  *   K_s = scaling_factor · upper(Σ_P B_P D_s B_P)
  * for any D, read in full (REST's _dsymm(B_P, D) then _dsymm(·, B_P), :2730-2732,
  * :2675-2677).  A symmetric D (max|D−Dᵀ| <= 1e-10·max|D| for every spin) is
- * factorised on the device as D = U Λ Uᵀ and the occupied route runs with
+ * factorised on the device, at FP64 a positive semidefinite one of low rank (nbf <= 4096)
+ * by pivoted Cholesky, else as D = U Λ Uᵀ, and the occupied route runs with
  * signed weights Λ at `prec`; any other D takes the general route at FP64,
  * K = upper(Σ_P (B_P D)(B_P)ᵀ) through the FP64 half-transform and one DGEMM
  * per block of auxiliary columns (about 6·nbf³ FLOP per column). */
