@@ -574,6 +574,12 @@ size_t half_frags(size_t nocc) {
     return (f + tiles - 1) / tiles * 2;
 }
 
+// Persistent work-groups per CU where the autotuner has not run.  Four hide the waits of the FP32 and FP64
+// tiles (one graph of 24 clusters of 2 to 16 waters, 2 against 4: FP32 8.58 and 7.90 ms, FP64 15.7 and 15.4; 3 of 24 to
+// 28 waters: 18.3 and 16.7, 33.7 and 33.0; 24 of 1 to 4: 0.32 and 0.28, 0.41 and 0.38).  The BF16 tiles hold two of
+// their work-groups a CU, and more in line only lengthen the last round (7.29 and 7.37 ms; 3: 7.75).
+int default_waves(int prec) { return is_bf(prec) ? 2 : 4; }
+
 bool valid_shape(size_t nbf, size_t naux, size_t nocc) {
     return nbf != 0 && naux != 0 && nocc != 0 && nocc <= nbf && nbf <= 32768 && naux <= (1u << 24);
 }
@@ -600,7 +606,7 @@ struct rjk_batch {
     size_t bytes_b = 0, bytes_total = 0;
     // launch configuration (autotuned)
     int khalf_cut = 256;             // nbf_pad below this uses the narrow tile class
-    int waves = 2;                   // persistent work-groups per CU for the tile kernels
+    int waves = 2;                   // persistent work-groups per CU for the tile kernels (default_waves)
     int ncu = 256;
     int t_sub_n[kHalfGroups] = {};
     size_t t_sub_items[kHalfGroups] = {};
@@ -902,6 +908,7 @@ int rjk_batch_create(int device, size_t nprob, const size_t* nbf, const size_t* 
     rjk_batch* b = new rjk_batch();
     b->device = device;
     b->prec = prec;
+    b->waves = default_waves(prec);
     auto fail_free = [&](int code) {
         rjk_batch_destroy(b);
         return code;
