@@ -181,7 +181,7 @@ int rjk_vk_upper_with_ri_v_use_dm_only_sync(rjk_ctx* ctx, const double* dm,
                                             int prec, double* vk_upper);
 /* Device form of the density-only route: dm_dev (spin_channel × nbf × nbf, column-major) and
  * vk_dev (spin_channel × npair) in HBM, the same semantics and routes as above; a D holding
- * NaN/Inf gives RJK_ERR_NONFINITE.  Synchronises the stream (the route is chosen on the host). */
+ * NaN/Inf gives RJK_ERR_NONFINITE.  Synchronises the stream: vk_dev holds the result on return. */
 int rjk_vk_upper_dm_dev(rjk_ctx* ctx, const double* dm_dev, size_t spin_channel,
                         double scaling_factor, int prec, double* vk_dev);
 

@@ -980,7 +980,11 @@ extern "C" int rjk_vk_upper_dm_dev(rjk_ctx* ctx, const double* dm_dev, size_t sp
     const void* b = nullptr;
     int rc = check_common(ctx, spin_channel, prec, true, &b);
     if (rc) return rc;
-    return vk_dm_device(ctx, b, dm_dev, spin_channel, scaling_factor, prec, vk_dev);
+    rc = vk_dm_device(ctx, b, dm_dev, spin_channel, scaling_factor, prec, vk_dev);
+    if (rc) return rc;
+    // the result is ready when the call returns, on every route and for a reader on any stream
+    RJK_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return RJK_OK;
 }
 
 extern "C" int rjk_vk_upper_with_rimatr_use_dm_only_sync(rjk_ctx* ctx, const double* dm, size_t spin_channel,
