@@ -38,7 +38,7 @@ size_t rlg_num_params(const rlg_net* net);
 int rlg_set_stream(rlg_net* net, void* stream);
 int rlg_set_params(rlg_net* net, const float* params_host);
 int rlg_get_params(rlg_net* net, float* params_host);
-/* y_dev[batch][n_out] = net(x_dev[batch][n_in]); batch <= max_batch. */
+/* y_dev[batch][n_out] = net(x_dev[batch][n_in]); batch <= max_batch; y_dev may overlap x_dev. */
 int rlg_forward(rlg_net* net, const float* x_dev, size_t batch, float* y_dev);
 /* Forward, masked-MSE loss and backward; the gradient stays on the device for
  * rlg_adam_step and is also copied to grad_host (rlg_num_params floats) when

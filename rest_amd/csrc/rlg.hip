@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -388,8 +389,14 @@ int rlg_forward(rlg_net* n, const float* x_dev, size_t batch, float* y_dev) {
     int rc = check_batch(n, batch);
     if (rc) return rc;
     RLG_HIP(n, hipSetDevice(n->device));
-    rc = forward(n, x_dev, batch, y_dev);
+    // without a hidden layer the one product reads x_dev while it writes: overlapping arrays take the copy
+    const size_t nx = batch * n->dims.front(), ny = batch * n->dims.back();
+    const bool overlap = nlayers(n) == 1 && (uintptr_t)x_dev < (uintptr_t)(y_dev + ny) && (uintptr_t)y_dev < (uintptr_t)(x_dev + nx);
+    float* const y = overlap ? n->act.back() : y_dev;
+    rc = forward(n, x_dev, batch, y);
     if (rc) return rc;
+    if (overlap)
+        RLG_HIP(n, hipMemcpyAsync(y_dev, y, ny * sizeof(float), hipMemcpyDeviceToDevice, n->stream));
     RLG_HIP(n, hipStreamSynchronize(n->stream));
     return RLG_OK;
 }
