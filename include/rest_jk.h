@@ -92,7 +92,8 @@ size_t rjk_ld_baspar(const rjk_ctx* ctx);
  * the context's own stream.  The stream must have default priority. */
 int rjk_set_stream(rjk_ctx* ctx, void* stream);
 int rjk_synchronize(rjk_ctx* ctx);
-/* Upper bound (bytes) for the K workspace; 0 = default (4 GiB). */
+/* Upper bound (bytes) for the workspace that K and the B build keep on the context; 0 = default (4 GiB).
+ * A build that needs more allocates it for the call. */
 int rjk_set_workspace_limit(rjk_ctx* ctx, size_t bytes);
 
 /* ---- B storage (replaces the SCF.rimatr / SCF.ri3fn fields,

@@ -9,8 +9,8 @@
 //      rocBLAS dgemm per slab into the padded [naux][ldb] layout.  Orbital shells beyond d:
 //      the slabs come from the host (OpenMP), slab k+1 beside the upload and GEMM of slab k.
 //
-// Matrices and slabs live in the context's grow-only workspace and the products use its
-// rocBLAS handle, so that a build allocates only what a first build of its size needs.
+// Within the workspace limit matrices and slabs live in the context's grow-only workspace and the products use
+// its rocBLAS handle, so that a build allocates only what a first build of its size needs.
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
 
@@ -38,6 +38,12 @@ struct Host {
     void* p = nullptr;
     ~Host() {
         if (p) (void)hipHostFree(p);
+    }
+};
+struct Blas {
+    rocblas_handle h = nullptr;
+    ~Blas() {
+        if (h) rocblas_destroy_handle(h);
     }
 };
 struct GpuInts {
@@ -468,18 +474,41 @@ extern "C" int rsi_build_rimatr(rjk_ctx* ctx, const rsi_basis* orb, const rsi_ba
         const int r = rsi::gpu3c_init(&g.g, dev3 ? orb : nullptr, *aux, dev3 ? cuts : std::vector<size_t>(), st);
         if (r) return rjk::fail(ctx, r, "rsi_build_rimatr: device integral set-up failed");
     }
-    // workspace: [U | V^{-1/2} | λ | E | w | info | the metric's scratch, then the X slab of the device route]
+    // Matrices: U; V^{-1/2} with λ, E, w and info behind it; the metric's scratch, then the X slab of the device
+    // route.  Within the workspace limit they are the context's workspace, which the next build finds again.
+    // Beyond it, or where that much memory is not to be had, each is an allocation of its own for as
+    // long as it is needed, and without room for the metric's scratch the eigenpairs serve.
     const size_t nn = rjk::round_up(naux * naux * sizeof(double), 256), nv = rjk::round_up(naux * sizeof(double), 256);
-    void* ws = nullptr;
-    rc = rjk::ws_get(ctx, 2 * nn + 3 * nv + 256 + std::max(metric_bytes(naux), dev3 ? maxq * naux * sizeof(double) : 0), &ws);
-    if (rc) return rc;
-    double* dU = (double*)ws;
-    double* dVm = (double*)((char*)ws + nn);
-    double* dlam = (double*)((char*)ws + 2 * nn);
+    const size_t vbytes = nn + 3 * nv + 256, xbytes = dev3 ? maxq * naux * sizeof(double) : 0;
+    const size_t need = nn + vbytes + std::max(metric_bytes(naux), xbytes);
+    Dev tU, tV, tS, tX;
+    const auto temp = [](Dev& d, size_t bytes) {
+        if (hipMalloc(&d.p, bytes) == hipSuccess) return true;
+        (void)hipGetLastError();
+        d.p = nullptr;
+        return false;
+    };
+    void *ws = nullptr, *dU_ = nullptr, *dV_ = nullptr, *dS = nullptr, *dX_ = nullptr;
+    const std::string err = ctx->err;
+    if (need <= std::max(ctx->ws_limit, ctx->ws_size) && rjk::ws_get(ctx, need, &ws) == RJK_OK) {
+        dU_ = ws;
+        dV_ = (char*)ws + nn;
+        dS = dX_ = (char*)dV_ + vbytes;
+    } else {
+        ctx->err = err;
+        if (!temp(tU, nn) || !temp(tV, vbytes))
+            return rjk::fail(ctx, RJK_ERR_NOMEM, "rsi_build_rimatr: device allocation of the metric failed");
+        (void)temp(tS, metric_bytes(naux));
+        dU_ = tU.p;
+        dV_ = tV.p;
+        dS = tS.p;
+    }
+    double* dU = (double*)dU_;
+    double* dVm = (double*)dV_;
+    double* dlam = (double*)((char*)dV_ + nn);
     double* dE = (double*)((char*)dlam + nv);
     double* dw = (double*)((char*)dE + nv);
     rocblas_int* dinfo = (rocblas_int*)((char*)dw + nv);
-    double* dX = (double*)((char*)dinfo + 256);
 
     // ---- V^{-1/2} ----------------------------------------------------------
     double t0 = now();
@@ -495,10 +524,15 @@ extern "C" int rsi_build_rimatr(rjk_ctx* ctx, const rsi_basis* orb, const rsi_ba
     }
     size_t kept = naux;
     bool polar = false;
-    rc = metric_polar(ctx, h, st, naux, thr, dU, dX, dVm, &polar);
+    if (dS) rc = metric_polar(ctx, h, st, naux, thr, dU, dS, dVm, &polar);
     if (rc) return rc;
+    if (tS.p) (void)hipFree(std::exchange(tS.p, nullptr));
     if (!polar) {
-        RSI_BLAS(ctx, rocsolver_dsyevd(h, rocblas_evect_original, rocblas_fill_upper, (rocblas_int)naux, dU,
+        // a handle of its own: the eigensolver's workspace goes with it
+        Blas own;
+        RSI_BLAS(ctx, rocblas_create_handle(&own.h));
+        RSI_BLAS(ctx, rocblas_set_stream(own.h, st));
+        RSI_BLAS(ctx, rocsolver_dsyevd(own.h, rocblas_evect_original, rocblas_fill_upper, (rocblas_int)naux, dU,
                                        (rocblas_int)naux, dlam, dE, dinfo));
         std::vector<double> lam(naux), w(naux);
         int info = 0;
@@ -520,12 +554,13 @@ extern "C" int rsi_build_rimatr(rjk_ctx* ctx, const rsi_basis* orb, const rsi_ba
                            (const double*)dw);
         RSI_HIP(ctx, hipGetLastError());
         const double one_ = 1.0, zero_ = 0.0;
-        RSI_BLAS(ctx, rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_transpose, (rocblas_int)naux,
+        RSI_BLAS(ctx, rocblas_dgemm(own.h, rocblas_operation_none, rocblas_operation_transpose, (rocblas_int)naux,
                                     (rocblas_int)naux, (rocblas_int)naux, &one_, dU, (rocblas_int)naux, dU,
                                     (rocblas_int)naux, &zero_, dVm, (rocblas_int)naux));
         RSI_HIP(ctx, hipStreamSynchronize(st));   // w is a host temporary
     }
     if (nkept) *nkept = kept;
+    if (tU.p) (void)hipFree(std::exchange(tU.p, nullptr));
     t_v = now() - t0;
 
     // the padding of the columns; the slabs' products write the rest
@@ -536,6 +571,9 @@ extern "C" int rsi_build_rimatr(rjk_ctx* ctx, const rsi_basis* orb, const rsi_ba
     int status = RJK_OK;
     if (dev3) {
         // device integrals: slab k's kernels and GEMM follow each other on the stream
+        if (!dX_ && !temp(tX, xbytes))
+            return rjk::fail(ctx, RJK_ERR_NOMEM, "rsi_build_rimatr: device allocation of the integral slab failed");
+        double* const dX = (double*)(dX_ ? dX_ : tX.p);
         int r = RJK_OK;
         std::vector<hipEvent_t> ev(2 * (cuts.size() - 1), nullptr);
         for (auto& e : ev) RSI_HIP(ctx, hipEventCreate(&e));
