@@ -823,8 +823,7 @@ int vk_dm_device(rjk_ctx* ctx, const void* b, const double* dm_dev, size_t spin_
     if (rc) return rc;
     hipStream_t st = ctx->stream;
     const bool chol = prec == RJK_PREC_FP64 && nbf <= 4096;
-    // columns worth finding: beyond 256 functions a step is one launch (5 us), and a quarter of the
-    // functions bounds what a D of higher rank costs in vain to a few percent of its eigenproblem
+    // columns worth finding: beyond 256 functions a step is one launch (5 us; 2 us once D is given up)
     const size_t kmax = std::min(nbf <= 256 ? std::max<size_t>(1, nbf / 2) : nbf / 4 + 64, kCholMaxRank);
     const size_t nb32 = (nbf + 31) / 32;
     const unsigned nblk = asym_stats_blocks(nbf);
@@ -838,7 +837,7 @@ int vk_dm_device(rjk_ctx* ctx, const void* b, const double* dm_dev, size_t spin_
     const size_t i_sel = cv.add(spin_channel * nbf * sizeof(double));
     const size_t i_idx = cv.add(spin_channel * nbf * sizeof(int));
     const size_t i_info = cv.add(sizeof(int));
-    const size_t i_blk = cv.add((nb32 * nb32 + 2) * sizeof(double));
+    const size_t i_blk = cv.add((nb32 * nb32 + 3) * sizeof(double));
     void* aux = nullptr;
     rc = buf_get(ctx, &ctx->aux, &ctx->aux_size, cv.total, &aux);
     if (rc) return rc;

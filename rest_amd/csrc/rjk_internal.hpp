@@ -188,7 +188,7 @@ unsigned asym_stats_blocks(size_t nbf);
 hipError_t launch_asym_stats(hipStream_t st, const double* dm, size_t nbf, double* out);
 // pivoted Cholesky factor of a symmetric positive semidefinite D, at most kmax columns L[k][nbf]; rank
 // (−1: not such a D, or more columns) and the largest element D leaves out, on the device.  diag: 2·nbf
-// doubles, blockmax: ceil(nbf / 32)² + 2
+// doubles, blockmax: ceil(nbf / 32)² + 3
 constexpr size_t kCholMaxRank = 1024;
 hipError_t launch_pivot_chol(hipStream_t st, const double* dm, size_t nbf, size_t kmax, double cut, double* diag, double* L,
                              int* rank, double* blockmax, double* residual);

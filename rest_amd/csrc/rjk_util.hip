@@ -161,6 +161,15 @@ __global__ void k_pack_upper(const double* __restrict__ g, size_t nbf, size_t ld
 // LDS as well, the products of a row are split over 1024 / nbf threads.
 // Stops when the largest remaining diagonal is at most cut·max diag(D); rank -> out[0], or -1 if a
 // diagonal falls below −cut·max (D is not positive semidefinite) or kmax columns do not suffice.
+// A D that will need more is given up early, so that an attempt in vain stays a small part of the eigenpairs
+// that follow it (nbf 256, eigenvalues 0.1 to 1: 128 columns in vain 0.8 ms of 7.9, given up after 8 7.1):
+//   a tail: the largest remaining diagonal below kCholTail of the first but above the cut (the last pivots
+//     of low-rank densities are 3% of the first or more);
+//   the columns so far extrapolated: k of them that take the share f of the trace need k/f in all or more,
+//     since later pivots take less (random and molecular densities of rank r: k/f <= r throughout).
+constexpr double kCholTail = 1e-4;
+constexpr int kCholProbe = 8;        // column after which the rank is extrapolated,
+constexpr int kCholProbeMin = 56;    // unless kmax is below this: so few columns cost little
 constexpr int kCholThreads = 1024;
 constexpr size_t kCholSmall = 256;   // largest nbf of the one-work-group kernel
 constexpr int kCholLds = 16384;   // doubles of L kept in LDS
@@ -179,9 +188,24 @@ __global__ __launch_bounds__(kCholThreads) void k_pivot_chol(const double* __res
     const int row = tid / G, q = tid % G;
     for (int i = tid; i < n; i += kCholThreads) dg[i] = dm[(size_t)i * n + i];
     __syncthreads();
-    double d0 = 0.0;
+    double d0 = 0.0, trace0 = 0.0;
     int rank = -1;
+    const auto trace = [&]() {
+        double s = tid < n ? dg[tid] : 0.0;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        if (lane == 0) part[wave] = s;
+        __syncthreads();
+        s = part[lane & 15];
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        __syncthreads();
+        return s;
+    };
+    const bool probe = kmax >= kCholProbeMin;
+    if (probe) trace0 = trace();
     for (int k = 0;; ++k) {
+        if (probe && k == kCholProbe && k * trace0 > kmax * (trace0 - trace())) break;
         double mx = -INFINITY, mn = INFINITY;
         int at = 0;
         for (int i = tid; i < n; i += kCholThreads) {
@@ -229,7 +253,7 @@ __global__ __launch_bounds__(kCholThreads) void k_pivot_chol(const double* __res
             rank = k;
             break;
         }
-        if (k == kmax) break;
+        if (k == kmax || top < kCholTail * d0) break;
         // D's column is on its way while row p of L is gathered and multiplied
         const double dcol = q == 0 && row < n ? 0.5 * (dm[(size_t)p * n + row] + dm[(size_t)row * n + p]) : 0.0;
         for (int j = tid; j < k; j += kCholThreads) lp[j] = j < klds ? ls[j * n + p] : L[(size_t)j * n + p];
@@ -277,7 +301,7 @@ __global__ void k_chol_start(const double* __restrict__ dm, int n, double* __res
 __global__ __launch_bounds__(256) void k_chol_step(const double* __restrict__ dm, int n, int k, int kmax, double cut,
                                                    double* __restrict__ diag, double* __restrict__ top0,
                                                    double* __restrict__ L, int* __restrict__ out) {
-    __shared__ double wmax[4], wmin[4], part[256], lp[kCholMaxRank];
+    __shared__ double wmax[4], wmin[4], wsum[4], part[256], lp[kCholMaxRank];
     __shared__ int widx[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (out[k & 1] != -2) {   // finished in an earlier launch (uniform): hand the verdict on
@@ -285,10 +309,11 @@ __global__ __launch_bounds__(256) void k_chol_step(const double* __restrict__ dm
         return;
     }
     const double* __restrict__ din = diag + (size_t)(k & 1) * n;
-    double mx = -INFINITY, mn = INFINITY;
+    double mx = -INFINITY, mn = INFINITY, sum = 0.0;
     int at = 0;
     for (int i = tid; i < n; i += 256) {
         const double d = din[i];
+        sum += d;
         if (d > mx) {
             mx = d;
             at = i;
@@ -304,10 +329,12 @@ __global__ __launch_bounds__(256) void k_chol_step(const double* __restrict__ dm
             at = a2;
         }
         mn = fmin(mn, __shfl_xor(mn, o, 64));
+        sum += __shfl_xor(sum, o, 64);
     }
     if (lane == 0) {
         wmax[wave] = mx;
         wmin[wave] = mn;
+        wsum[wave] = sum;
         widx[wave] = at;
     }
     __syncthreads();
@@ -322,11 +349,17 @@ __global__ __launch_bounds__(256) void k_chol_step(const double* __restrict__ dm
     }
     const double d0 = k == 0 ? top : top0[0];
     const bool bad = low < -cut * d0 || !(top >= 0.0), done = top <= cut * d0;
+    sum = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+    const bool over = k == kmax || top < kCholTail * d0 ||
+                      (k == kCholProbe && k * top0[1] > kmax * (top0[1] - sum));
     if (blockIdx.x == 0 && tid == 0) {
-        if (k == 0) top0[0] = top;
-        out[(k + 1) & 1] = bad ? -1 : (done ? k : (k == kmax ? -1 : -2));   // the next launch's state
+        if (k == 0) {
+            top0[0] = top;
+            top0[1] = sum;
+        }
+        out[(k + 1) & 1] = bad ? -1 : (done ? k : (over ? -1 : -2));   // the next launch's state
     }
-    if (bad || done || k == kmax) return;   // uniform over the grid
+    if (bad || done || over) return;   // uniform over the grid
     for (int j = tid; j < k; j += 256) lp[j] = L[(size_t)j * n + p];
     __syncthreads();
     const int i = blockIdx.x * kCholRows + lane;
