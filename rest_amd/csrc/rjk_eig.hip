@@ -529,7 +529,7 @@ __global__ __launch_bounds__(256) void k_eig_mul(const double* __restrict__ Z, c
         if (ii < n && jj < n) {
             if (GRAM) {
                 const double one = ii == jj ? 1.0 : 0.0, dev = fabs(acc[r] - one);
-                m = dev <= m ? m : dev;   // a NaN stays
+                m = max_nan(m, dev);
                 out[(size_t)jj * n + ii] = 1.5 * one - 0.5 * acc[r];
             } else {
                 out[(size_t)jj * n + ii] = acc[r];
@@ -537,14 +537,11 @@ __global__ __launch_bounds__(256) void k_eig_mul(const double* __restrict__ Z, c
         }
     }
     if (!GRAM) return;
-    for (int o = 32; o > 0; o >>= 1) {
-        const double m2 = __shfl_xor(m, o, 64);
-        m = m2 <= m ? m : m2;
-    }
+    for (int o = 32; o > 0; o >>= 1) m = max_nan(m, __shfl_xor(m, o, 64));
     if (lane == 0) red[wave] = m;
     __syncthreads();
     if (threadIdx.x) return;
-    for (int q = 1; q < 4; ++q) m = red[q] <= m ? m : red[q];
+    for (int q = 1; q < 4; ++q) m = max_nan(m, red[q]);
     part[blockIdx.y * gridDim.x + blockIdx.x] = m;
 }
 

@@ -15,6 +15,12 @@ struct _rocblas_handle;   // rocblas_handle is _rocblas_handle*
 
 namespace rjk {
 
+// the larger of the two, NaN if either is: the maxima that decide whether a result is good must not lose one
+__host__ __device__ constexpr double max_nan(double a, double b) { return a >= b || a != a ? a : b; }
+static_assert(max_nan(1.0, 2.0) == 2.0 && max_nan(2.0, 1.0) == 2.0, "maximum");
+static_assert(max_nan(__builtin_nan(""), 1.0) != max_nan(__builtin_nan(""), 1.0), "NaN first");
+static_assert(max_nan(1.0, __builtin_nan("")) != max_nan(1.0, __builtin_nan("")), "NaN second");
+
 constexpr size_t kFp32Chain = 4096;   // products per FP32 accumulator in the K SYRK before FP64
 constexpr size_t kLdAlign = 64;      // elements; device B columns start 512-B aligned (FP64)
 constexpr int kNumPhases = 5;        // J-gamma, J-acc, K-half, K-syrk, K-other

@@ -412,12 +412,12 @@ __global__ __launch_bounds__(256) void k_chol_residual(const double* __restrict_
     if (bi <= bj)
         for (int q = 0; q < 4; ++q) {
             const int i = bi + x, j = bj + y + 8 * q;
-            if (i < n && j < n) m = fmax(m, fabs(0.5 * (dm[(size_t)j * n + i] + dm[(size_t)i * n + j]) - acc[q]));
+            if (i < n && j < n) m = max_nan(m, fabs(0.5 * (dm[(size_t)j * n + i] + dm[(size_t)i * n + j]) - acc[q]));
         }
     red[threadIdx.x] = m;
     __syncthreads();
     for (int h = 128; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + h]);
+        if ((int)threadIdx.x < h) red[threadIdx.x] = max_nan(red[threadIdx.x], red[threadIdx.x + h]);
         __syncthreads();
     }
     if (threadIdx.x == 0) out[blockIdx.y * gridDim.x + blockIdx.x] = red[0];
@@ -427,11 +427,11 @@ __global__ __launch_bounds__(256) void k_chol_residual(const double* __restrict_
 __global__ __launch_bounds__(256) void k_max(const double* __restrict__ x, int n, double* __restrict__ out) {
     __shared__ double red[256];
     double m = 0.0;
-    for (int i = threadIdx.x; i < n; i += 256) m = fmax(m, x[i]);
+    for (int i = threadIdx.x; i < n; i += 256) m = max_nan(m, x[i]);
     red[threadIdx.x] = m;
     __syncthreads();
     for (int h = 128; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + h]);
+        if ((int)threadIdx.x < h) red[threadIdx.x] = max_nan(red[threadIdx.x], red[threadIdx.x + h]);
         __syncthreads();
     }
     if (threadIdx.x == 0) out[0] = red[0];

@@ -287,17 +287,14 @@ __global__ __launch_bounds__(256) void k_met_step(double* __restrict__ G, int n,
     for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < (size_t)n * n; t += (size_t)gridDim.x * 256) {
         const bool d = t / n == t % n;
         const double g = G[t], e = fabs(g - (d ? 1.0 : 0.0));
-        m = e <= m ? m : e;   // a NaN stays
+        m = rjk::max_nan(m, e);
         G[t] = (d ? a : 0.0) - b * g;
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        const double e = __shfl_xor(m, o, 64);
-        m = e <= m ? m : e;
-    }
+    for (int o = 32; o > 0; o >>= 1) m = rjk::max_nan(m, __shfl_xor(m, o, 64));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < 4; ++w) m = red[w] <= m ? m : red[w];
+        for (int w = 1; w < 4; ++w) m = rjk::max_nan(m, red[w]);
         part[blockIdx.x] = m;
     }
 }
@@ -420,7 +417,7 @@ int metric_polar(rjk_ctx* ctx, rocblas_handle h, hipStream_t st, size_t n, doubl
     RSI_HIP(ctx, hipStreamSynchronize(st));
     double dev = 0.0, norm2 = 0.0;
     for (unsigned k = 0; k < parts; ++k) {
-        dev = pt[k] <= dev ? dev : pt[k];      // of the last step's XᵀX from one
+        dev = rjk::max_nan(dev, pt[k]);        // of the last step's XᵀX from one
         norm2 += pt[kMetParts + k];
     }
     // 1/‖V^{-1/2}‖² is at most V's smallest eigenvalue: above thr, the eigenpairs would all be kept
