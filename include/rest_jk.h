@@ -200,6 +200,20 @@ int rjk_profile_read(rjk_ctx* ctx, double* ms, uint64_t* launches);
  * (2·nbf²·nk·P per half-transform, nbf(nbf+1)·nk·P per SYRK), 0 for phase 4.
  * Resets the counters like rjk_profile_read. */
 int rjk_profile_read_detail(rjk_ctx* ctx, double* ms, uint64_t* launches, double* work);
+/* How often this context took each of its solvers, and what it falls back to: a result alone does not
+ * tell, since every route ends in the same numbers to rounding.  counts[RJK_NUM_ROUTES]. */
+enum {
+    RJK_ROUTE_DM_CHOLESKY = 0, /* density-only K on the columns of a Cholesky factor            */
+    RJK_ROUTE_DM_EIGENPAIRS,   /*   on eigenpairs (rocSOLVER)                                   */
+    RJK_ROUTE_DM_GENERAL,      /*   of a D that is not symmetric                                */
+    RJK_ROUTE_EIG_OWN,         /* SCF eigenproblem by the library's own kernels                 */
+    RJK_ROUTE_EIG_DIVIDE,      /*   handed on to divide and conquer on the same tridiagonal     */
+    RJK_ROUTE_EIG_ROCSOLVER,   /*   of a size that goes to rocSOLVER at once                    */
+    RJK_ROUTE_METRIC_POLAR,    /* B build with V^{-1/2} from the polar factor                   */
+    RJK_ROUTE_METRIC_EIGENPAIRS, /* from V's eigenpairs (rocSOLVER)                             */
+    RJK_NUM_ROUTES
+};
+int rjk_route_counts(const rjk_ctx* ctx, uint64_t* counts);
 /* A plain device copy of `bytes` bytes (HBM-traffic calibration for counters). */
 int rjk_copy_dev(rjk_ctx* ctx, void* dst_dev, const void* src_dev, size_t bytes);
 

@@ -879,6 +879,7 @@ int vk_dm_device(rjk_ctx* ctx, const void* b, const double* dm_dev, size_t spin_
             else ncol[s] = (size_t)rank;
         }
     }
+    ++ctx->routes[general ? RJK_ROUTE_DM_GENERAL : (low_rank ? RJK_ROUTE_DM_CHOLESKY : RJK_ROUTE_DM_EIGENPAIRS)];
     if (general) return vk_dm_general(ctx, dm_dev, ns, scaling_factor, vk_dev);
     if (low_rank) {
         KPlan kp;
@@ -1002,6 +1003,12 @@ extern "C" int rjk_vk_upper_with_ri_v_use_dm_only_sync(rjk_ctx* ctx, const doubl
 extern "C" int rjk_profile_enable(rjk_ctx* ctx, int on) {
     if (!ctx) return RJK_ERR_ARG;
     ctx->prof = on != 0;
+    return RJK_OK;
+}
+
+extern "C" int rjk_route_counts(const rjk_ctx* ctx, uint64_t* counts) {
+    if (!ctx || !counts) return RJK_ERR_ARG;
+    std::copy(ctx->routes, ctx->routes + RJK_NUM_ROUTES, counts);
     return RJK_OK;
 }
 

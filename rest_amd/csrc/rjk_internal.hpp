@@ -69,6 +69,7 @@ struct rjk_ctx {
     double* scf_x = nullptr;          // SCF driver: orthogonaliser S^-1/2 of the last S seen
     std::vector<double> scf_s;        // that S (host copy, compared before reuse)
     std::string err;
+    uint64_t routes[RJK_NUM_ROUTES] = {};
     // phase timing
     bool prof = false;
     double prof_ms[rjk::kNumPrec][rjk::kNumPhases] = {};     // [RJK_PREC_*][phase]

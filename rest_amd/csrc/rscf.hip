@@ -553,6 +553,7 @@ int scf_core(rjk_ctx* ctx, const char* who, const double* S_h, const double* H_h
     // the same tridiagonal matrix.  dsyevd at n 192: 3863 us, here 526 (1690 with divide and conquer); n 336: 7.0 ms, here 2.2.
     auto eigen = [&](double* M, double* w, double** vec) -> int {
         *vec = eigws ? T1 : M;
+        ++ctx->routes[eigws ? RJK_ROUTE_EIG_OWN : RJK_ROUTE_EIG_ROCSOLVER];
         if (eigws) SCF_HIP(rjk::launch_eig(st, M, n, w, T1, eigws, (int*)info_d));
         else
             SCF_BLAS(rocsolver_dsyevd(h, rocblas_evect_original, rocblas_fill_upper, (rocblas_int)n, M, (rocblas_int)n, w,
@@ -560,6 +561,8 @@ int scf_core(rjk_ctx* ctx, const char* who, const double* S_h, const double* H_h
         return RJK_OK;
     };
     auto eigen_again = [&](double* w, double* vec) -> int {
+        --ctx->routes[RJK_ROUTE_EIG_OWN];
+        ++ctx->routes[RJK_ROUTE_EIG_DIVIDE];
         SCF_HIP(hipMemcpyAsync(w, eigws, n * sizeof(double), hipMemcpyDeviceToDevice, st));
         SCF_HIP(hipMemcpyAsync(Ework, eigws + n, n * sizeof(double), hipMemcpyDeviceToDevice, st));
         SCF_BLAS(rocsolver_dstedc(h, rocblas_evect_tridiagonal, (rocblas_int)n, w, Ework, vec, (rocblas_int)n,

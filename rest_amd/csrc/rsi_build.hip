@@ -523,6 +523,7 @@ extern "C" int rsi_build_rimatr(rjk_ctx* ctx, const rsi_basis* orb, const rsi_ba
     bool polar = false;
     if (dS) rc = metric_polar(ctx, h, st, naux, thr, dU, dS, dVm, &polar);
     if (rc) return rc;
+    ++ctx->routes[polar ? RJK_ROUTE_METRIC_POLAR : RJK_ROUTE_METRIC_EIGENPAIRS];
     if (tS.p) (void)hipFree(std::exchange(tS.p, nullptr));
     if (!polar) {
         // a handle of its own: the eigensolver's workspace goes with it

@@ -48,6 +48,7 @@ EXPORTS = [
     "rjk_vj_upper_with_rimatr_v_sync", "rjk_vj_upper_with_ri_v_sync", "rjk_vj_upper_dev", "rjk_vj_upper_dev_noalloc",
     "rjk_vk_upper_with_ri_v_sync", "rjk_vk_upper_occ_dev", "rjk_vk_upper_with_rimatr_use_dm_only_sync",
     "rjk_vk_upper_with_ri_v_use_dm_only_sync", "rjk_vk_upper_dm_dev", "rjk_profile_enable", "rjk_profile_read", "rjk_profile_read_detail", "rjk_copy_dev",
+    "rjk_route_counts",
     # include/rest_ri.h
     "rsi_basis_create", "rsi_basis_destroy", "rsi_basis_nbf", "rsi_last_error", "rsi_int1e", "rsi_int2c2e",
     "rsi_int3c2e_packed", "rsi_int3c2e_packed_dev", "rsi_build_rimatr", "rsi_cart2sph",
@@ -122,6 +123,7 @@ def load_library(path: Optional[Path] = None) -> C.CDLL:
         "rjk_profile_read": (i, [vp, pd, C.POINTER(C.c_uint64)]),
         "rjk_profile_read_detail": (i, [vp, pd, C.POINTER(C.c_uint64), pd]),
         "rjk_copy_dev": (i, [vp, vp, vp, sz]),
+        "rjk_route_counts": (i, [vp, vp]),
         "rsi_basis_create": (i, [sz, vp, vp, vp, vp, vp, sz, vp, C.POINTER(vp)]),
         "rsi_basis_destroy": (i, [vp]),
         "rsi_basis_nbf": (sz, [vp]),
@@ -346,6 +348,15 @@ class DeviceRI:
         return {(p, name): (ms[5 * pi + k], int(n[5 * pi + k]), w[5 * pi + k])
                 for pi, p in enumerate(("fp64", "fp32", "bf16x2", "bf16x3", "bf16x1"))
                 for k, name in enumerate(self.PHASES)}
+
+    ROUTES = ("dm_cholesky", "dm_eigenpairs", "dm_general", "eig_own", "eig_divide", "eig_rocsolver", "metric_polar",
+              "metric_eigenpairs")
+
+    def route_counts(self) -> dict:
+        """How often the context took each of its solvers and their fallbacks (rjk_route_counts)."""
+        n = (C.c_uint64 * len(self.ROUTES))()
+        self._check(self.lib.rjk_route_counts(self.h, n))
+        return {name: int(v) for name, v in zip(self.ROUTES, n)}
 
     def copy_dev(self, dst_ptr: int, src_ptr: int, nbytes: int):
         self._check(self.lib.rjk_copy_dev(self.h, C.c_void_p(dst_ptr), C.c_void_p(src_ptr), int(nbytes)))
