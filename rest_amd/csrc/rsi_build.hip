@@ -72,7 +72,7 @@ __global__ void k_scale_cols(double* U, int n, const double* w) {
 // pivots take 3.5, the 19 steps' products 4.0 (47 TFLOP/s), the updates 0.9, the triangular solve 0.5.
 constexpr int kMetBlock = 64;      // pivots between updates of the whole remainder
 constexpr int kMetRows = 64;       // rows of a work-group in one pivot's step
-constexpr double kMetCut = 1e-13;  // smallest pivot relative to the largest
+constexpr double kMetCut = 1e-13;  // smallest pivot relative to the largest (a pivot up to thr ends it too: V's least eigenvalue is no larger)
 constexpr int kMetParts = 1024;    // partial results of a reduction
 
 __global__ __launch_bounds__(256) void k_met_rowsum(const double* __restrict__ V, int n, double* __restrict__ out,
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(256) void k_met_rowsum(const double* __restrict__ V
 // Pivot k, the block's first being k0: S holds V less the blocks before.  Every work-group finds the pivot in
 // diag[k % 2] by itself (NaN marks a row that has been one) and writes its rows' diagonals to the other
 // half; state[k % 2] is what launch k finds: −2 running, else stopped at that rank.
-__global__ __launch_bounds__(256) void k_met_pivot(const double* __restrict__ S, int n, int k, int k0,
+__global__ __launch_bounds__(256) void k_met_pivot(const double* __restrict__ S, int n, int k, int k0, double thr,
                                                    double* __restrict__ diag, double* __restrict__ top0,
                                                    double* __restrict__ L, int* __restrict__ piv,
                                                    int* __restrict__ state) {
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void k_met_pivot(const double* __restrict__ S,
             p = widx[w];
         }
     const double d0 = k == 0 ? top : top0[0];
-    const bool stop = !(top > kMetCut * d0) || !(top < INFINITY);
+    const bool stop = !(top > kMetCut * d0 && top > thr) || !(top < INFINITY);
     if (blockIdx.x == 0 && tid == 0) {
         if (k == 0) top0[0] = top;
         piv[k] = p;
@@ -177,7 +177,7 @@ template <class F, int... U>
 __device__ __forceinline__ void steps(const F& f, std::integer_sequence<int, U...>) {
     (void)(f(std::integral_constant<int, U>()) && ...);   // in order, until one says no; u a constant in each
 }
-__global__ __launch_bounds__(1024) void k_met_panel(const double* __restrict__ S, int n, int k0, int kb,
+__global__ __launch_bounds__(1024) void k_met_panel(const double* __restrict__ S, int n, int k0, int kb, double thr,
                                                     double* __restrict__ diag, double* __restrict__ top0,
                                                     double* __restrict__ L, int* __restrict__ piv,
                                                     int* __restrict__ state) {
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(1024) void k_met_panel(const double* __restrict__ S
             d0 = mx;
             if (tid == 0) top0[0] = mx;
         }
-        if (!(mx > kMetCut * d0) || !(mx < INFINITY)) {   // uniform over the work-group
+        if (!(mx > kMetCut * d0 && mx > thr) || !(mx < INFINITY)) {   // uniform over the work-group
             if (tid == 0) state[0] = k0 + u;
             return false;
         }
@@ -364,11 +364,11 @@ int metric_polar(rjk_ctx* ctx, rocblas_handle h, hipStream_t st, size_t n, doubl
     for (size_t k0 = 0; k0 < n; k0 += block) {
         const size_t k1 = std::min(n, k0 + block);
         if (panel)
-            hipLaunchKernelGGL(k_met_panel, dim3(1), dim3(1024), 0, st, S, (int)n, (int)k0, (int)(k1 - k0), diag, top0, L, piv,
+            hipLaunchKernelGGL(k_met_panel, dim3(1), dim3(1024), 0, st, S, (int)n, (int)k0, (int)(k1 - k0), thr, diag, top0, L, piv,
                                state);
         for (size_t k = panel ? k1 : k0; k < k1; ++k)
             hipLaunchKernelGGL(k_met_pivot, dim3((unsigned)((n + kMetRows - 1) / kMetRows)), dim3(256), 0, st, S, (int)n, (int)k,
-                               (int)k0, diag, top0, L, piv, state);
+                               (int)k0, thr, diag, top0, L, piv, state);
         if (k1 < n)
             RSI_BLAS(ctx, rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_transpose, ni, ni,
                                         (rocblas_int)(k1 - k0), &minus, L + k0 * n, ni, L + k0 * n, ni, &one, S, ni));
@@ -526,11 +526,16 @@ extern "C" int rsi_build_rimatr(rjk_ctx* ctx, const rsi_basis* orb, const rsi_ba
     ++ctx->routes[polar ? RJK_ROUTE_METRIC_POLAR : RJK_ROUTE_METRIC_EIGENPAIRS];
     if (tS.p) (void)hipFree(std::exchange(tS.p, nullptr));
     if (!polar) {
-        // a handle of its own: the eigensolver's workspace goes with it
+        // the eigensolver's workspace, a few matrices, stays with its handle: a large one gets a handle of its own (up
+        // to 2147 functions the 128 MiB that any handle holds are enough; a handle takes 0.4 ms to make)
         Blas own;
-        RSI_BLAS(ctx, rocblas_create_handle(&own.h));
-        RSI_BLAS(ctx, rocblas_set_stream(own.h, st));
-        RSI_BLAS(ctx, rocsolver_dsyevd(own.h, rocblas_evect_original, rocblas_fill_upper, (rocblas_int)naux, dU,
+        rocblas_handle hs = h;
+        if (nn > size_t(32) << 20) {
+            RSI_BLAS(ctx, rocblas_create_handle(&own.h));
+            RSI_BLAS(ctx, rocblas_set_stream(own.h, st));
+            hs = own.h;
+        }
+        RSI_BLAS(ctx, rocsolver_dsyevd(hs, rocblas_evect_original, rocblas_fill_upper, (rocblas_int)naux, dU,
                                        (rocblas_int)naux, dlam, dE, dinfo));
         std::vector<double> lam(naux), w(naux);
         int info = 0;
@@ -552,7 +557,7 @@ extern "C" int rsi_build_rimatr(rjk_ctx* ctx, const rsi_basis* orb, const rsi_ba
                            (const double*)dw);
         RSI_HIP(ctx, hipGetLastError());
         const double one_ = 1.0, zero_ = 0.0;
-        RSI_BLAS(ctx, rocblas_dgemm(own.h, rocblas_operation_none, rocblas_operation_transpose, (rocblas_int)naux,
+        RSI_BLAS(ctx, rocblas_dgemm(hs, rocblas_operation_none, rocblas_operation_transpose, (rocblas_int)naux,
                                     (rocblas_int)naux, (rocblas_int)naux, &one_, dU, (rocblas_int)naux, dU,
                                     (rocblas_int)naux, &zero_, dVm, (rocblas_int)naux));
         RSI_HIP(ctx, hipStreamSynchronize(st));   // w is a host temporary

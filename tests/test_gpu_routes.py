@@ -104,3 +104,22 @@ def test_metric_routes(waters):
             m.build_rimatr(r, threshold=share * lam[0])
             polar += 1.0 / (1.0 / lam).sum() > share * lam[0]
         assert taken(r) == {"metric_polar": polar, "metric_eigenpairs": 3 - polar} and polar < 3
+
+
+@pytest.mark.parametrize("waters,share", [(1, 0.1), (2, 0.5), (5, 0.02), (19, 0.3)])
+def test_threshold_among_the_eigenvalues(waters, share):
+    """A threshold above that share of the eigenvalues ends the factor at a pivot below it: the eigenpairs, and as
+    many of them as numpy keeps; B V^(1/2) = X P over the kept space to 1e-9."""
+    m = ri.Molecule.water_cluster(wl.water_cluster(3, waters))
+    lam, U = np.linalg.eigh(m.int2c2e())
+    cut = int(share * m.naux)
+    thr = float(np.sqrt(lam[cut - 1] * lam[cut]))
+    print(f"[gpu-case] metric of {m.naux} functions, threshold {thr:.2e} above {cut} eigenvalues", flush=True)
+    with jk.DeviceRI(m.nbf, m.naux) as r:
+        assert m.build_rimatr(r, threshold=thr)["naux_kept"] == m.naux - cut
+        assert taken(r) == {"metric_eigenpairs": 1}
+        if waters < 10:
+            X = m.int3c2e_packed()
+            kept = U[:, cut:]
+            d = r.get_rimatr() @ (kept * np.sqrt(lam[cut:])) @ kept.T - X @ kept @ kept.T
+            assert np.abs(d).max() <= 1e-9 * np.abs(X).max()
