@@ -65,9 +65,10 @@ __global__ void k_scale_cols(double* U, int n, const double* w) {
 // V = L Lᵀ by Cholesky with the largest remaining diagonal as pivot; the polar factor Q of Lᵀ by scaled
 // Newton–Schulz steps X ← X (a − b XᵀX) (Higham, Functions of Matrices, ch. 8); then Lᵀ = Q V^{1/2}
 // and V^{-1/2} = L^{-T} Q.  Singular values of Lᵀ are the square roots of V's eigenvalues, and pivoting
-// grades its rows, which every step's product on the right keeps: B of 2 to 5 waters errs by 2e-12 of
-// its norm against 80-bit arithmetic, by 3 to 7e-12 from the eigenpairs (from an unpivoted factor
-// 1 to 7e-11).  1356 auxiliary functions: 9.3 ms against 31 with dsyevd, whose tridiagonal reduction
+// grades its rows, which every step's product on the right keeps.  Against integrals and root in 80 bits B of
+// 1 to 3 waters errs by 0.2 to 0.8e-12 of its norm; from rocSOLVER's eigenpairs of the same V by 0.2 to 1.3e-12, of
+// the host's V, as before, by 0.7 to 1.7e-12 (V's own rounding is most of it; an unpivoted factor adds 1 to
+// 7e-11).  1356 auxiliary functions: 9.3 ms against 31 with dsyevd, whose tridiagonal reduction
 // is five dependent launches a column; 113: 1.2 against 2.4; 3164: 75 against 283.  Of the 9.3 ms the
 // pivots take 3.5, the 19 steps' products 4.0 (47 TFLOP/s), the updates 0.9, the triangular solve 0.5.
 constexpr int kMetBlock = 64;      // pivots between updates of the whole remainder
