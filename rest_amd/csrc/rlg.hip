@@ -28,7 +28,7 @@ struct rlg_net {
     float* adam_v = nullptr;
     std::vector<size_t> w_off, b_off;
     std::vector<float*> act;   // act[0] = input copy pointer (not owned), act[l+1] = layer l output
-    std::vector<float*> pre;   // pre-activation of every layer
+    std::vector<float*> pre;   // pre-activation of every hidden layer
     float* g0 = nullptr;       // backward activation gradients (ping-pong)
     float* g1 = nullptr;
     float* split = nullptr;    // split-K partials of the weight gradients
@@ -215,7 +215,7 @@ __global__ void k_loss_grad(const float* __restrict__ Y, const float* __restrict
 
 // out[i] = Σ_z part[z*count + i] for the weight gradient (i < count), then the bias gradient from
 // colsum[z*nb + i] (nb columns).  The bias gradient used to be one thread a column over the whole
-// batch: 937 of 1085 us a layer at batch 4096. 
+// batch: 937 of 1085 us a layer at batch 4096.
 __global__ void k_sum_splits(const float* __restrict__ part, const float* __restrict__ colsum, int splits, size_t count,
                              int nb, float* __restrict__ out) {
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -252,6 +252,8 @@ hipError_t gemm_t(hipStream_t st, const float* A, long sam, long sak, const floa
         return hipGetLastError();
     };
     const bool bk = sbk == 1 && sbn != 1;   // a one-column B keeps the path that forms column sums
+    if constexpr (EPI == EPI_SILU || EPI == EPI_LINEAR) return go(k_gemm<true, false, EPI>);   // forward: A's rows, W's rows
+    if constexpr (EPI == EPI_SILU_BWD) return bk ? go(k_gemm<true, true, EPI>) : go(k_gemm<true, false, EPI>);
     if (sak == 1) return bk ? go(k_gemm<true, true, EPI>) : go(k_gemm<true, false, EPI>);
     return bk ? go(k_gemm<false, true, EPI>) : go(k_gemm<false, false, EPI>);
 }
@@ -319,9 +321,10 @@ int rlg_create(int device, size_t n_in, size_t n_hidden, size_t n_hidden_layers,
     n->stream = n->own;
     ok = ok && alloc(&n->params, off) && alloc(&n->grads, off) && alloc(&n->adam_m, off) && alloc(&n->adam_v, off);
     n->act.assign(L + 1, nullptr);
-    n->pre.assign(L, nullptr);
+    n->pre.assign(L - 1, nullptr);
     for (int l = 0; l < L && ok; ++l) {
-        ok = alloc(&n->pre[l], max_batch * n->dims[l + 1]) && alloc(&n->act[l + 1], max_batch * n->dims[l + 1]);
+        ok = alloc(&n->act[l + 1], max_batch * n->dims[l + 1]);
+        if (l + 1 < L) ok = ok && alloc(&n->pre[l], max_batch * n->dims[l + 1]);
     }
     ok = ok && alloc(&n->g0, max_batch * widest) && alloc(&n->g1, max_batch * widest);
     ok = ok && hipMalloc((void**)&n->part, 2 * kLossBlocks * sizeof(double)) == hipSuccess;
