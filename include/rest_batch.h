@@ -42,7 +42,8 @@ extern "C" {
 typedef struct rjk_batch rjk_batch;
 
 /* Stages timed by rjk_batch_profile: 0 D weights, 1 γ, 2 J accumulation, 3 C' preparation,
- * 4 / 5 K half-transform (narrow / wide tile class; BF16: up to / above 32 columns a tile), 6 / 7 K SYRK (narrow / wide: 64- / 128-row tiles), 8 split reduction. */
+ * 4 / 5 K half-transform (narrow / wide tile class; BF16: up to / above 32 columns a tile),
+ * 6 / 7 K SYRK (narrow / wide: 64- / 128-row tiles), 8 split reduction. */
 #define RJK_BATCH_NUM_STAGES 9
 
 /* Device bytes rjk_batch_create allocates for these problems at precision prec (B, inputs,

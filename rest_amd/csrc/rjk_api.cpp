@@ -416,7 +416,6 @@ extern "C" int rjk_vj_upper_dev(rjk_ctx* ctx, const double* dm_dev, size_t spin_
 
 namespace {
 
-// staging of the host-pointer entry points: the context's grow-only io buffer
 // Host arrays of up to kPinBytes pass through pinned memory: from pageable memory every copy, up or down, is a
 // wait of its own in the runtime (a J and a K call, nbf 24: 64 us against 82; nbf 60: 88 against 106).  Larger
 // ones gain nothing (nbf 250, 500 kB: 587 against 590) and go directly.  The buffer is free again
@@ -454,6 +453,7 @@ int from_device(rjk_ctx* ctx, void* dst, const void* src, size_t bytes) {
     return RJK_OK;
 }
 
+// staging of the host-pointer entry points: the context's grow-only io buffer
 int io_get(rjk_ctx* ctx, size_t bytes, void** out) { return buf_get(ctx, &ctx->io, &ctx->io_size, bytes, out); }
 
 int check_host_finite(rjk_ctx* ctx, const double* x, size_t n, const char* what) {
@@ -809,8 +809,8 @@ int vk_dm_general(rjk_ctx* ctx, const double* dm_dev, int ns, double scale, doub
 // squares add up to (D + Dᵀ)/2; otherwise the general route above reads every D in full.  The
 // columns, per call:
 //   FP64, nbf <= 4096, D positive semidefinite of low rank (an SCF density has rank nocc):
-//     the pivoted Cholesky factor, unless it leaves out more than kCholTol·max|D| (nbf 192, rank
-//     40: 0.15 ms against 3 ms for the eigenpairs; nbf 1536, rank 320: 3 against 38);
+//     the pivoted Cholesky factor, unless it is given up (rjk_util.hip) or leaves out more than
+//     kCholTol·max|D| (nbf 192, rank 40: 0.15 ms against 3 ms for the eigenpairs; nbf 1536, rank 320: 3 against 38);
 //   else the eigenpairs with |λ| > kEigRelCut·max|λ| (rocSOLVER dsyevd), weights λ.
 // The lower precisions keep the eigenpairs: their K depends on the columns at its own rounding.
 int vk_dm_device(rjk_ctx* ctx, const void* b, const double* dm_dev, size_t spin_channel, double scaling_factor,

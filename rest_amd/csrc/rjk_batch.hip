@@ -55,9 +55,9 @@ struct BProb {
     double* gamma;        // [naux]
     double* vj;           // [npair]
     double* vk;           // [npair]
-    void* cocc;           // [nbf_pad][nk]; BF16: C'ᵀ planes [S][nk][nbf_pad]
+    void* cocc;           // [nbf_pad][nk]; BF16: C'ᵀ planes [S] of nk × nbf_pad as fragments (rjk_bftile.hpp)
     void* sign;           // [nk]; BF16: sign masks (0x8000 for a negative weight) [nk]
-    void* m;              // [naux][nk][nbf_pad]; BF16: M' planes [S][naux][nbf_pad][nk]
+    void* m;              // [naux][nk][nbf_pad]; BF16: M' planes [S][naux] of nbf_pad × nk as fragments
     double* kpart;        // [nsplit][nbf_pad][nbf_pad]
 };
 

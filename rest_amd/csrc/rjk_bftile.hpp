@@ -43,9 +43,8 @@ struct Cfg {
     static constexpr int LDS_ELEMS = S * (WGX + WGY) * TK;
     static_assert(TK == 32 || TK == 64, "k-block");
     static_assert(FX * WX * 16 == WGX && FY * WY * 16 == WGY, "tile shape");
-    // MFMA phase at raised wave priority: measured faster with 64-deep k-blocks (two-plane half-
-    // transform 5.42 -> 5.08 ms, SYRK 2.65 -> 2.51 ms; three-plane half-transform 6.75 -> 6.64 ms) and
-    // slower with 32-deep ones (three-plane SYRK 3.54 -> 3.91 ms)
+    // MFMA phase at raised wave priority: measured faster with 64-deep k-blocks (two-plane SYRK 2.65 -> 2.51
+    // ms) and slower with 32-deep ones (three-plane SYRK 3.54 -> 3.91 ms)
     static constexpr bool PRIO = TK == 64;
 };
 

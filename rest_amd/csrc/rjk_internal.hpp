@@ -52,7 +52,7 @@ struct rjk_ctx {
     hipStream_t stream = nullptr;
     double* b64 = nullptr;    // [naux][ldb]
     float* b32 = nullptr;     // [naux][ldb]
-    void* bpl = nullptr;      // BF16 planes [kBfStoredPlanes][naux][nbf_pad][nbf_pad]
+    void* bpl = nullptr;      // BF16 planes [kBfStoredPlanes][naux] of nbf_pad × nbf_pad squares as fragments (rjk_bftile.hpp)
     size_t bpl_pad = 0;       // nbf_pad of the planes
     size_t ws_limit = size_t(4) << 30;
     void* ws = nullptr;       // grow-only workspace
@@ -165,8 +165,8 @@ hipError_t launch_ksyrk(hipStream_t st, int prec, const void* m, size_t nbf, siz
 hipError_t launch_kreduce(hipStream_t st, const double* kpart, const KPlan& kp, int nspin, size_t nbf,
                           double scale, double* vk);
 
-// K on BF16 planes (rjk_kbf.hip): C' planes [S][nk][nbf_pad], sign masks [nk] (uint16),
-// M' planes [S][Pc][nbf_pad][nk]
+// K on BF16 planes (rjk_kbf.hip), matrices as 16 × 32 fragments (rjk_bftile.hpp): C'ᵀ planes [S] of nk × nbf_pad,
+// sign masks [nk] (uint16), M' planes [S][Pc] of nbf_pad × nk
 int bf_planes(int prec);
 hipError_t launch_bf_planes_b(hipStream_t st, const double* b64, size_t ldb, size_t nbf, size_t nbf_pad,
                               size_t naux, void* planes);
@@ -204,9 +204,10 @@ hipError_t launch_pivot_chol(hipStream_t st, const double* dm, size_t nbf, size_
 // and off-diagonal [n].  *bad: the pairs are not good enough; eigenvectors of T in Z then become A's by
 // launch_eig_back.
 constexpr size_t kEigMax = 1024;
-// The SCF's smaller problems, free atoms among them, stay with dsyevd: an atom's shells are exactly
-// degenerate, so these kernels would hand most of them on, and which way an open shell points, hence the
-// guess made of it, is whichever vectors the solver gives.
+// The SCF's smaller problems stay with dsyevd, for the sake of free atoms: an atom's shells are exactly degenerate, so
+// these kernels would hand most of them on, and which way an open shell points, hence the guess made of it,
+// is whichever vectors the solver gives.  The size stands for the atom: atoms of the packaged basis sets have up to 14
+// functions; one of more than 40 takes these kernels, and its open shell may point elsewhere than by dsyevd.
 constexpr size_t kEigMin = 40;
 size_t eig_ws(size_t n);
 hipError_t launch_eig(hipStream_t st, const double* A, size_t n, double* w, double* Z, double* ws, int* bad);

@@ -15,7 +15,7 @@
 //   B planes  [S][naux] of nbf_pad × nbf_pad   full symmetric squares
 //   C' planes [S] of nk × nbf_pad              C'ᵀ: column c of C' as a row
 //   M' planes [S][Pc] of nbf_pad × nk          c along the rows of a fragment: both SYRK operands
-// Stage 1: M'_P[μ][c] = Σ_ν C'ᵀ[c][ν] B_P[ν][μ]                  (128 μ × up to 160 c tiles)
+// Stage 1: M'_P[μ][c] = Σ_ν C'ᵀ[c][ν] B_P[ν][μ]                  (128 or 256 μ × up to 192 c tiles)
 // Stage 2: Kpart[split][s][ν][μ] (+)= Σ_{P,c} sign_c M'_P[ν][c] M'_P[μ][c]  (128 × 128 upper tiles)
 // Stage 3: the FP64 split reduction of rjk_k.hip.
 #include <hip/hip_runtime.h>

@@ -298,8 +298,8 @@ __device__ __forceinline__ void khalf_tile(BP __restrict__ bcol_, int nbf, int m
 // ---------------------------------------------------------------------------
 // Stage 2: Kpart (+)= Σ_{P,c} M'[P][c][μ] sign_c M'[P][c][ν] over the upper tiles
 //   (mu0 <= nu0) of 32·F × 32·F, split-K over P, 2 × 2 waves of F × F fragments.  In a
-//   diagonal tile the wave below the diagonal computes nothing and the two on it only
-//   their fragments i <= j; waves beyond nbf compute nothing (`rot` as in stage 1).
+//   diagonal tile the wave below the diagonal computes nothing (the two on it all of
+//   theirs), nor do waves beyond nbf (`rot` as in stage 1).
 //   Same pipeline as stage 1 over the flattened (P, 16-column block) index: lane offsets
 //   within a k-block's 16 rows are fixed, the base moves by scalar arithmetic.  A diagonal
 //   tile stages its rows once for both operands.  Signs are looked at once per tile and

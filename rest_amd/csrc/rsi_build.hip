@@ -1,4 +1,4 @@
-// rsi_build.cpp — packed B = (μν|Q)·V^{-1/2} written straight into the
+// rsi_build.hip — packed B = (μν|Q)·V^{-1/2} written straight into the
 // HBM-resident storage of an rjk_ctx (Molecule::prepare_rimatr_for_ri_v_rayon_v02,
 // src/molecule_io/mod.rs:1563-1721).
 //
@@ -66,9 +66,8 @@ __global__ void k_scale_cols(double* U, int n, const double* w) {
 // Newton–Schulz steps X ← X (a − b XᵀX) (Higham, Functions of Matrices, ch. 8); then Lᵀ = Q V^{1/2}
 // and V^{-1/2} = L^{-T} Q.  Singular values of Lᵀ are the square roots of V's eigenvalues, and pivoting
 // grades its rows, which every step's product on the right keeps.  Against integrals and root in 80 bits B of
-// 1 to 3 waters errs by 0.2 to 0.8e-12 of its norm; from rocSOLVER's eigenpairs of the same V by 0.2 to 1.3e-12, of
-// the host's V, as before, by 0.7 to 1.7e-12 (V's own rounding is most of it; an unpivoted factor adds 1 to
-// 7e-11).  1356 auxiliary functions: 9.3 ms against 31 with dsyevd, whose tridiagonal reduction
+// 1 to 3 waters errs by 0.2 to 0.8e-12 of its norm; from rocSOLVER's eigenpairs of the host's V, as before, by 0.7 to
+// 1.7e-12 (V's own rounding is most of it; an unpivoted factor adds 1 to 7e-11).  1356 auxiliary functions: 9.3 ms against 31 with dsyevd, whose tridiagonal reduction
 // is five dependent launches a column; 113: 1.2 against 2.4; 3164: 75 against 283.  Of the 9.3 ms the
 // pivots take 3.5, the 19 steps' products 4.0 (47 TFLOP/s), the updates 0.9, the triangular solve 0.5.
 constexpr int kMetBlock = 64;      // pivots between updates of the whole remainder
@@ -351,7 +350,7 @@ int metric_polar(rjk_ctx* ctx, rocblas_handle h, hipStream_t st, size_t n, doubl
     double *S = (double*)base, *L = (double*)(base + nn), *X = (double*)(base + 2 * nn), *X2 = (double*)(base + 3 * nn);
     double* diag = (double*)(base + 4 * nn);
     double* part = diag + 2 * n;               // [2][kMetParts]
-    double* top0 = part + 2 * kMetParts;       // and the row sums behind it, before the steps
+    double* top0 = part + 2 * kMetParts;       // the first pivot; the row sums are in X until the steps
     int* state = (int*)(top0 + 2);
     int* piv = state + 2;
     const rocblas_int ni = (rocblas_int)n;
